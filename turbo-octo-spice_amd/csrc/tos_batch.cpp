@@ -134,13 +134,45 @@ void add_buffer_key(std::vector<uint64_t> &k, int32_t n, const tos_batch_job *jo
         put(k, p->other.ptr);
         put(k, p->csep.ptr);
         put(k, jobs[j].cat->pix.ptr);
+        k.push_back((uint64_t)p->tiles.state);
     }
     for (const TuneEntry &t : ctx->tuned) k.push_back(((uint64_t)t.block << 32) | (uint32_t)t.blocks_per_cu);
 }
 
+// Workgroups of the jobs of one tile launch: shares of kTileRounds times the
+// resident ones by visits, at least one each, the largest job's first.  A
+// workgroup ends when its job has no tile left and makes room for the next
+// job's, so several rounds only cost their histograms.
+constexpr int kTileRounds = 4;
+
+void plan_tile_group(const tos_ctx *ctx, BatchGroup &G, int max_slots, const tos_batch_job *jobs,
+                     std::vector<XiKernelArgs> &args, std::vector<XiWgTask> &tasks, std::vector<uint64_t> &task_cost,
+                     std::vector<int> &job_nwg)
+{
+    G.lds = tile_lds_bytes(max_slots);
+    G.block = tile_block_size(max_slots);
+    const int resident = ctx->ncu * (kTileBlockMax / G.block);
+    double total = 0;
+    for (int j : G.jobs) total += (double)jobs[j].pairs->tiles.total;
+    std::vector<int> order = G.jobs;
+    std::stable_sort(order.begin(), order.end(),
+                     [&](int x, int y) { return jobs[x].pairs->tiles.total > jobs[y].pairs->tiles.total; });
+    G.task_begin = (int)tasks.size();
+    for (int j : order) {
+        const double share = total > 0 ? (double)jobs[j].pairs->tiles.total / total : 0.0;
+        const int want = std::min(resident, std::max(1, (int)std::ceil(kTileRounds * resident * share)));
+        const int nwg = tile_workgroups(jobs[j].pairs, args[(size_t)j].tile, want, G.block);
+        job_nwg[(size_t)j] = nwg;
+        for (int w = 0; w < nwg; ++w) tasks.push_back(XiWgTask{j, 0, 0, w});
+    }
+    task_cost.resize(tasks.size(), 0);   // bounded by kTileVisits
+    G.n_wg = (int)tasks.size() - G.task_begin;
+}
+
 }  // namespace
 
-int batch_prepare(tos_ctx *ctx, int32_t n, const tos_batch_job *jobs, BatchState &B, const ItemSlice *slices)
+int batch_prepare(tos_ctx *ctx, int32_t n, const tos_batch_job *jobs, BatchState &B, const ItemSlice *slices,
+                  bool tiles)
 {
     // group jobs by kernel variant, decided from each job's own constants
     std::map<VariantKey, std::vector<int>> by;
@@ -150,7 +182,16 @@ int batch_prepare(tos_ctx *ctx, int32_t n, const tos_batch_job *jobs, BatchState
         fill_args(jobs[j].cat, jobs[j].pairs, jobs[j].grid, true, args[(size_t)j]);
         bool fixed, simple;
         xi_variant(jobs[j].grid.type, args[(size_t)j].ge, args[(size_t)j].gf, fixed, simple);
-        by[VariantKey{jobs[j].grid.type, jobs[j].precision, fixed, simple}].push_back(j);
+        // jobs of the tile path: the precision and `simple` make no difference
+        const tos_batch_job &J = jobs[j];
+        const bool tile = tiles && tile_job(J.cat, J.pairs, J.grid, J.accum) && J.pairs->tiles.state == 1 &&
+                          tile_args(J.pairs, J.grid, args[(size_t)j]) &&
+                          (int64_t)tile_lds_bytes((int)args[(size_t)j].ge.nslots) + 64 <= ctx->max_lds_block &&
+                          J.pairs->tiles.total / kTileVisits < (uint64_t)kMaxTasks;
+        if (tile)
+            by[VariantKey{J.grid.type, TOS_FP64, tile_fixed((int)args[(size_t)j].ge.nslots), true, true}].push_back(j);
+        else
+            by[VariantKey{J.grid.type, J.precision, fixed, simple, false}].push_back(j);
         B.nbins[(size_t)j] = jobs[j].grid.nbins[0] * jobs[j].grid.nbins[1] * jobs[j].grid.nbins[2];
     }
     std::vector<XiWgTask> tasks;
@@ -162,7 +203,8 @@ int batch_prepare(tos_ctx *ctx, int32_t n, const tos_batch_job *jobs, BatchState
     // partial-row offsets, output offsets
     size_t cnt_words = 0, sum_words = 0;
     B.out_off.assign((size_t)n, 0);
-    B.res_words = 2 * (size_t)n;   // counters first: [rechecks, evaluated] per job
+    // counters first: [rechecks, evaluated] per job, then the tile counters
+    B.res_words = 3 * (size_t)n;
     B.max_fields = 0;
     for (auto &kv : by) {
         BatchGroup G;
@@ -174,6 +216,11 @@ int batch_prepare(tos_ctx *ctx, int32_t n, const tos_batch_job *jobs, BatchState
             GridExact ge;
             grid_exact_consts(jobs[j].grid, ge);
             max_slots = std::max(max_slots, (int)ge.nslots);
+        }
+        if (G.key.tile) {
+            plan_tile_group(ctx, G, max_slots, jobs, args, tasks, task_cost, job_nwg);
+            B.groups.push_back(G);
+            continue;
         }
         G.lds = xi_lds_bytes(TOS_ACC_CORE, max_slots);
         if ((int64_t)G.lds + 64 > ctx->max_lds_block) {
@@ -287,14 +334,17 @@ int batch_prepare(tos_ctx *ctx, int32_t n, const tos_batch_job *jobs, BatchState
         a.part_cnt = (uint32_t *)B.parts_cnt.ptr + co;
         a.part_sum = (double *)B.parts_sum.ptr + so;
         a.n_recheck = (unsigned long long *)(res + 2 * j);
+        a.tile.next = (uint32_t *)(res + 2 * n + j);
         red[(size_t)j].part_cnt = a.part_cnt;
         red[(size_t)j].part_sum = a.part_sum;
         red[(size_t)j].out_cnt = res + B.out_off[(size_t)j];
         red[(size_t)j].out_sum = (double *)(res + B.out_off[(size_t)j] + B.nbins[(size_t)j]);
     }
     for (const BatchGroup &G : B.groups) {
-        const int e = launch_xi_batch(G.key.coord, G.key.prec, G.key.fixed, G.key.simple, XiBatchArgs{}, 0, G.block,
-                                      G.lds, ctx->stream);
+        const int e = G.key.tile ? launch_tile_batch(G.key.coord, G.key.fixed, XiBatchArgs{}, 0, G.block, G.lds,
+                                                     ctx->stream)
+                                 : launch_xi_batch(G.key.coord, G.key.prec, G.key.fixed, G.key.simple, XiBatchArgs{},
+                                                   0, G.block, G.lds, ctx->stream);
         if (e != hipSuccess) return hip_fail(ctx, (hipError_t)e, "batched kernel LDS limit");
     }
     int rc;
@@ -313,15 +363,16 @@ int batch_prepare(tos_ctx *ctx, int32_t n, const tos_batch_job *jobs, BatchState
 // every result into pinned host memory.  No memset nodes (graph-safe).
 int batch_enqueue(tos_ctx *ctx, BatchState &B, int32_t n, hipStream_t stream)
 {
-    int e = launch_zero_u64((unsigned long long *)B.res.ptr, 2 * (int64_t)n, stream);
+    int e = launch_zero_u64((unsigned long long *)B.res.ptr, 3 * (int64_t)n, stream);
     if (e != hipSuccess) return hip_fail(ctx, (hipError_t)e, "batch counter clear");
     for (const BatchGroup &G : B.groups) {
         if (G.n_wg == 0) continue;
         XiBatchArgs ba;
         ba.jobs = (const XiKernelArgs *)B.args.ptr;
         ba.wg = (const XiWgTask *)B.tasks.ptr + G.task_begin;
-        e = launch_xi_batch(G.key.coord, G.key.prec, G.key.fixed, G.key.simple, ba, G.n_wg, G.block, G.lds,
-                            stream);
+        e = G.key.tile ? launch_tile_batch(G.key.coord, G.key.fixed, ba, G.n_wg, G.block, G.lds, stream)
+                       : launch_xi_batch(G.key.coord, G.key.prec, G.key.fixed, G.key.simple, ba, G.n_wg, G.block,
+                                         G.lds, stream);
         if (e != hipSuccess) return hip_fail(ctx, (hipError_t)e, "batched pair kernel launch");
     }
     e = launch_reduce_batch((const XiReduceJob *)B.red.ptr, n, B.max_fields, stream);
@@ -413,7 +464,7 @@ int xi_run_per_skybin(tos_ctx *ctx, const tos_catalog *cat, tos_pairs *p, const 
     bool fixed, simple;
     xi_variant(g.type, base.ge, base.gf, fixed, simple);
     BatchGroup G;
-    G.key = VariantKey{g.type, prec, fixed, simple};
+    G.key = VariantKey{g.type, prec, fixed, simple, false};
     GridExact ge;
     grid_exact_consts(g, ge);
     G.lds = xi_lds_bytes(TOS_ACC_CORE, (int)ge.nslots);
@@ -453,7 +504,7 @@ int xi_run_per_skybin(tos_ctx *ctx, const tos_catalog *cat, tos_pairs *p, const 
     // partial rows, outputs
     B.nbins.assign((size_t)nk, nbins);
     B.out_off.assign((size_t)nk, 0);
-    B.res_words = 2 * (size_t)nk;
+    B.res_words = 3 * (size_t)nk;
     B.max_fields = (int64_t)nbins * 3;
     std::vector<size_t> row_off((size_t)nk, 0);
     size_t total_rows = 0;
@@ -580,6 +631,7 @@ extern "C" int tos_batch_run(tos_ctx *ctx, int32_t n, const tos_batch_job *jobs,
         if ((rc = ensure_items(ctx, p, true, nullptr, tuned_step_cap(ctx, jobs[j].grid, jobs[j].precision))) !=
             TOS_OK)
             return rc;
+        if (tile_job(jobs[j].cat, p, jobs[j].grid, jobs[j].accum) && (rc = ensure_tile_plan(ctx, p)) != TOS_OK) return rc;
         if (jobs[j].grid.type == TOS_OBSERVING && (rc = ensure_theta(ctx, p, jobs[j].grid)) != TOS_OK) return rc;
     }
     if (!ctx->batch) {
@@ -595,7 +647,7 @@ extern "C" int tos_batch_run(tos_ctx *ctx, int32_t n, const tos_batch_job *jobs,
     if (key != B.key) {
         B.drop_graph();
         B.key.clear();
-        if ((rc = batch_prepare(ctx, n, jobs, B)) != TOS_OK) return rc;
+        if ((rc = batch_prepare(ctx, n, jobs, B, nullptr, true)) != TOS_OK) return rc;
         B.key = key;
     }
     hipError_t he;
@@ -631,6 +683,8 @@ extern "C" int tos_batch_run(tos_ctx *ctx, int32_t n, const tos_batch_job *jobs,
     hipEventElapsedTime(&ms, B.ev0, B.ev1);
     if (batch_ms) *batch_ms = ms;
     batch_collect(B, n, ms, out);
+    for (int32_t j = 0; j < n; ++j)
+        if (jobs[j].precision == TOS_FP64) out[j].num_guard_rechecks = 0;
     return TOS_OK;
 }
 

@@ -422,6 +422,7 @@ extern "C" int tos_catalog_free(tos_ctx *ctx, tos_catalog *cat)
     cat->pix.release();
     cat->los.release();
     cat->trig.release();
+    cat->ladder.release();
     delete cat;
     return TOS_OK;
 }
@@ -577,6 +578,7 @@ extern "C" int tos_pairs_free(tos_ctx *ctx, tos_pairs *p)
     p->items.release();
     p->cost_prefix.release();
     p->theta.release();
+    p->tiles.release();
     delete p;
     return TOS_OK;
 }
@@ -610,6 +612,7 @@ void catalog_detach(tos_catalog *cat, std::vector<void *> &dev)
     detach(cat->pix, dev);
     detach(cat->los, dev);
     detach(cat->trig, dev);
+    for (DevBuf *b : {&cat->ladder.pix, &cat->ladder.d, &cat->ladder.l, &cat->ladder.place}) detach(*b, dev);
     delete cat;
 }
 
@@ -620,6 +623,8 @@ void pairs_detach(tos_pairs *p, std::vector<void *> &dev)
     detach(p->items, dev);
     detach(p->cost_prefix, dev);
     detach(p->theta, dev);
+    TilePlan &t = p->tiles;
+    for (DevBuf *b : {&t.masks, &t.rec, &t.batch_ptr, &t.visits}) detach(*b, dev);
     delete p;
 }
 

@@ -41,6 +41,25 @@ struct TuneEntry {
     int step_cap;             // partner pixels per work item (0: default)
 };
 
+// A catalogue on its ladder (tos_tile.cpp).
+struct Ladder {
+    int state = 0;                // 0: not looked for, 1: built, 2: none
+    int nblk = 0;
+    DevBuf pix, d, l, place;
+    std::vector<float> h_d, h_l;  // [16 nblk]
+    void release();
+};
+
+// Tile plan of a pair list (tos_tile.cpp).
+struct TilePlan {
+    int state = 0;                // as Ladder::state
+    int n_batches = 0;
+    int words = 0;                // mask words of a batch
+    uint64_t total = 0;           // visits of all tiles
+    DevBuf masks, rec, batch_ptr, visits;
+    void release();
+};
+
 struct BatchState;                 // tos_batch.cpp
 void batch_release(tos_ctx *ctx);
 
@@ -82,6 +101,7 @@ struct tos_catalog {
     tos::DevBuf pix;    // float4 {distance, loglam, weight, weight*value}
     tos::DevBuf los;    // LosInfo
     tos::DevBuf trig;   // double4 {sin dec, cos dec, sin ra, cos ra} (device search)
+    tos::Ladder ladder;
     std::vector<tos::LosInfo> h_los;
     std::vector<int64_t> h_offsets;
     std::vector<double> h_ra, h_dec;
@@ -112,6 +132,7 @@ struct tos_pairs {
     tos::DevBuf theta;
     double theta_key[3] = {0, 0, 0};
     int32_t theta_n = -1;
+    tos::TilePlan tiles;
 };
 
 namespace tos {
@@ -148,7 +169,19 @@ int plan_launch(tos_ctx *ctx, const tos_xi_opts *opts, int prec, int accum, cons
                 XiLaunch &L, uint32_t band_rows = 0);
 // Axis-0 rows per LDS histogram of a grid with this accumulator set: all
 // of them when the grid fits, else the most that fit (0: not even one).
-uint32_t band_rows_for(const tos_ctx *ctx, int accum, const tos_grid &g);
+uint32_t band_rows_for(const tos_ctx *ctx, int accum, const tos_grid &g, bool tiles = false);
+// The tile path's launch: LDS, partial rows and workgroups (false: more
+// partial rows than allowed).
+bool plan_tiles(tos_ctx *ctx, const tos_pairs *p, const tos_grid &g, XiKernelArgs &a, XiLaunch &L, uint32_t band_rows);
+// The tile path (tos_tile.cpp): whether a job may take it, its plan
+// (tiles.state 1 when built; 2: the general path), its kernel arguments
+// (false: the edge bound is too wide).
+bool tile_job(const tos_catalog *cat, const tos_pairs *p, const tos_grid &g, int accum);
+int ensure_ladder(tos_ctx *ctx, tos_catalog *cat);
+int ensure_tile_plan(tos_ctx *ctx, tos_pairs *p);
+bool tile_args(const tos_pairs *p, const tos_grid &g, XiKernelArgs &a);
+// Workgroups of a tile pass that should have `want` of them.
+int tile_workgroups(const tos_pairs *p, const TileArgs &a, int want, int block);
 // Resolves this device's static scratch array of tos_xi_run_noalloc
 // (tos_noalloc.hip); the device must be current.
 int noalloc_setup(tos_ctx *ctx);

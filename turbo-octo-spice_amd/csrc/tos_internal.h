@@ -56,6 +56,7 @@ struct GridExact {
     uint32_t nslots;      // n0 * (rowlen + pad)
     uint32_t row8;        // 8 (rowlen + pad): byte stride of an axis-0 row of FP64 sums
     uint32_t nz8;         // 8 n2
+    double width1;        // axis-1 bin width
 };
 
 // Constants of the FP32 fast path with its guard band.  The kernel forms
@@ -73,6 +74,41 @@ struct GridFast {
     uint32_t nonneg;      // bit k: t_k >= 0 for every pair (skip the > -1 test)
     uint32_t small_safe;  // 1 (Cartesian): r_perp^2 < small implies bin 0 in both arithmetics
     uint32_t zero_min;    // bit k: axis k starts at exactly 0, so a zero coordinate is bin 0 exactly
+};
+
+// The tile path (tos_tileplan.hip, tos_tilepass.hip): catalogues whose pixels
+// all sit on one ladder of (distance, loglam) steps, as survey spectra on a
+// common wavelength grid do.  The ladder is cut into blocks of 16 steps.
+constexpr int32_t kBlockSteps = 16;
+constexpr int32_t kMaxLadder = 2048;                         // ladder steps (blocks fit a byte)
+constexpr int32_t kMaxBatch = 16384;                         // pairs per batch (sorted in LDS)
+
+// Where a sightline sits on the ladder: its pixels' block B starts at byte
+// off + 256 B (modulo 2^32) of TileArgs::pix; it covers blocks [b0, b0 + nb).
+struct LadderLos {
+    uint32_t off;
+    uint32_t b0_nb;               // b0 | nb << 8
+};
+
+struct TileArgs {
+    const float4 *pix;            // per ladder step of a sightline {w, w*delta, 1, 0}; absent pixels are 0
+    const float *d, *l;           // [16 nblk] the ladder (padded with its last step)
+    // [n_batches][2][nblk][words] 64 pairs a word: those whose first / second
+    // sightline covers the block
+    const uint64_t *masks;
+    const uint4 *rec;             // [pairs] {off_i, off_j, f32 bits of 2 (1 - c), pair index}, ascending
+                                  //   2 (1 - c) within a batch
+    const int32_t *batch_ptr;     // [n_batches + 1] pair ranges
+    const uint32_t *visits;       // [n_batches][nblk][nblk] pairs covering each tile
+    uint32_t *next;               // the next tile to draw (0 at the launch)
+    int32_t nblk;                 // ladder blocks
+    int32_t band;                 // tiles (B1, B2) with |B1 - B2| <= band are visited
+    int32_t n_batches;
+    int32_t words;
+    // a bin edge's 2 (1 - c) is known within a relative eps; one that lies
+    // `ulps` float steps below a pair's value is certainly below it
+    uint32_t ulps;
+    double eps;
 };
 
 struct XiKernelArgs {
@@ -113,6 +149,7 @@ struct XiKernelArgs {
     uint32_t band_len8;
     int32_t band_bin0;
     int32_t banded;
+    TileArgs tile;                // tile path only
 };
 
 // One workgroup's task in a batched launch: items [begin, end) of job
@@ -206,6 +243,53 @@ struct ItemArgs {
     uint64_t *item_cost;
 };
 int launch_items(const ItemArgs &a, bool fill, void *stream);
+
+// Tile path: ladder and plan kernels (tos_tileplan.hip).
+struct LadderArgs {
+    const float4 *pix;
+    const LosInfo *los;
+    int64_t n_los, n_pix;
+    uint64_t *table;              // [kLadderTable] {loglam bits << 32 | distance bits}, all ones: empty
+    uint32_t *state;              // [0] not a ladder, [1] entries, [2] blocks in all
+    const uint16_t *step;         // [kLadderTable] ladder step of each table entry
+    LadderLos *place;             // [n_los]
+    uint32_t *nblk_of;            // [n_los] blocks of each sightline, then their exclusive prefix
+    float4 *out;
+};
+constexpr int32_t kLadderTable = 8192;
+int launch_ladder_collect(const LadderArgs &a, void *stream);
+int launch_ladder_place(const LadderArgs &a, void *stream);
+int launch_ladder_fill(const LadderArgs &a, int64_t n_blocks, void *stream);
+struct TilePlanArgs {
+    const int32_t *row_los;
+    const int64_t *row_ptr;
+    const int32_t *other;
+    const double *csep;
+    const LadderLos *place;
+    int64_t n_rows;
+    int32_t n_batches, max_batch, nblk;
+    const int32_t *batch_ptr;
+    int32_t words;
+    uint32_t *cover;              // [pairs] blocks of both sightlines: bi0 | nbi << 8 | bj0 << 16 | nbj << 24
+    uint64_t *masks;
+    uint4 *rec;
+    uint32_t *visits;             // [n_batches][nblk][nblk] pairs covering each tile
+    unsigned long long *state;    // [0] set when a pair's separation is unusable, [1] visits of all tiles
+};
+int launch_tile_plan(const TilePlanArgs &a, void *stream);
+// The pass itself (tos_tilepass.hip): its wavefronts take tiles off one
+// counter, so any number of workgroups does the whole job as long as their
+// counts can hold it: a workgroup stops taking tiles after kTileVisits visits.
+constexpr int kTileBlockMax = 1024;
+constexpr uint32_t kTileVisits = 1u << 23;
+static_assert((kTileVisits + (uint64_t)(kTileBlockMax / 64) * kMaxBatch) * 256 < (1ull << 32),
+              "a workgroup's counts are 32-bit");
+bool tile_fixed(int nslots);           // the kernel variant with the fixed histogram layout
+int tile_block_size(int nslots);
+size_t tile_lds_bytes(int nslots);
+int launch_tile_pass(int coord, const XiKernelArgs &a, int n_wg, int block, size_t lds_bytes, void *stream);
+int launch_tile_batch(int coord, bool fixed, const XiBatchArgs &b, int n_wg, int block, size_t lds_bytes,
+                      void *stream);
 
 // Zero n 64-bit words with a kernel (safe inside a captured graph).
 int launch_zero_u64(unsigned long long *p, int64_t n, void *stream);

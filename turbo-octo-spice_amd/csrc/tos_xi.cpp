@@ -226,13 +226,29 @@ int plan_launch(tos_ctx *ctx, const tos_xi_opts *opts, int prec, int accum, cons
     return TOS_OK;
 }
 
-uint32_t band_rows_for(const tos_ctx *ctx, int accum, const tos_grid &g)
+bool plan_tiles(tos_ctx *ctx, const tos_pairs *p, const tos_grid &g, XiKernelArgs &a, XiLaunch &L, uint32_t band_rows)
+{
+    GridExact ge;
+    grid_exact_consts(g, ge);
+    const bool banded = band_rows > 0 && band_rows < ge.n[0];
+    const int slots = banded ? (int)(band_rows * (ge.rowlen + ge.pad)) : (int)ge.nslots;
+    L.nbins = banded ? (int)(band_rows * ge.rowlen) : (int)ge.ntot;
+    L.nsum = 2;
+    L.lds = tile_lds_bytes(slots);
+    L.block = tile_block_size(slots);
+    L.n_wg = tile_workgroups(p, a.tile, ctx->ncu * (2048 / kTileBlockMax), L.block);
+    L.n_seg = std::min(32, L.n_wg);
+    return (int64_t)L.n_wg * L.nbins * (4 + 8 * L.nsum) <= kMaxPartialBytes;
+}
+
+uint32_t band_rows_for(const tos_ctx *ctx, int accum, const tos_grid &g, bool tiles)
 {
     GridExact ge;
     grid_exact_consts(g, ge);
     const uint32_t rowslots = ge.rowlen + ge.pad;
     auto fits = [&](uint32_t rows) {
-        return (int64_t)xi_lds_bytes(accum, (int)(rows * rowslots)) + 64 <= ctx->max_lds_block;
+        const int slots = (int)(rows * rowslots);
+        return (int64_t)(tiles ? tile_lds_bytes(slots) : xi_lds_bytes(accum, slots)) + 64 <= ctx->max_lds_block;
     };
     if (fits(ge.n[0])) return ge.n[0];
     uint32_t lo = 0, hi = ge.n[0];   // the most rows that fit
@@ -336,8 +352,20 @@ extern "C" int tos_xi_run(tos_ctx *ctx, const tos_catalog *cat, const tos_pairs 
     out->kernel_ms = 0;
 
     const int flags = opts ? opts->flags : 0;
-    int rc = ensure_items(ctx, p, !(flags & TOS_XI_NO_TRANSPOSE), nullptr, tuned_step_cap(ctx, g, prec));
-    if (rc != TOS_OK) return rc;
+    int rc;
+    // the tile path: catalogues on a ladder, no work scheme switched off and
+    // no launch shape asked for
+    bool tiles = flags == 0 && (!opts || (opts->block_size == 0 && opts->blocks_per_cu == 0 && opts->wg_per_slot == 0)) &&
+                 tile_job(cat, p, g, accum);
+    XiKernelArgs a;
+    if (tiles) {
+        if ((rc = ensure_tile_plan(ctx, p)) != TOS_OK) return rc;
+        tiles = p->tiles.state == 1;
+    }
+    // the work items in either case: tos_xi_run_noalloc takes them up on any
+    // grid
+    if ((rc = ensure_items(ctx, p, !(flags & TOS_XI_NO_TRANSPOSE), nullptr, tuned_step_cap(ctx, g, prec))) != TOS_OK)
+        return rc;
     const size_t n_items = (size_t)p->n_items;
     if (n_items == 0) {
         std::memset(out->num_pairs, 0, sizeof(uint64_t) * nbins);
@@ -347,10 +375,20 @@ extern "C" int tos_xi_run(tos_ctx *ctx, const tos_catalog *cat, const tos_pairs 
             for (double *a : {out->di, out->dj, out->wi, out->wj, out->z}) std::memset(a, 0, sizeof(double) * nbins);
         return TOS_OK;
     }
+    // the theta bins before the kernel arguments, which hold their address
     if (g.type == TOS_OBSERVING && (rc = ensure_theta(ctx, p, g)) != TOS_OK) return rc;
+    if (tiles) {
+        fill_args(cat, p, g, true, a);
+        tiles = tile_args(p, g, a);
+    }
     // a grid too large for one LDS histogram runs in bands of axis-0 rows,
     // one full pass over the pairs per band
-    const uint32_t rows = band_rows_for(ctx, accum, g);
+    uint32_t rows = band_rows_for(ctx, accum, g, tiles);
+    XiLaunch L;
+    if (tiles && (rows == 0 || !plan_tiles(ctx, p, g, a, L, rows))) {
+        tiles = false;
+        rows = band_rows_for(ctx, accum, g);
+    }
     if (rows == 0) {
         set_err(ctx, "one axis-0 row of the grid has too many bins for the LDS histogram");
         return TOS_ERR_INVALID;
@@ -358,12 +396,13 @@ extern "C" int tos_xi_run(tos_ctx *ctx, const tos_catalog *cat, const tos_pairs 
     GridExact ge;
     grid_exact_consts(g, ge);
     const bool banded = rows < ge.n[0];
-    XiLaunch L;
-    if ((rc = plan_launch(ctx, opts, prec, accum, g, n_items, L, banded ? rows : 0)) != TOS_OK) return rc;
+    if (!tiles && (rc = plan_launch(ctx, opts, prec, accum, g, n_items, L, banded ? rows : 0)) != TOS_OK) return rc;
     if ((rc = reserve_scratch(ctx, L, nbins)) != TOS_OK) return rc;
-    std::vector<int32_t> wgp;
-    balance_items(p->item_cost, L.n_wg, wgp);
-    {
+    if (tiles) {
+        a.tile.next = (uint32_t *)((unsigned long long *)ctx->recheck.ptr + 2);
+    } else {
+        std::vector<int32_t> wgp;
+        balance_items(p->item_cost, L.n_wg, wgp);
         // a workgroup's u32 partial counts hold at most its items' cost
         // (pixel pairs before the windows)
         uint64_t worst = 0;
@@ -376,19 +415,18 @@ extern "C" int tos_xi_run(tos_ctx *ctx, const tos_catalog *cat, const tos_pairs 
             set_err(ctx, "tos_xi_run: a workgroup would count 2^32 pixel pairs; split the catalogue");
             return TOS_ERR_INVALID;
         }
+        if ((rc = upload(ctx, ctx->wgptr, wgp.data(), wgp.size() * sizeof(int32_t), "workgroup ranges")) != TOS_OK)
+            return rc;
+        fill_args(cat, p, g, !(flags & TOS_XI_NO_WINDOW), a);
+        a.interleave = (flags & TOS_XI_NO_INTERLEAVE) ? 0 : 1;
+        a.zconst = (flags & TOS_XI_NO_ZCONST) ? 0 : 1;
+        a.wg_item_ptr = (const int32_t *)ctx->wgptr.ptr;
     }
-    if ((rc = upload(ctx, ctx->wgptr, wgp.data(), wgp.size() * sizeof(int32_t), "workgroup ranges")) != TOS_OK) return rc;
-
-    XiKernelArgs a;
-    fill_args(cat, p, g, !(flags & TOS_XI_NO_WINDOW), a);
-    a.interleave = (flags & TOS_XI_NO_INTERLEAVE) ? 0 : 1;
-    a.zconst = (flags & TOS_XI_NO_ZCONST) ? 0 : 1;
-    a.wg_item_ptr = (const int32_t *)ctx->wgptr.ptr;
     a.part_cnt = (uint32_t *)ctx->part_cnt.ptr;
     a.part_sum = (double *)ctx->part_sum.ptr;
     a.n_recheck = (unsigned long long *)ctx->recheck.ptr;
-    hipError_t he = hipMemsetAsync(ctx->recheck.ptr, 0, 16, ctx->stream);
-    if (he != hipSuccess) return hip_fail(ctx, he, "tos_xi_run memset");
+    int e = launch_zero_u64(a.n_recheck, 3, ctx->stream);   // both tallies and the tile counter
+    if (e != hipSuccess) return hip_fail(ctx, (hipError_t)e, "tos_xi_run counter clear");
     hipEventRecord(ctx->ev0, ctx->stream);
     const uint32_t rowslots = ge.rowlen + ge.pad;
     for (uint32_t r0 = 0; r0 < ge.n[0]; r0 += rows) {
@@ -400,7 +438,10 @@ extern "C" int tos_xi_run(tos_ctx *ctx, const tos_catalog *cat, const tos_pairs 
             a.band_bin0 = (int32_t)(r0 * ge.rowlen);
             a.nbins = (int32_t)((r1 - r0) * ge.rowlen);
         }
-        int e = launch_xi(g.type, prec, accum, a, L.n_wg, L.block, L.lds, ctx->stream);
+        if (tiles && r0 > 0 && (e = launch_zero_u64(a.n_recheck + 2, 1, ctx->stream)) != hipSuccess)
+            return hip_fail(ctx, (hipError_t)e, "tile counter clear");
+        e = tiles ? launch_tile_pass(g.type, a, L.n_wg, L.block, L.lds, ctx->stream)
+                  : launch_xi(g.type, prec, accum, a, L.n_wg, L.block, L.lds, ctx->stream);
         if (e != hipSuccess) return hip_fail(ctx, (hipError_t)e, "xi kernel launch");
         if (!banded) hipEventRecord(ctx->ev1, ctx->stream);   // the pair kernel alone
         e = launch_reduce(a.part_cnt, a.part_sum, L.n_wg, a.nbins, L.nsum, (uint64_t *)ctx->out_cnt.ptr + a.band_bin0,
@@ -414,12 +455,12 @@ extern "C" int tos_xi_run(tos_ctx *ctx, const tos_catalog *cat, const tos_pairs 
     hipMemcpyAsync(out->num_pairs, ctx->out_cnt.ptr, (size_t)nbins * 8, hipMemcpyDeviceToHost, ctx->stream);
     hipMemcpyAsync(sums.data(), ctx->out_sum.ptr, sums.size() * 8, hipMemcpyDeviceToHost, ctx->stream);
     hipMemcpyAsync(nre, ctx->recheck.ptr, 16, hipMemcpyDeviceToHost, ctx->stream);
-    he = hipStreamSynchronize(ctx->stream);
+    const hipError_t he = hipStreamSynchronize(ctx->stream);
     if (he != hipSuccess) return hip_fail(ctx, he, "tos_xi_run");
     float ms = 0;
     hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1);
     out->kernel_ms = ms;
-    out->num_guard_rechecks = nre[0];
+    out->num_guard_rechecks = prec == TOS_FP32C ? nre[0] : 0;
     out->num_pairs_evaluated = nre[1];
     uint64_t used = 0;
     for (int b = 0; b < nbins; ++b) {
