@@ -128,3 +128,23 @@ def test_catalogues_without_a_ladder(dev, field, change):
     close(h, ref.num_pairs, {"didj": ref.didj, "wgt": ref.wgt})
     pairs.free()
     dcat.free()
+
+
+def test_a_weighted_value_that_overflows(dev, field):
+    """A w d beyond the float range reaches the bins of its own pairs only."""
+    cat = synth.Catalog(field.ra, field.dec, field.offsets, field.value.copy(), field.loglam, field.weight.copy(),
+                        field.distance, field.zq, field.scale)
+    for k, v in ((cat.n_pix // 3, 1e30), (cat.n_pix // 2, -1e30)):
+        cat.weight[k], cat.value[k] = 1e30, v
+    grid = GridSpec.cartesian()
+    dcat = dev.upload(cat)
+    pairs = dcat.pairs(grid.max_angular_scale(cat.scale), order=3, nthreads=8)
+    ref = pairs.run(grid, precision=tos_amd.FP64, flags=tos_amd.XI_NO_ZCONST)
+    h = pairs.run(grid, precision=tos_amd.FP64)
+    assert np.array_equal(h.num_pairs, ref.num_pairs)
+    assert 0 < np.sum(~np.isfinite(ref.didj)) < ref.didj.size
+    assert np.array_equal(np.isnan(h.didj), np.isnan(ref.didj))
+    assert np.array_equal(np.isinf(h.didj), np.isinf(ref.didj))
+    assert rel_err(h.wgt, ref.wgt) <= SUM_RTOL
+    pairs.free()
+    dcat.free()

@@ -136,7 +136,8 @@ __global__ void __launch_bounds__(256) zero_f4(float4 *p, int64_t n)
 }
 
 // One wavefront per sightline: its pixels onto the ladder.  The steps must
-// ascend within the sightline (state[0] otherwise).
+// ascend within the sightline and the weights be finite (state[0] otherwise):
+// where one of two sightlines has no pixel the pass multiplies by zero.
 __global__ void __launch_bounds__(256) ladder_fill(LadderArgs a)
 {
     const int lane = threadIdx.x & (kWave - 1);
@@ -160,7 +161,8 @@ __global__ void __launch_bounds__(256) ladder_fill(LadderArgs a)
         int before = __shfl_up(st, 1);
         if (lane == 0) before = prev;
         const uint32_t at = (uint32_t)st - b0 * kBlockSteps;
-        const bool ok = !in || (st > before && at < nb * kBlockSteps);
+        const bool ok = !in || (st > before && at < nb * kBlockSteps && __builtin_isfinite(v.z) &&
+                                __builtin_isfinite(v.w));
         if (!ok) a.state[0] = 1;
         if (in && ok) a.out[(size_t)first * kBlockSteps + at] = make_float4(v.z, v.w, 1.0f, 0.0f);
         prev = __shfl(st, kWave - 1);
