@@ -148,3 +148,23 @@ def test_a_weighted_value_that_overflows(dev, field):
     assert rel_err(h.wgt, ref.wgt) <= SUM_RTOL
     pairs.free()
     dcat.free()
+
+
+@pytest.mark.parametrize("spec", [GRIDS[k] for k in (0, 1, 3, 4, 8, 9, 11)],
+                         ids=[f"{GRIDS[k][0]}-{GRIDS[k][1]}-{GRIDS[k][3]}" for k in (0, 1, 3, 4, 8, 9, 11)])
+def test_seven_sums_equal_the_general_kernel(dev, field, spec):
+    grid = GridSpec.from_specs(*spec)
+    wide = GridSpec.cartesian() if spec[0] == CART else GridSpec.observing()
+    dcat = dev.upload(field)
+    pairs = dcat.pairs(wide.max_angular_scale(field.scale), order=3, nthreads=8)
+    print(f"case: grid {grid.specs} type {grid.type}", flush=True)
+    ref = pairs.run(grid, precision=tos_amd.FP64, accum=tos_amd.ACC_ALL, flags=tos_amd.XI_NO_ZCONST)
+    h = pairs.run(grid, precision=tos_amd.FP64, accum=tos_amd.ACC_ALL)
+    close(h, ref.num_pairs, {"didj": ref.didj, "wgt": ref.wgt})
+    for k in ("wi", "wj", "z"):
+        assert rel_err(h.extra[k], ref.extra[k]) <= SUM_RTOL, k
+    # signed: against the weights of the same pixels
+    assert signed_sum_err(h.extra["di"], ref.extra["di"], ref.extra["wi"]) <= SUM_RTOL
+    assert signed_sum_err(h.extra["dj"], ref.extra["dj"], ref.extra["wj"]) <= SUM_RTOL
+    pairs.free()
+    dcat.free()

@@ -149,9 +149,9 @@ void plan_tile_group(const tos_ctx *ctx, BatchGroup &G, int max_slots, const tos
                      std::vector<XiKernelArgs> &args, std::vector<XiWgTask> &tasks, std::vector<uint64_t> &task_cost,
                      std::vector<int> &job_nwg)
 {
-    G.lds = tile_lds_bytes(max_slots);
-    G.block = tile_block_size(max_slots);
-    const int resident = ctx->ncu * (kTileBlockMax / G.block);
+    G.lds = tile_lds_bytes(2, max_slots);
+    G.block = tile_block_size(2, max_slots);
+    const int resident = ctx->ncu * tile_threads_per_cu(2) / G.block;
     double total = 0;
     for (int j : G.jobs) total += (double)jobs[j].pairs->tiles.total;
     std::vector<int> order = G.jobs;
@@ -184,9 +184,9 @@ int batch_prepare(tos_ctx *ctx, int32_t n, const tos_batch_job *jobs, BatchState
         xi_variant(jobs[j].grid.type, args[(size_t)j].ge, args[(size_t)j].gf, fixed, simple);
         // jobs of the tile path: the precision and `simple` make no difference
         const tos_batch_job &J = jobs[j];
-        const bool tile = tiles && tile_job(J.cat, J.pairs, J.grid, J.accum) && J.pairs->tiles.state == 1 &&
+        const bool tile = tiles && tile_job(J.cat, J.pairs, J.grid) && J.pairs->tiles.state == 1 &&
                           tile_args(J.pairs, J.grid, args[(size_t)j]) &&
-                          (int64_t)tile_lds_bytes((int)args[(size_t)j].ge.nslots) + 64 <= ctx->max_lds_block &&
+                          (int64_t)tile_lds_bytes(2, (int)args[(size_t)j].ge.nslots) + 64 <= ctx->max_lds_block &&
                           J.pairs->tiles.total / kTileVisits < (uint64_t)kMaxTasks;
         if (tile)
             by[VariantKey{J.grid.type, TOS_FP64, tile_fixed((int)args[(size_t)j].ge.nslots), true, true}].push_back(j);
@@ -631,7 +631,7 @@ extern "C" int tos_batch_run(tos_ctx *ctx, int32_t n, const tos_batch_job *jobs,
         if ((rc = ensure_items(ctx, p, true, nullptr, tuned_step_cap(ctx, jobs[j].grid, jobs[j].precision))) !=
             TOS_OK)
             return rc;
-        if (tile_job(jobs[j].cat, p, jobs[j].grid, jobs[j].accum) && (rc = ensure_tile_plan(ctx, p)) != TOS_OK) return rc;
+        if (tile_job(jobs[j].cat, p, jobs[j].grid) && (rc = ensure_tile_plan(ctx, p)) != TOS_OK) return rc;
         if (jobs[j].grid.type == TOS_OBSERVING && (rc = ensure_theta(ctx, p, jobs[j].grid)) != TOS_OK) return rc;
     }
     if (!ctx->batch) {

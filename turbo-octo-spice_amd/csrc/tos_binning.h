@@ -179,6 +179,19 @@ struct Hist {
         unsafeAtomicAdd(reinterpret_cast<double *>(bs + off8 + st8), ww);
     }
 
+    // The other five sums of the seven.
+    __device__ __forceinline__ void add8n_more(uint32_t off8, double wd1, double wd2, double w1, double w2,
+                                               double z) const
+    {
+        const uint32_t st8 = 8u * stride();
+        char *bs = reinterpret_cast<char *>(hs);
+        unsafeAtomicAdd(reinterpret_cast<double *>(bs + off8 + 2 * st8), wd1);
+        unsafeAtomicAdd(reinterpret_cast<double *>(bs + off8 + 3 * st8), wd2);
+        unsafeAtomicAdd(reinterpret_cast<double *>(bs + off8 + 4 * st8), w1);
+        unsafeAtomicAdd(reinterpret_cast<double *>(bs + off8 + 5 * st8), w2);
+        unsafeAtomicAdd(reinterpret_cast<double *>(bs + off8 + 6 * st8), z);
+    }
+
     // One pixel pair into the slot at byte offset off8 = 8 * slot of the
     // FP64 arrays (the count sits at off8 / 2 of the u32 array), so one
     // address register serves every array through immediate offsets.

@@ -285,9 +285,10 @@ constexpr uint32_t kTileVisits = 1u << 23;
 static_assert((kTileVisits + (uint64_t)(kTileBlockMax / 64) * kMaxBatch) * 256 < (1ull << 32),
               "a workgroup's counts are 32-bit");
 bool tile_fixed(int nslots);           // the kernel variant with the fixed histogram layout
-int tile_block_size(int nslots);
-size_t tile_lds_bytes(int nslots);
-int launch_tile_pass(int coord, const XiKernelArgs &a, int n_wg, int block, size_t lds_bytes, void *stream);
+int tile_threads_per_cu(int nsum);       // resident, by the vector registers
+int tile_block_size(int nsum, int nslots);
+size_t tile_lds_bytes(int nsum, int nslots);
+int launch_tile_pass(int coord, int nsum, const XiKernelArgs &a, int n_wg, int block, size_t lds_bytes, void *stream);
 int launch_tile_batch(int coord, bool fixed, const XiBatchArgs &b, int n_wg, int block, size_t lds_bytes,
                       void *stream);
 

@@ -222,9 +222,9 @@ int ensure_tile_plan(tos_ctx *ctx, tos_pairs *p)
 // pass costs what it saves.
 constexpr int64_t kTileMinPairs = 400;
 
-bool tile_job(const tos_catalog *cat, const tos_pairs *p, const tos_grid &g, int accum)
+bool tile_job(const tos_catalog *cat, const tos_pairs *p, const tos_grid &g)
 {
-    if (g.type == TOS_POLAR || accum != TOS_ACC_CORE || p->n_pairs < kTileMinPairs) return false;
+    if (g.type == TOS_POLAR || p->n_pairs < kTileMinPairs) return false;
     if (cat->ladder.state == 2 || p->tiles.state == 2) return false;
     // the edge bound needs squared separations well above their rounding
     if (!(cat->dmin > 1e-3) || cat->dmax > 1e5) return false;

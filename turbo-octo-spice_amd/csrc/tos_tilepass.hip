@@ -32,6 +32,12 @@
 // Measured, us per pass, general kernel / this one: 3,450 sightline pairs 551
 // / 273; 1.47 million (1.3e10 pixel pairs) FP64 24620 / 6990; 37 million
 // (3.3e11) 336,000 / 159,000; Observing, 1.3 million pairs 13730 / 5290.
+//
+// With seven sums a second instruction forms (w d)1, (w d)2, w1 and w2 as
+// products by 1, exactly; the mean wavelength is one number per cell.  141,344
+// pairs, 50 x 50 x 3 bins in four bands: 65,110 / 5,230 us (the general kernel
+// makes three full passes with eight atomics per pixel pair; here a band takes
+// the tiles it has cells in).
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -127,6 +133,7 @@ __device__ __forceinline__ SlowBin slow_cart(const GridExact &ge, uint32_t band_
 template <int NSUM>
 struct Cell {                          // one (k1, k2) of a lane
     double dd, ww;                     // running sums
+    double x[NSUM == 7 ? 4 : 1];       // (w d)1, (w d)2, w1, w2
     float n;                           // pairs in them (exact: below 2^24)
     uint32_t off8;                     // LDS byte offset of their slot, kReject: none
     float thr;                         // K of the next edge (lower bound); < 0: bin every pair exactly
@@ -163,6 +170,9 @@ __device__ __forceinline__ void tile_block(const XiKernelArgs &a, size_t part_ro
     // register r of the result holds the steps 4 r + g of its four lane groups
     const uint32_t lane_a = 16u * (4u * (col & 3) + (col >> 2)) + 4u * g;
     const uint32_t lane_b = 16u * col + 4u * g;
+    // the second instruction's blocks: (w d)1 1, 1 (w d)2, w1 1, 1 w2
+    const uint32_t lane_a2 = lane_a - 4u * g + 4u * (g == 0 ? 1 : g == 2 ? 0 : 2);
+    const uint32_t lane_b2 = lane_b - 4u * g + 4u * (g == 1 ? 1 : g == 3 ? 0 : 2);
     const TOS_GLOBAL char *pixels = global<char>(t.pix);
     const TOS_GLOBAL float *step_d = global<float>(t.d), *step_l = global<float>(t.l);
     const TOS_GLOBAL uint4_v *records = global<uint4_v>(t.rec);
@@ -195,13 +205,19 @@ __device__ __forceinline__ void tile_block(const XiKernelArgs &a, size_t part_ro
         float inv_dd[4];               // Cartesian: (1 - eps) / (d1 d2), pair_base
         float base[4];
         uint32_t f0[4];                // Observing: flat bin of the cell at theta bin 0
+        float lsum[4];                 // seven sums: loglam1 + loglam2
         Cell<NSUM> cell[4];
         bool any = false;
+        auto clear = [](Cell<NSUM> &c) {
+            c.dd = c.ww = 0.0;
+            if constexpr (NSUM == 7) c.x[0] = c.x[1] = c.x[2] = c.x[3] = 0.0;
+            c.n = 0.0f;
+        };
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const float d1 = step_d[16 * b1 + 4 * r + g], l1 = step_l[16 * b1 + 4 * r + g];
-            cell[r].dd = cell[r].ww = 0.0;
-            cell[r].n = 0.0f;
+            clear(cell[r]);
+            if constexpr (NSUM == 7) lsum[r] = l1 + l2;
             cell[r].off8 = kReject;
             cell[r].edge = 0.0f;
             const double x0 = (double)(COORD == TOS_OBSERVING ? fabsf(l1 - l2) : fabsf(d1 - d2));
@@ -228,12 +244,17 @@ __device__ __forceinline__ void tile_block(const XiKernelArgs &a, size_t part_ro
 
         auto empty = [&](Cell<NSUM> &c, uint32_t n) {
             neval += n;
-            c.dd = c.ww = 0.0;
-            c.n = 0.0f;
+            clear(c);
         };
-        auto flush = [&](Cell<NSUM> &c) {
+        auto add = [&](const Cell<NSUM> &c, uint32_t n, float ls) {
+            H.add8n(c.off8, n, c.dd, c.ww);
+            // every pair of a cell has the same mean wavelength
+            if constexpr (NSUM == 7)
+                H.add8n_more(c.off8, c.x[0], c.x[1], c.x[2], c.x[3], (double)n * (0.5 * (double)ls));
+        };
+        auto flush = [&](Cell<NSUM> &c, float ls) {
             const uint32_t n = (uint32_t)c.n;
-            if (n > 0u && c.off8 < a.band_len8) H.add8n(c.off8, n, c.dd, c.ww);
+            if (n > 0u && c.off8 < a.band_len8) add(c, n, ls);
             empty(c, n);
         };
         // K reaches the threshold of some cell of the wavefront: cells that
@@ -249,7 +270,7 @@ __device__ __forceinline__ void tile_block(const XiKernelArgs &a, size_t part_ro
                 if (c.thr <= K && __float_as_uint(c.thr) <= kb_safe) {
                     const uint32_t n = (uint32_t)c.n;
                     // (a band of a larger grid holds a part of the slots)
-                    if (FIXED || c.off8 < a.band_len8) H.add8n(c.off8, n, c.dd, c.ww);
+                    if (FIXED || c.off8 < a.band_len8) add(c, n, lsum[r]);
                     empty(c, n);
                     const bool out = c.edge >= (float)ge.n[1];
                     c.off8 = out ? kReject : c.off8 + ge.nz8;
@@ -267,7 +288,7 @@ __device__ __forceinline__ void tile_block(const XiKernelArgs &a, size_t part_ro
                 for (int r = 0; r < 4; ++r)
                     if (cell[r].thr <= K) {
                         slow |= 1u << r;
-                        flush(cell[r]);
+                        flush(cell[r], lsum[r]);
                     }
                 // one copy of the code for the four cells
 #pragma unroll 1
@@ -295,13 +316,13 @@ __device__ __forceinline__ void tile_block(const XiKernelArgs &a, size_t part_ro
         auto turn = [&](uint32_t th) {
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                flush(cell[r]);
+                flush(cell[r], lsum[r]);
                 const uint32_t f = f0[r] + th * ge.n[2];
                 cell[r].off8 = cell[r].thr < 0.0f && f < ge.ntot ? 8u * slot_of(ge, f) - a.band_lo8 : kReject;
             }
             theta = th;
         };
-        auto visit = [&](float A, float B) {
+        auto visit = [&](float A, float B, float A2, float B2) {
             const float16_v zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
             const float16_v D = __builtin_amdgcn_mfma_f32_16x16x1f32(A, B, zero, 0, 0, 0);
 #pragma unroll
@@ -310,8 +331,17 @@ __device__ __forceinline__ void tile_block(const XiKernelArgs &a, size_t part_ro
                 cell[r].dd += (double)D[4 + r];
                 cell[r].n += D[8 + r];
             }
+            if constexpr (NSUM == 7) {
+                const float16_v E = __builtin_amdgcn_mfma_f32_16x16x1f32(A2, B2, zero, 0, 0, 0);
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) cell[r].x[j] += (double)E[4 * j + r];
+            }
         };
         auto load_a = [&](uint32_t off) { return *(const TOS_GLOBAL float *)(pixels + (off + lane_a)); };
+        auto load_a2 = [&](uint32_t off) { return NSUM == 7 ? *(const TOS_GLOBAL float *)(pixels + (off + lane_a2)) : 0.f; };
+        auto load_b2 = [&](uint32_t off) { return NSUM == 7 ? *(const TOS_GLOBAL float *)(pixels + (off + lane_b2)) : 0.f; };
         auto load_b = [&](uint32_t off) { return *(const TOS_GLOBAL float *)(pixels + (off + lane_b)); };
 
         // the batch's pairs that cover the tile: the words of 64 pairs whose
@@ -371,12 +401,14 @@ __device__ __forceinline__ void tile_block(const XiKernelArgs &a, size_t part_ro
             }
             // four entries at a time; each operand register is loaded for the
             // entry four ahead as soon as its visit is done
-            float A[4], B[4];
+            float A[4], B[4], A2[4], B2[4];
             uint32_t Z[4];             // K, or the theta bin
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 A[q] = load_a(queue[q].x);
                 B[q] = load_b(queue[q].y);
+                A2[q] = load_a2(queue[q].x);
+                B2[q] = load_b2(queue[q].y);
                 Z[q] = queue[q].z;
             }
             if (COORD == TOS_OBSERVING && fresh) {
@@ -393,9 +425,11 @@ __device__ __forceinline__ void tile_block(const XiKernelArgs &a, size_t part_ro
                     } else {
                         if (__any(next <= __uint_as_float(Z[q]))) cross(__uint_as_float(Z[q]), queue[k + q].w);
                     }
-                    visit(A[q], B[q]);
+                    visit(A[q], B[q], A2[q], B2[q]);
                     A[q] = load_a(xa);
                     B[q] = load_b(xb);
+                    A2[q] = load_a2(xa);
+                    B2[q] = load_b2(xb);
                     Z[q] = xk;
                 }
             }
@@ -410,7 +444,7 @@ __device__ __forceinline__ void tile_block(const XiKernelArgs &a, size_t part_ro
             if (COORD == TOS_CARTESIAN && !__any(next < __builtin_inff())) break;
         }
 #pragma unroll
-        for (int r = 0; r < 4; ++r) flush(cell[r]);
+        for (int r = 0; r < 4; ++r) flush(cell[r], lsum[r]);
     }
 
     if (nre) __hip_atomic_fetch_add(&ctl.recheck, (unsigned long long)nre, __ATOMIC_RELAXED,
@@ -433,9 +467,11 @@ __device__ __forceinline__ void tile_block(const XiKernelArgs &a, size_t part_ro
     }
 }
 
+// The seven sums take twice the vector registers and their histogram leaves
+// room for one workgroup of eight wavefronts on a CU.
 template <int COORD, int NSUM, bool FIXED>
-__global__ void __launch_bounds__(kTileBlockMax) __attribute__((amdgpu_waves_per_eu(4, 4)))
-tile_pass_kernel(XiKernelArgs a)
+__global__ void __launch_bounds__(NSUM == 7 ? 512 : kTileBlockMax)
+__attribute__((amdgpu_waves_per_eu(NSUM == 7 ? 2 : 4, NSUM == 7 ? 2 : 4))) tile_pass_kernel(XiKernelArgs a)
 {
     tile_block<COORD, NSUM, FIXED>(a, blockIdx.x);
 }
@@ -466,27 +502,33 @@ hipError_t launch_one(void (*fn)(A), const A &a, int n_wg, int block, size_t lds
 
 bool tile_fixed(int nslots) { return (uint32_t)nslots <= kFixedSlots; }
 
-// 512 threads where two workgroups share a CU's LDS, else 1024: 16
-// wavefronts per CU either way (128 vector registers).
-int tile_block_size(int nslots) { return tile_fixed(nslots) ? 512 : 1024; }
+int tile_threads_per_cu(int nsum) { return nsum == 7 ? 512 : 1024; }
 
-size_t tile_lds_bytes(int nslots)
+// 512 threads where two workgroups share a CU's LDS, else 1024: 16
+// wavefronts per CU either way (128 vector registers); 512 with seven sums.
+int tile_block_size(int nsum, int nslots) { return nsum == 7 || tile_fixed(nslots) ? 512 : 1024; }
+
+size_t tile_lds_bytes(int nsum, int nslots)
 {
-    const bool fixed = tile_fixed(nslots);
-    const size_t hist = fixed ? hist_bytes<2, true>(nslots) : hist_bytes<2, false>(nslots);
+    const size_t hist = nsum == 7           ? hist_bytes<7, false>(nslots)
+                        : tile_fixed(nslots) ? hist_bytes<2, true>(nslots)
+                                             : hist_bytes<2, false>(nslots);
     return ((hist + 15) & ~(size_t)15) + kTileCtlBytes +
-           (size_t)(tile_block_size(nslots) / kWave) * kQueue * sizeof(uint4);
+           (size_t)(tile_block_size(nsum, nslots) / kWave) * kQueue * sizeof(uint4);
 }
 
-int launch_tile_pass(int coord, const XiKernelArgs &a, int n_wg, int block, size_t lds, void *stream)
+int launch_tile_pass(int coord, int nsum, const XiKernelArgs &a, int n_wg, int block, size_t lds, void *stream)
 {
     hipStream_t st = (hipStream_t)stream;
     const bool fixed = !a.banded && tile_fixed((int)a.ge.nslots);
-    if (coord == TOS_OBSERVING)
-        return (int)(fixed ? launch_one(tile_pass_kernel<TOS_OBSERVING, 2, true>, a, n_wg, block, lds, st)
-                           : launch_one(tile_pass_kernel<TOS_OBSERVING, 2, false>, a, n_wg, block, lds, st));
-    return (int)(fixed ? launch_one(tile_pass_kernel<TOS_CARTESIAN, 2, true>, a, n_wg, block, lds, st)
-                       : launch_one(tile_pass_kernel<TOS_CARTESIAN, 2, false>, a, n_wg, block, lds, st));
+    void (*fn)(XiKernelArgs);
+    if (nsum == 7)
+        fn = coord == TOS_OBSERVING ? tile_pass_kernel<TOS_OBSERVING, 7, false> : tile_pass_kernel<TOS_CARTESIAN, 7, false>;
+    else if (coord == TOS_OBSERVING)
+        fn = fixed ? tile_pass_kernel<TOS_OBSERVING, 2, true> : tile_pass_kernel<TOS_OBSERVING, 2, false>;
+    else
+        fn = fixed ? tile_pass_kernel<TOS_CARTESIAN, 2, true> : tile_pass_kernel<TOS_CARTESIAN, 2, false>;
+    return (int)launch_one(fn, a, n_wg, block, lds, st);
 }
 
 int launch_tile_batch(int coord, bool fixed, const XiBatchArgs &b, int n_wg, int block, size_t lds, void *stream)

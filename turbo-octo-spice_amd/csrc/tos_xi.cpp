@@ -226,17 +226,18 @@ int plan_launch(tos_ctx *ctx, const tos_xi_opts *opts, int prec, int accum, cons
     return TOS_OK;
 }
 
-bool plan_tiles(tos_ctx *ctx, const tos_pairs *p, const tos_grid &g, XiKernelArgs &a, XiLaunch &L, uint32_t band_rows)
+bool plan_tiles(tos_ctx *ctx, const tos_pairs *p, int accum, const tos_grid &g, XiKernelArgs &a, XiLaunch &L,
+                uint32_t band_rows)
 {
     GridExact ge;
     grid_exact_consts(g, ge);
     const bool banded = band_rows > 0 && band_rows < ge.n[0];
     const int slots = banded ? (int)(band_rows * (ge.rowlen + ge.pad)) : (int)ge.nslots;
     L.nbins = banded ? (int)(band_rows * ge.rowlen) : (int)ge.ntot;
-    L.nsum = 2;
-    L.lds = tile_lds_bytes(slots);
-    L.block = tile_block_size(slots);
-    L.n_wg = tile_workgroups(p, a.tile, ctx->ncu * (2048 / kTileBlockMax), L.block);
+    L.nsum = xi_nsum(accum);
+    L.lds = tile_lds_bytes(L.nsum, slots);
+    L.block = tile_block_size(L.nsum, slots);
+    L.n_wg = tile_workgroups(p, a.tile, ctx->ncu * tile_threads_per_cu(L.nsum) / L.block, L.block);
     L.n_seg = std::min(32, L.n_wg);
     return (int64_t)L.n_wg * L.nbins * (4 + 8 * L.nsum) <= kMaxPartialBytes;
 }
@@ -248,7 +249,7 @@ uint32_t band_rows_for(const tos_ctx *ctx, int accum, const tos_grid &g, bool ti
     const uint32_t rowslots = ge.rowlen + ge.pad;
     auto fits = [&](uint32_t rows) {
         const int slots = (int)(rows * rowslots);
-        return (int64_t)(tiles ? tile_lds_bytes(slots) : xi_lds_bytes(accum, slots)) + 64 <= ctx->max_lds_block;
+        return (int64_t)(tiles ? tile_lds_bytes(xi_nsum(accum), slots) : xi_lds_bytes(accum, slots)) + 64 <= ctx->max_lds_block;
     };
     if (fits(ge.n[0])) return ge.n[0];
     uint32_t lo = 0, hi = ge.n[0];   // the most rows that fit
@@ -356,7 +357,7 @@ extern "C" int tos_xi_run(tos_ctx *ctx, const tos_catalog *cat, const tos_pairs 
     // the tile path: catalogues on a ladder, no work scheme switched off and
     // no launch shape asked for
     bool tiles = flags == 0 && (!opts || (opts->block_size == 0 && opts->blocks_per_cu == 0 && opts->wg_per_slot == 0)) &&
-                 tile_job(cat, p, g, accum);
+                 tile_job(cat, p, g);
     XiKernelArgs a;
     if (tiles) {
         if ((rc = ensure_tile_plan(ctx, p)) != TOS_OK) return rc;
@@ -385,7 +386,7 @@ extern "C" int tos_xi_run(tos_ctx *ctx, const tos_catalog *cat, const tos_pairs 
     // one full pass over the pairs per band
     uint32_t rows = band_rows_for(ctx, accum, g, tiles);
     XiLaunch L;
-    if (tiles && (rows == 0 || !plan_tiles(ctx, p, g, a, L, rows))) {
+    if (tiles && (rows == 0 || !plan_tiles(ctx, p, accum, g, a, L, rows))) {
         tiles = false;
         rows = band_rows_for(ctx, accum, g);
     }
@@ -440,7 +441,7 @@ extern "C" int tos_xi_run(tos_ctx *ctx, const tos_catalog *cat, const tos_pairs 
         }
         if (tiles && r0 > 0 && (e = launch_zero_u64(a.n_recheck + 2, 1, ctx->stream)) != hipSuccess)
             return hip_fail(ctx, (hipError_t)e, "tile counter clear");
-        e = tiles ? launch_tile_pass(g.type, a, L.n_wg, L.block, L.lds, ctx->stream)
+        e = tiles ? launch_tile_pass(g.type, L.nsum, a, L.n_wg, L.block, L.lds, ctx->stream)
                   : launch_xi(g.type, prec, accum, a, L.n_wg, L.block, L.lds, ctx->stream);
         if (e != hipSuccess) return hip_fail(ctx, (hipError_t)e, "xi kernel launch");
         if (!banded) hipEventRecord(ctx->ev1, ctx->stream);   // the pair kernel alone
