@@ -62,3 +62,24 @@ def test_many_pixels(dev):
     dc, _ = synth.cosmo_distances(10.0 ** (uniq.astype(np.float64) - math.log10(1216.0)) - 1.0, 0.7, 0.3)
     u = ulps(d, dc.astype(np.float32)[inv])
     assert u.max() <= 1 and (u == 0).mean() >= 0.999
+
+
+@pytest.mark.parametrize("n", [1, 63, 65, 1023, 1025, 4095, 4096, 4097, 8192, 20001])
+def test_distinct_wavelengths_and_repeated_ones(dev, n):
+    """A call's distinct wavelengths take one evaluation each up to a limit
+    and one per pixel beyond: both give the bits of small calls."""
+    rng = np.random.default_rng(n)
+    uniq = np.unique(rng.uniform(3.3, 3.75, 2 * n).astype(np.float32))[:n]
+    rng.shuffle(uniq)
+    small = np.concatenate([dev.pixel_distances(uniq[s:s + 300]) for s in range(0, len(uniq), 300)])
+    assert np.array_equal(dev.pixel_distances(uniq), small)
+    pick = rng.integers(0, len(uniq), 3 * n + 7)
+    assert np.array_equal(dev.pixel_distances(uniq[pick]), small[pick])
+    # signed zeros, infinities and NaNs of every payload among them
+    odd = np.array([0.0, -0.0, np.inf, -np.inf, np.nan], np.float32)
+    odd = np.concatenate([odd, np.array([0xffffffff, 0x7f800001], np.uint32).view(np.float32)])
+    d = dev.pixel_distances(np.concatenate([uniq, odd]))
+    assert np.array_equal(d[:len(uniq)], small)
+    for x, y in zip(odd, d[len(uniq):]):
+        one = dev.pixel_distances(np.array([x], np.float32))[0]
+        assert one == y or (math.isnan(one) and math.isnan(y))

@@ -71,36 +71,47 @@ TOS_HD double hubble_e(double ol, double om, double z)
     return sqrt(om * a * a * a + ok * a * a + ol);
 }
 
-// D_C(z) in Mpc/h.
-TOS_HD double los_comoving(double ol, double om, double z)
+constexpr int kLosPanels = 64;
+constexpr int kLosTerms = 8 * kLosPanels;
+constexpr double kLosScale = 2997.92458;   // c/H0 in Mpc/h
+
+// Term t of the integral: node t mod 8 of panel t / 8, panels of width h.
+TOS_HD double los_term(double ol, double om, double h, int t)
 {
     const double xg[8] = {-0.9602898564975363, -0.7966664774136267, -0.5255324099163290, -0.1834346424956498,
                           0.1834346424956498,  0.5255324099163290,  0.7966664774136267,  0.9602898564975363};
     const double wg[8] = {0.1012285362903763, 0.2223810344533745, 0.3137066458778873, 0.3626837833783620,
                           0.3626837833783620, 0.3137066458778873, 0.2223810344533745, 0.1012285362903763};
-    const double c_over_h0 = 2997.92458;
-    if (z == 0) return 0.0;
-    const double L = log1p_rn(z);
-    const int panels = 64;
-    const double h = L / panels;
-    double acc = 0;
-    for (int p = 0; p < panels; ++p) {
-        const double mid = (p + 0.5) * h;
-        for (int k = 0; k < 8; ++k) {
-            const double x = mid + 0.5 * h * xg[k];
-            const double a = exp_rn(x);   // 1 + z'
-            acc += wg[k] * a / hubble_e(ol, om, a - 1.0);
-        }
-    }
-    return c_over_h0 * acc * 0.5 * h;
+    const int k = t & 7;
+    const double mid = ((t >> 3) + 0.5) * h;
+    const double x = mid + 0.5 * h * xg[k];
+    const double a = exp_rn(x);   // 1 + z'
+    return wg[k] * a / hubble_e(ol, om, a - 1.0);
 }
 
-// The pixel distance of h5healxi.cc:200-203: D_C(10^(loglam - log10 Lya) - 1)
-// (loglamToRedshift, h5healxi.cc:38-40), rounded to the pixel's float.
+// D_C(z) in Mpc/h.
+TOS_HD double los_comoving(double ol, double om, double z)
+{
+    if (z == 0) return 0.0;
+    const double h = log1p_rn(z) / kLosPanels;
+    double acc = 0;
+    for (int p = 0; p < kLosTerms; p += 8)
+        for (int k = 0; k < 8; ++k) acc += los_term(ol, om, h, p + k);
+    return kLosScale * acc * 0.5 * h;
+}
+
+// z of a pixel: 10^(loglam - log10 Lya) - 1 (loglamToRedshift,
+// h5healxi.cc:38-40).
+TOS_HD double pixel_redshift(double log_lya, float loglam)
+{
+    return exp_rn(((double)loglam - log_lya) * 2.30258509299404568402) - 1.0;
+}
+
+// The pixel distance of h5healxi.cc:200-203: D_C(z), rounded to the pixel's
+// float.
 TOS_HD float pixel_distance(double ol, double om, double log_lya, float loglam)
 {
-    const double z = exp_rn(((double)loglam - log_lya) * 2.30258509299404568402) - 1.0;
-    return (float)los_comoving(ol, om, z);
+    return (float)los_comoving(ol, om, pixel_redshift(log_lya, loglam));
 }
 
 #undef TOS_HD
