@@ -168,3 +168,60 @@ def test_seven_sums_equal_the_general_kernel(dev, field, spec):
     assert signed_sum_err(h.extra["dj"], ref.extra["dj"], ref.extra["wj"]) <= SUM_RTOL
     pairs.free()
     dcat.free()
+
+
+# mu axes that end inside [0, 1], start above 0 or below it, finer than the
+# r axis; r axes that start above 0 or below it, narrower than a tile's
+# spread, in several LDS bands; z axes with several bins or left
+POLAR_GRIDS = [
+    ("[0:200]*50", "[0:1]*20", "[3.556:3.735]*1"),
+    ("[0:200]*50", "[0:1]*20", "[3.556:3.735]*3"),
+    ("[20:150]*13", "[0.1:0.9]*7", "[3.556:3.735]*2"),
+    ("[-5:90]*19", "[-0.3:0.5]*8", "[3.556:3.735]*1"),
+    ("[0:200]*3", "[0:1]*500", "[3.556:3.735]*1"),
+    ("[0:200]*400", "[0:1]*3", "[3.556:3.735]*1"),
+    ("[0:200]*100", "[0:1]*100", "[3.556:3.735]*1"),
+    ("[0:1.5]*3", "[0:1]*4", "[3.556:3.735]*1"),
+    ("[0:200]*20", "[0:1]*1", "[0.6:3.0]*3"),
+    ("[0:200]*20", "[0.5:0.9]*1", "[4.6:5.0]*2"),
+    ("[0:200]*64", "[0:1.5]*16", "[3.556:3.735]*1"),
+]
+
+
+@pytest.mark.parametrize("spec", POLAR_GRIDS, ids=["-".join(s) for s in POLAR_GRIDS])
+def test_polar_tile_pass_equals_the_general_kernel(dev, field, spec):
+    grid = GridSpec.from_specs(tos_amd.POLAR, *spec)
+    dcat = dev.upload(field)
+    pairs = dcat.pairs(GridSpec.polar().max_angular_scale(field.scale), order=3, nthreads=8)
+    assert pairs.stats()["num_sightline_pairs_used"] > 20000
+    for prec in (tos_amd.FP64, tos_amd.FP32C):
+        print(f"case: polar grid {grid.specs} precision {prec}", flush=True)
+        ref = pairs.run(grid, precision=prec, flags=tos_amd.XI_NO_ZCONST)
+        h = pairs.run(grid, precision=prec)
+        close(h, ref.num_pairs, {"didj": ref.didj, "wgt": ref.wgt})
+        assert h.num_pixel_pairs_used == ref.num_pixel_pairs_used
+    ref = pairs.run(grid, precision=tos_amd.FP64, accum=tos_amd.ACC_ALL, flags=tos_amd.XI_NO_ZCONST)
+    h = pairs.run(grid, precision=tos_amd.FP64, accum=tos_amd.ACC_ALL)
+    close(h, ref.num_pairs, {"didj": ref.didj, "wgt": ref.wgt})
+    for k in ("wi", "wj", "z"):
+        assert rel_err(h.extra[k], ref.extra[k]) <= SUM_RTOL, k
+    pairs.free()
+    dcat.free()
+
+
+def test_polar_tile_pass_against_the_oracle(dev, field):
+    from oracle import oracle as ora
+    grid = GridSpec.from_specs(tos_amd.POLAR, *POLAR_GRIDS[1])
+    ref = ora.xi_run(field, grid, field.scale, order=3, nthreads=8)
+    dcat = dev.upload(field)
+    pairs = dcat.pairs(grid.max_angular_scale(field.scale), order=3, nthreads=8)
+    for prec in (tos_amd.FP64, tos_amd.FP32C):
+        print(f"case: polar grid {grid.specs} precision {prec}", flush=True)
+        close(pairs.run(grid, precision=prec), ref["raw"]["num_pairs"], ref["raw"])
+    jobs = [(pairs, grid, tos_amd.FP64), (pairs, GridSpec.polar(), tos_amd.FP32C)]
+    h = dev.batch_run(jobs)[0]
+    close(h[0], ref["raw"]["num_pairs"], ref["raw"])
+    one = pairs.run(GridSpec.polar(), precision=tos_amd.FP64, flags=tos_amd.XI_NO_ZCONST)
+    close(h[1], one.num_pairs, {"didj": one.didj, "wgt": one.wgt})
+    pairs.free()
+    dcat.free()

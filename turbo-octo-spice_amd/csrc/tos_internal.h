@@ -56,7 +56,7 @@ struct GridExact {
     uint32_t nslots;      // n0 * (rowlen + pad)
     uint32_t row8;        // 8 (rowlen + pad): byte stride of an axis-0 row of FP64 sums
     uint32_t nz8;         // 8 n2
-    double width1;        // axis-1 bin width
+    double width0, width1;   // bin widths of axes 0 and 1
 };
 
 // Constants of the FP32 fast path with its guard band.  The kernel forms

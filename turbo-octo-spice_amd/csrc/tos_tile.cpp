@@ -224,10 +224,18 @@ constexpr int64_t kTileMinPairs = 400;
 
 bool tile_job(const tos_catalog *cat, const tos_pairs *p, const tos_grid &g)
 {
-    if (g.type == TOS_POLAR || p->n_pairs < kTileMinPairs) return false;
+    if (p->n_pairs < kTileMinPairs) return false;
     if (cat->ladder.state == 2 || p->tiles.state == 2) return false;
     // the edge bound needs squared separations well above their rounding
     if (!(cat->dmin > 1e-3) || cat->dmax > 1e5) return false;
+    // bins far past an axis stay there: the reference's cast wraps only
+    // beyond 2^31 of them
+    auto wraps = [&](double top, int k) { return (top + std::fabs(g.min[k])) / g.width[k] > 1e9; };
+    if (g.type == TOS_CARTESIAN) return !wraps(2.0 * cat->dmax, 1);
+    // Polar: |d1 - d2| exact, two bin numbers in one word
+    if (g.type == TOS_POLAR)
+        return cat->dmax <= 2.0 * cat->dmin && g.nbins[0] < 65000 && g.nbins[1] < 65000 && !wraps(2.0 * cat->dmax, 0) &&
+               !wraps(1.0, 1);
     return true;
 }
 
@@ -265,9 +273,23 @@ bool tile_args(const tos_pairs *p, const tos_grid &g, XiKernelArgs &a)
     //   and their product)
     //   + (7e-15 dmax^2 (the reference's FP64 rounding of r^2) + 2^-24 base) / 4,
     // base <= ulp32(dmax^2) + 2 * 2^-24 dmax * axis-0 range; doubled
+    // (Polar: base <= ulp32(dmax^2), six more roundings in the threshold, and
+    // r^2 = r_par^2 / mu^2 as the reference's rounded mu, of at least (smallest
+    // step) / R, has it)
     const double u = std::ldexp(1.0, -24);
-    const double base = 2.0 * u * cat->dmax * cat->dmax + 4.0 * u * cat->dmax * std::fabs(g.max[0]);
-    t.eps = 2.0 * (4.0 * u + (7e-15 * cat->dmax * cat->dmax + u * base) / 4.0);
+    double base = 2.0 * u * cat->dmax * cat->dmax + 4.0 * u * cat->dmax * std::fabs(g.max[0]);
+    double ops = 4.0, abs_err = 7e-15 * cat->dmax * cat->dmax;
+    if (g.type == TOS_POLAR) {
+        base = 2.0 * u * cat->dmax * cat->dmax;
+        ops = 10.0;
+        double step = INFINITY;
+        for (size_t k = 1; k < L.h_d.size(); ++k)
+            if (L.h_d[k] > L.h_d[k - 1]) step = std::min(step, (double)L.h_d[k] - (double)L.h_d[k - 1]);
+        const double R = std::fabs(g.min[0]) + g.nbins[0] * g.width[0];
+        const double M = 1.0 + std::fabs(g.min[1]) + g.nbins[1] * g.width[1];
+        abs_err += 1e-15 * R * R * (4.0 + M * R / step);
+    }
+    t.eps = 2.0 * (ops * u + (abs_err + u * base) / 4.0);
     t.ulps = (uint32_t)std::ceil(2.2 * t.eps / u) + 2;
     return t.eps < 1e-4;
 }

@@ -130,21 +130,127 @@ __device__ __forceinline__ SlowBin slow_cart(const GridExact &ge, uint32_t band_
     return s;
 }
 
-template <int NSUM>
+// Polar: r^2 = K d1 d2 + r_par^2 + base, where base = f32(d1^2) - d1^2 since
+// |d1 - d2| is exact (tile_job asks for dmax <= 2 dmin).  Each (k1, k2) meets
+// the edges of r upwards and those of mu = r_par / r downwards.
+struct PolarStep {
+    double rr, base;                   // r_par^2, base
+    float rpar, inv;                   // inv = (1 - eps) / (d1 d2)
+};
+
+__device__ __forceinline__ PolarStep polar_step(float d1, float d2, float keep)
+{
+    PolarStep p;
+    const float sq = d1 * d1;
+    p.base = (double)-__builtin_fmaf(d1, d1, -sq);
+    p.rpar = fabsf(d1 - d2);
+    p.rr = (double)p.rpar * (double)p.rpar;
+    p.inv = keep * __builtin_amdgcn_rcpf(d1 * d2);
+    return p;
+}
+
+// K of r edge e (in bins), lowered by its error bound
+__device__ __forceinline__ float polar_kr(const GridExact &ge, const PolarStep &p, float e)
+{
+    const double s = __builtin_fma((double)e, ge.width0, ge.min[0]);
+    return (float)(__builtin_fma(s, s, -p.rr) - p.base) * p.inv;
+}
+
+// K of mu edge m (in bins), lowered by its error bound; none below mu = 0,
+// nor for two pixels at one distance (mu = 0)
+__device__ __forceinline__ float polar_km(const GridExact &ge, const PolarStep &p, float m)
+{
+    const double mu = __builtin_fma((double)m, ge.width1, ge.min[1]);
+    if (!(mu > 0.0) || p.rpar == 0.0f) return __builtin_inff();
+    double y = __builtin_amdgcn_rcp(mu);
+    y = __builtin_fma(__builtin_fma(-mu, y, 1.0), y, y);
+    y = __builtin_fma(__builtin_fma(-mu, y, 1.0), y, y);
+    const double r = (double)p.rpar * y;
+    return (float)(__builtin_fma(r, r, -p.rr) - p.base) * p.inv;
+}
+
+struct SlowPolar {
+    uint32_t off8, edges;
+    float kr, km;
+};
+
+// The next edges of a cell: r edge e (in bins) and mu edge m >= -1.
+__device__ __forceinline__ uint32_t polar_pack(float e, float m)
+{
+    return (uint32_t)(int32_t)e | ((uint32_t)((int32_t)m + 1) << 16);
+}
+__device__ __forceinline__ float polar_e(uint32_t edges) { return (float)(edges & 0xffffu); }
+__device__ __forceinline__ float polar_m(uint32_t edges) { return (float)((int32_t)(edges >> 16) - 1); }
+
+__device__ __forceinline__ SlowPolar slow_polar(const GridExact &ge, uint32_t band_lo8, float d1, float l1, float d2,
+                                                float l2, double c, float keep, float K, float k_safe)
+{
+    const double d2d = (double)d2;
+    const double r1_sq = (double)(d1 * d1), two = (double)(2.0f * d1) * c;
+    const uint32_t slot = exact_bin_polar(ge, d1, l1, r1_sq, two, d2, l2, false, 0);
+    const PolarStep p = polar_step(d1, d2, keep);
+    const double r_sq = r1_sq + (d2d - two) * d2d;
+    const double r = sqrt_no_tiny(r_sq);
+    const double t0 = (r - ge.min[0]) * ge.inv[0], t1 = ((double)p.rpar / r - ge.min[1]) * ge.inv[1];
+    const double n0 = (double)ge.n[0], n1 = (double)ge.n[1];
+    // the edges around t0 and t1 (the cast truncates: (-1, 1) is one bin)
+    const double lo0 = t0 >= n0 ? n0 : t0 >= 1.0 ? floor(t0) : -1.0;
+    const double up0 = floor(t0 < 0.0 ? 0.0 : t0) + 1.0;
+    const double lo1 = t1 >= n1 ? n1 : t1 >= 1.0 ? floor(t1) : -1.0;
+    const double up1 = t1 <= -1.0 ? -1.0 : floor(t1 < 0.0 ? 0.0 : t1) + 1.0;
+    const bool no_lo0 = __builtin_fma(lo0, ge.width0, ge.min[0]) <= 0.0;
+    const float k0 = no_lo0 ? -1.0f : polar_kr(ge, p, (float)lo0);
+    const float k1 = t1 >= n1 || p.rpar == 0.0f ? -1.0f : polar_km(ge, p, (float)up1);
+    const float kr = polar_kr(ge, p, (float)up0), km = polar_km(ge, p, (float)lo1);
+    const bool dead = t0 >= n0 || t1 <= -1.0;
+    const uint32_t iz = z_bin_exact(ge, l1, l2);
+    const bool settled = r_sq - p.rr >= 4.0 && t0 > -1.0 && k0 <= k_safe && k1 <= k_safe && iz < ge.n[2] &&
+                         (dead || (K < kr && K < km));
+    SlowPolar s;
+    if (!settled) {
+        s.off8 = slot == kReject ? kReject : (slot << 3) - band_lo8;
+        s.edges = 0u;                  // m = -1: in the mu axis
+        s.kr = -1.0f;
+        s.km = __builtin_inff();
+    } else if (dead) {
+        s.off8 = kReject;
+        s.edges = 0u;
+        s.kr = s.km = __builtin_inff();
+    } else {
+        // above the mu axis (lo1 = n1) the slot is that of a bin past the row
+        const uint32_t i1 = t1 >= n1 ? ge.n[1] : (uint32_t)(int32_t)t1;
+        s.off8 = (slot3(ge, (uint32_t)(int32_t)t0, i1, iz) << 3) - band_lo8;
+        s.edges = polar_pack((float)up0, (float)lo1);
+        s.kr = kr;
+        s.km = km;
+    }
+    return s;
+}
+
+template <int NSUM, bool POLAR>
 struct Cell {                          // one (k1, k2) of a lane
     double dd, ww;                     // running sums
     double x[NSUM == 7 ? 4 : 1];       // (w d)1, (w d)2, w1, w2
     float n;                           // pairs in them (exact: below 2^24)
     uint32_t off8;                     // LDS byte offset of their slot, kReject: none
-    float thr;                         // K of the next edge (lower bound); < 0: bin every pair exactly
+    float thr;                         // K of the next edge (lower bound; Polar: of r); < 0: bin every pair exactly
     float edge;                        // that edge, in bins
+    float km;                          // Polar: K of the next edge of mu
+    uint32_t edges;                    // Polar: the next edges of both axes, in bins
+
+    __device__ __forceinline__ float at() const { return POLAR ? fminf(thr, km) : thr; }
+    // the running sums have a slot (Polar: mu is not above its axis)
+    __device__ __forceinline__ bool in_axis(const GridExact &ge) const { return !POLAR || (edges >> 16) <= ge.n[1]; }
 };
 
 template <int COORD, int NSUM, bool FIXED>
 __device__ __forceinline__ void tile_block(const XiKernelArgs &a, size_t part_row)
 {
+    constexpr bool POLAR = COORD == TOS_POLAR;
+    using CellT = Cell<NSUM, POLAR>;
     const GridExact &ge = a.ge;
     const TileArgs &t = a.tile;
+    const float keep = (float)(1.0 - t.eps);
     extern __shared__ double lds_tile[];
     const uint32_t nslots = FIXED ? ge.nslots : a.band_len8 / 8u;
     const Hist<NSUM, FIXED> H(lds_tile, nslots);
@@ -204,11 +310,12 @@ __device__ __forceinline__ void tile_block(const XiKernelArgs &a, size_t part_ro
         const float d2 = step_d[16 * b2 + col], l2 = step_l[16 * b2 + col];
         float inv_dd[4];               // Cartesian: (1 - eps) / (d1 d2), pair_base
         float base[4];
+        float dist1[4];                // Polar: distances of the rows
         uint32_t f0[4];                // Observing: flat bin of the cell at theta bin 0
         float lsum[4];                 // seven sums: loglam1 + loglam2
-        Cell<NSUM> cell[4];
+        CellT cell[4];
         bool any = false;
-        auto clear = [](Cell<NSUM> &c) {
+        auto clear = [](CellT &c) {
             c.dd = c.ww = 0.0;
             if constexpr (NSUM == 7) c.x[0] = c.x[1] = c.x[2] = c.x[3] = 0.0;
             c.n = 0.0f;
@@ -220,6 +327,16 @@ __device__ __forceinline__ void tile_block(const XiKernelArgs &a, size_t part_ro
             if constexpr (NSUM == 7) lsum[r] = l1 + l2;
             cell[r].off8 = kReject;
             cell[r].edge = 0.0f;
+            if constexpr (POLAR) {
+                // r >= r_par, up to rounding: past the window none is in range
+                dist1[r] = d1;
+                const bool live = !a.window || (double)fabsf(d1 - d2) < a.win_half;
+                cell[r].edges = 0u;
+                cell[r].thr = live ? -1.0f : __builtin_inff();
+                cell[r].km = __builtin_inff();
+                any |= live;
+                continue;
+            }
             const double x0 = (double)(COORD == TOS_OBSERVING ? fabsf(l1 - l2) : fabsf(d1 - d2));
             const uint32_t i0 = axis_checked((x0 - ge.min[0]) * ge.inv[0], ge.n[0]);
             // dead cells: outside axis 0, or (Cartesian, with a regular z bin)
@@ -231,30 +348,30 @@ __device__ __forceinline__ void tile_block(const XiKernelArgs &a, size_t part_ro
             any |= live;
             if constexpr (COORD == TOS_OBSERVING) {
                 f0[r] = iz + i0 * ge.rowlen;
-            } else {
+            } else if constexpr (COORD == TOS_CARTESIAN) {
                 base[r] = pair_base(d1, d2);
                 inv_dd[r] = pair_inv(d1, d2, t.eps);
             }
         }
         if (!__any(any)) continue;
         if (lane == 0) __hip_atomic_fetch_add(&ctl.visits, visits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-        float next = -1.0f;            // Cartesian: smallest thr of the lane's cells
+        float next = -1.0f;            // Cartesian, Polar: K of the first edge of the lane's cells
         bool fresh = true;             // Observing: theta, the running sums' theta bin, is not set
         uint32_t theta = 0;
 
-        auto empty = [&](Cell<NSUM> &c, uint32_t n) {
+        auto empty = [&](CellT &c, uint32_t n) {
             neval += n;
             clear(c);
         };
-        auto add = [&](const Cell<NSUM> &c, uint32_t n, float ls) {
+        auto add = [&](const CellT &c, uint32_t n, float ls) {
             H.add8n(c.off8, n, c.dd, c.ww);
             // every pair of a cell has the same mean wavelength
             if constexpr (NSUM == 7)
                 H.add8n_more(c.off8, c.x[0], c.x[1], c.x[2], c.x[3], (double)n * (0.5 * (double)ls));
         };
-        auto flush = [&](Cell<NSUM> &c, float ls) {
+        auto flush = [&](CellT &c, float ls) {
             const uint32_t n = (uint32_t)c.n;
-            if (n > 0u && c.off8 < a.band_len8) add(c, n, ls);
+            if (n > 0u && c.off8 < a.band_len8 && c.in_axis(ge)) add(c, n, ls);
             empty(c, n);
         };
         // K reaches the threshold of some cell of the wavefront: cells that
@@ -265,13 +382,33 @@ __device__ __forceinline__ void tile_block(const XiKernelArgs &a, size_t part_ro
             const uint32_t kb_safe = kb > t.ulps ? kb - t.ulps : 0u;
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                Cell<NSUM> &c = cell[r];
+                CellT &c = cell[r];
                 // as unsigned bits a negative thr is above every K
-                if (c.thr <= K && __float_as_uint(c.thr) <= kb_safe) {
+                if (c.at() <= K && __float_as_uint(c.at()) <= kb_safe) {
                     const uint32_t n = (uint32_t)c.n;
                     // (a band of a larger grid holds a part of the slots)
-                    if (FIXED || c.off8 < a.band_len8) add(c, n, lsum[r]);
+                    if ((FIXED || c.off8 < a.band_len8) && c.in_axis(ge)) add(c, n, lsum[r]);
                     empty(c, n);
+                    if constexpr (POLAR) {
+                        float d1 = dist1[r];
+                        asm volatile("" : "+v"(d1));   // its terms are formed here, not kept
+                        const PolarStep p = polar_step(d1, d2, keep);
+                        if (c.thr <= c.km) {
+                            const bool out = (c.edges & 0xffffu) >= ge.n[0];
+                            c.off8 = out ? kReject : c.off8 + ge.row8;
+                            c.edges += 1u;
+                            c.thr = out ? __builtin_inff() : polar_kr(ge, p, polar_e(c.edges));
+                            c.km = out ? __builtin_inff() : c.km;
+                        } else {
+                            // bin m - 1; below bin 0 the next edge is at -1
+                            const bool out = c.edges < 0x10000u;
+                            c.off8 = out ? kReject : c.off8 - ge.nz8;
+                            c.edges -= out ? 0u : c.edges < 0x30000u ? (c.edges & 0xffff0000u) : 0x10000u;
+                            c.thr = out ? __builtin_inff() : c.thr;
+                            c.km = out ? __builtin_inff() : polar_km(ge, p, polar_m(c.edges));
+                        }
+                        continue;
+                    }
                     const bool out = c.edge >= (float)ge.n[1];
                     c.off8 = out ? kReject : c.off8 + ge.nz8;
                     c.edge += 1.0f;
@@ -280,13 +417,13 @@ __device__ __forceinline__ void tile_block(const XiKernelArgs &a, size_t part_ro
                     c.thr = out ? __builtin_inff() : edge_k(ge.min[1], ge.width1, c.edge, bs, inv_dd[r]);
                 }
             }
-            next = fminf(fminf(cell[0].thr, cell[1].thr), fminf(cell[2].thr, cell[3].thr));
+            next = fminf(fminf(cell[0].at(), cell[1].at()), fminf(cell[2].at(), cell[3].at()));
             if (__any(next <= K)) {
                 const double cs = global<double>(a.csep)[p];
                 uint32_t slow = 0;
 #pragma unroll
                 for (int r = 0; r < 4; ++r)
-                    if (cell[r].thr <= K) {
+                    if (cell[r].at() <= K) {
                         slow |= 1u << r;
                         flush(cell[r], lsum[r]);
                     }
@@ -295,6 +432,19 @@ __device__ __forceinline__ void tile_block(const XiKernelArgs &a, size_t part_ro
                 for (int r = 0; r < 4; ++r) {
                     if ((slow >> r) & 1u) {
                         const int k1 = 16 * b1 + 4 * r + g;
+                        if constexpr (POLAR) {
+                            const SlowPolar s = slow_polar(ge, a.band_lo8, step_d[k1], step_l[k1], d2, l2, cs, keep, K,
+                                                           __uint_as_float(kb_safe));
+                            nre += s.kr < 0.0f ? 1u : 0u;
+#pragma unroll
+                            for (int q = 0; q < 4; ++q) {
+                                cell[q].off8 = r == q ? s.off8 : cell[q].off8;
+                                cell[q].edges = r == q ? s.edges : cell[q].edges;
+                                cell[q].thr = r == q ? s.kr : cell[q].thr;
+                                cell[q].km = r == q ? s.km : cell[q].km;
+                            }
+                            continue;
+                        }
                         const SlowBin s = slow_cart(ge, a.band_lo8, step_d[k1], step_l[k1], d2, l2, cs, t.eps, K,
                                                     __uint_as_float(kb_safe));
                         nre += s.thr < 0.0f ? 1u : 0u;
@@ -306,7 +456,7 @@ __device__ __forceinline__ void tile_block(const XiKernelArgs &a, size_t part_ro
                         }
                     }
                 }
-                next = fminf(fminf(cell[0].thr, cell[1].thr), fminf(cell[2].thr, cell[3].thr));
+                next = fminf(fminf(cell[0].at(), cell[1].at()), fminf(cell[2].at(), cell[3].at()));
                 // nothing of this branch in flight where it joins the visits
                 __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0)
             }
@@ -441,7 +591,7 @@ __device__ __forceinline__ void tile_block(const XiKernelArgs &a, size_t part_ro
             }
             fill = rest;
             // past the last edge of every cell
-            if (COORD == TOS_CARTESIAN && !__any(next < __builtin_inff())) break;
+            if (COORD != TOS_OBSERVING && !__any(next < __builtin_inff())) break;
         }
 #pragma unroll
         for (int r = 0; r < 4; ++r) flush(cell[r], lsum[r]);
@@ -523,7 +673,11 @@ int launch_tile_pass(int coord, int nsum, const XiKernelArgs &a, int n_wg, int b
     const bool fixed = !a.banded && tile_fixed((int)a.ge.nslots);
     void (*fn)(XiKernelArgs);
     if (nsum == 7)
-        fn = coord == TOS_OBSERVING ? tile_pass_kernel<TOS_OBSERVING, 7, false> : tile_pass_kernel<TOS_CARTESIAN, 7, false>;
+        fn = coord == TOS_OBSERVING ? tile_pass_kernel<TOS_OBSERVING, 7, false>
+             : coord == TOS_POLAR   ? tile_pass_kernel<TOS_POLAR, 7, false>
+                                    : tile_pass_kernel<TOS_CARTESIAN, 7, false>;
+    else if (coord == TOS_POLAR)
+        fn = fixed ? tile_pass_kernel<TOS_POLAR, 2, true> : tile_pass_kernel<TOS_POLAR, 2, false>;
     else if (coord == TOS_OBSERVING)
         fn = fixed ? tile_pass_kernel<TOS_OBSERVING, 2, true> : tile_pass_kernel<TOS_OBSERVING, 2, false>;
     else
@@ -537,6 +691,9 @@ int launch_tile_batch(int coord, bool fixed, const XiBatchArgs &b, int n_wg, int
     if (coord == TOS_OBSERVING)
         return (int)(fixed ? launch_one(tile_batch_kernel<TOS_OBSERVING, 2, true>, b, n_wg, block, lds, st)
                            : launch_one(tile_batch_kernel<TOS_OBSERVING, 2, false>, b, n_wg, block, lds, st));
+    if (coord == TOS_POLAR)
+        return (int)(fixed ? launch_one(tile_batch_kernel<TOS_POLAR, 2, true>, b, n_wg, block, lds, st)
+                           : launch_one(tile_batch_kernel<TOS_POLAR, 2, false>, b, n_wg, block, lds, st));
     return (int)(fixed ? launch_one(tile_batch_kernel<TOS_CARTESIAN, 2, true>, b, n_wg, block, lds, st)
                        : launch_one(tile_batch_kernel<TOS_CARTESIAN, 2, false>, b, n_wg, block, lds, st));
 }
