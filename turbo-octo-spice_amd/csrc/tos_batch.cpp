@@ -149,7 +149,9 @@ void plan_tile_group(const tos_ctx *ctx, BatchGroup &G, int max_slots, const tos
                      std::vector<XiKernelArgs> &args, std::vector<XiWgTask> &tasks, std::vector<uint64_t> &task_cost,
                      std::vector<int> &job_nwg)
 {
-    G.lds = tile_lds_bytes(2, max_slots);
+    int max_edges = 0;
+    for (int j : G.jobs) max_edges = std::max(max_edges, tile_edges(jobs[j].grid));
+    G.lds = tile_lds_bytes(2, max_slots, max_edges);
     G.block = tile_block_size(2, max_slots);
     const int resident = ctx->ncu * tile_threads_per_cu(2) / G.block;
     double total = 0;
@@ -186,7 +188,7 @@ int batch_prepare(tos_ctx *ctx, int32_t n, const tos_batch_job *jobs, BatchState
         const tos_batch_job &J = jobs[j];
         const bool tile = tiles && tile_job(J.cat, J.pairs, J.grid) && J.pairs->tiles.state == 1 &&
                           tile_args(J.pairs, J.grid, args[(size_t)j]) &&
-                          (int64_t)tile_lds_bytes(2, (int)args[(size_t)j].ge.nslots) + 64 <= ctx->max_lds_block &&
+                          (int64_t)tile_lds_bytes(2, (int)args[(size_t)j].ge.nslots, kTileMaxEdges) + 64 <= ctx->max_lds_block &&
                           J.pairs->tiles.total / kTileVisits < (uint64_t)kMaxTasks;
         if (tile)
             by[VariantKey{J.grid.type, TOS_FP64, tile_fixed((int)args[(size_t)j].ge.nslots), true, true}].push_back(j);

@@ -81,17 +81,36 @@ struct GridFast {
 // common wavelength grid do.  The ladder is cut into blocks of 16 steps.
 constexpr int32_t kBlockSteps = 16;
 constexpr int32_t kMaxLadder = 2048;                         // ladder steps (blocks fit a byte)
-constexpr int32_t kMaxBatch = 16384;                         // pairs per batch (sorted in LDS)
+constexpr int32_t kMaxBatch = 16384;                         // pairs per batch
+// Pairs sorted by separation together, then cut into batches.  Measured, ms
+// per pass at 16384 (a batch alone) / 65536 / 262144 / 1048576: 37 million
+// pairs 149 / 130 / 120 / 116; 1.47 million Cartesian 7.0 / 6.3 / 5.9 / 5.8,
+// Polar 12.7 / 8.4 / 6.1 / 5.3.  A doubling is one more merge: 0.19 ms for 9.2
+// million pairs.
+constexpr int32_t kMaxGroup = 1048576;
+constexpr int32_t kSortRun = 16384;                          // of them sorted at a time (in LDS)
+
+// A block of a sightline's pixels: channel by channel, so that the lanes of a
+// quarter wavefront load one 64-byte line (step by step, 16 B each, a load of
+// 256 B made some 25 cache accesses).
+constexpr uint32_t kChannelBytes = 4 * kBlockSteps;
+constexpr uint32_t kBlockBytes = 3 * kChannelBytes;
+
+// Step at place p of a block (its own inverse): register r of lane group g of
+// a 16 x 16 matrix result holds row 4 g + r, and so step 4 r + g; lanes that
+// meet an edge together spread over the four registers less than in order
+// (149 against 158 ms for 37 million sightline pairs).
+__host__ __device__ inline int block_place(int p) { return 4 * (p & 3) + (p >> 2); }
 
 // Where a sightline sits on the ladder: its pixels' block B starts at byte
-// off + 256 B (modulo 2^32) of TileArgs::pix; it covers blocks [b0, b0 + nb).
+// off + kBlockBytes B (modulo 2^32) of TileArgs::pix; it covers blocks [b0, b0 + nb).
 struct LadderLos {
     uint32_t off;
     uint32_t b0_nb;               // b0 | nb << 8
 };
 
 struct TileArgs {
-    const float4 *pix;            // per ladder step of a sightline {w, w*delta, 1, 0}; absent pixels are 0
+    const float *pix;             // blocks of 16 w, 16 w*delta, 16 ones; absent pixels are 0
     const float *d, *l;           // [16 nblk] the ladder (padded with its last step)
     // [n_batches][2][nblk][words] 64 pairs a word: those whose first / second
     // sightline covers the block
@@ -254,7 +273,7 @@ struct LadderArgs {
     const uint16_t *step;         // [kLadderTable] ladder step of each table entry
     LadderLos *place;             // [n_los]
     uint32_t *nblk_of;            // [n_los] blocks of each sightline, then their exclusive prefix
-    float4 *out;
+    float *out;
 };
 constexpr int32_t kLadderTable = 8192;
 int launch_ladder_collect(const LadderArgs &a, void *stream);
@@ -268,8 +287,11 @@ struct TilePlanArgs {
     const LadderLos *place;
     int64_t n_rows;
     int32_t n_batches, max_batch, nblk;
+    int32_t n_groups, max_group;
+    const int32_t *group_ptr;     // [n_groups + 1] pairs sorted together, each whole batches
     const int32_t *batch_ptr;
     int32_t words;
+    uint64_t *keys, *keys2;       // [pairs] each, of groups longer than kSortRun: sorted runs
     uint32_t *cover;              // [pairs] blocks of both sightlines: bi0 | nbi << 8 | bj0 << 16 | nbj << 24
     uint64_t *masks;
     uint4 *rec;
@@ -287,7 +309,9 @@ static_assert((kTileVisits + (uint64_t)(kTileBlockMax / 64) * kMaxBatch) * 256 <
 bool tile_fixed(int nslots);           // the kernel variant with the fixed histogram layout
 int tile_threads_per_cu(int nsum);       // resident, by the vector registers
 int tile_block_size(int nsum, int nslots);
-size_t tile_lds_bytes(int nsum, int nslots);
+size_t tile_lds_bytes(int nsum, int nslots, int n_edges);
+inline int tile_edges(const tos_grid &g) { return g.type == TOS_POLAR ? g.nbins[0] + g.nbins[1] : 0; }
+constexpr int kTileMaxEdges = 512;     // 4 KiB: two workgroups of the fixed layout still share a CU's LDS
 int launch_tile_pass(int coord, int nsum, const XiKernelArgs &a, int n_wg, int block, size_t lds_bytes, void *stream);
 int launch_tile_batch(int coord, bool fixed, const XiBatchArgs &b, int n_wg, int block, size_t lds_bytes,
                       void *stream);

@@ -15,7 +15,7 @@ namespace tos {
 namespace {
 
 struct Scratch {   // released on every return
-    DevBuf b[5];
+    DevBuf b[7];
     ~Scratch()
     {
         for (DevBuf &x : b) x.release();
@@ -121,11 +121,11 @@ int ensure_ladder(tos_ctx *ctx, tos_catalog *cat)
     if (e != hipSuccess) return hip_fail(ctx, (hipError_t)e, "ladder placement");
     if ((rc = copy_back(ctx, st, state.ptr, sizeof(st), "ladder block count")) != TOS_OK) return rc;
     if (st[0] || st[2] >= (1u << 24) ||   // 32-bit byte offsets
-        L.pix.reserve((size_t)st[2] * kBlockSteps * sizeof(float4)) != TOS_OK) {
+        L.pix.reserve((size_t)st[2] * kBlockBytes) != TOS_OK) {
         L.release();
         return TOS_OK;
     }
-    a.out = (float4 *)L.pix.ptr;
+    a.out = (float *)L.pix.ptr;
     e = launch_ladder_fill(a, st[2], ctx->stream);
     if (e != hipSuccess) return hip_fail(ctx, (hipError_t)e, "ladder fill");
     if ((rc = copy_back(ctx, st, state.ptr, sizeof(st), "ladder state copy")) != TOS_OK) return rc;
@@ -137,19 +137,25 @@ int ensure_ladder(tos_ctx *ctx, tos_catalog *cat)
     return TOS_OK;
 }
 
-// Pairs per batch: a tile keeps its running sums between two edges of axis 1,
-// so longer batches add fewer times to the histogram; shorter ones make more
-// tiles for the device's 4096 resident wavefronts.  Measured, us per pass at
-// 1024 / 2048 / 4096-16384 pairs per batch: 3,450 pairs 298 / 373 / -;
-// 9,061 pairs 383 / 410 / -; 120,901 pairs 1407 / - / 1140; 1.47 million
-// pairs - / - / 7110 (11500) and 7200 (16384).
-constexpr int64_t kBatchMin = 1024;
-
+// Pairs per batch.  A group's batches split its range of separations, so a
+// short batch costs no more bin edges, only tiles: each is drawn from one
+// counter (some 10 ns a draw) and starts its cells anew.  Long ones make large
+// last tiles.  Measured, ms per pass at n / 64 pairs a batch (8192 at most) /
+// n / 128 / n / 256 / n / 512: 141,344 pairs in four bands 3.7 / 4.0 / 7.0 /
+// 13.4; 1.47 million pairs 5.3 / 5.4 / 5.2 / 5.3 (16384 a batch: 5.9); twelve
+// jobs of 2,000 to 12,000 sightlines - / 27.4 / 30.6 / 37.3; 3,450 pairs at
+// 512 / 1024 a batch 0.256 / 0.286; 37 million at 8192 / 16384 122 / 120.
 static int64_t batch_pairs(int64_t n_pairs)
 {
-    const int64_t q = std::max<int64_t>(kBatchMin, std::min<int64_t>(kMaxBatch, n_pairs / 32));
-    const int64_t nb = (n_pairs + q - 1) / q;   // equal batches
-    return (n_pairs + nb - 1) / nb;
+    const int64_t q = std::max<int64_t>(std::min<int64_t>(n_pairs / 64, 8192), n_pairs / 1024);
+    return std::max<int64_t>(512, std::min<int64_t>(kMaxBatch, q));
+}
+
+// [0, n) in the fewest equal parts of at most `most`, appended from `first`.
+static void cut_equal(std::vector<int32_t> &ptr, int64_t first, int64_t n, int64_t most)
+{
+    const int64_t parts = (n + most - 1) / most;
+    for (int64_t k = 0; k < parts; ++k) ptr.push_back((int32_t)(first + n * k / parts));
 }
 
 int ensure_tile_plan(tos_ctx *ctx, tos_pairs *p)
@@ -162,25 +168,33 @@ int ensure_tile_plan(tos_ctx *ctx, tos_pairs *p)
     if (rc != TOS_OK) return rc;
     const Ladder &L = cat->ladder;
     if (L.state != 1 || p->n_pairs == 0) return TOS_OK;
-    const int64_t q = batch_pairs(p->n_pairs);
-    std::vector<int32_t> bp;
-    for (int64_t b = 0; b < p->n_pairs; b += q) bp.push_back((int32_t)b);
+    std::vector<int32_t> gp, bp;
+    cut_equal(gp, 0, p->n_pairs, kMaxGroup);
+    gp.push_back((int32_t)p->n_pairs);
+    int32_t max_group = 0;
+    for (size_t k = 0; k + 1 < gp.size(); ++k) {
+        max_group = std::max(max_group, gp[k + 1] - gp[k]);
+        cut_equal(bp, gp[k], gp[k + 1] - gp[k], batch_pairs(p->n_pairs));
+    }
     bp.push_back((int32_t)p->n_pairs);
+    int32_t q = 0;
+    for (size_t k = 0; k + 1 < bp.size(); ++k) q = std::max(q, bp[k + 1] - bp[k]);
     T.n_batches = (int)bp.size() - 1;
     if ((int64_t)T.n_batches * L.nblk * (2 * L.nblk + 1) >= (1ll << 31)) return TOS_OK;
     Scratch sc;
-    DevBuf &rlos = sc.b[0], &rptr = sc.b[1], &state = sc.b[2], &cover = sc.b[3];
+    DevBuf &rlos = sc.b[0], &rptr = sc.b[1], &state = sc.b[2], &cover = sc.b[3], &keys = sc.b[4], &groups = sc.b[5], &keys2 = sc.b[6];
     T.words = (int)((q + 63) / 64);
     const size_t np = (size_t)p->n_pairs, rows = (size_t)T.n_batches * L.nblk;
     if (cover.reserve(np * 4) != TOS_OK || T.masks.reserve(rows * 2 * T.words * 8) != TOS_OK || T.rec.reserve(np * 16) != TOS_OK ||
         T.visits.reserve(rows * L.nblk * 4) != TOS_OK ||
-        state.reserve(16) != TOS_OK) {
+        state.reserve(16) != TOS_OK || (max_group > kSortRun && (keys.reserve(np * 8) != TOS_OK || keys2.reserve(np * 8) != TOS_OK))) {
         T.release();
         T.state = 2;
         return TOS_OK;
     }
     uint64_t st[2] = {0, 0};
     if ((rc = upload(ctx, T.batch_ptr, bp.data(), bp.size() * 4, "tile batches")) != TOS_OK ||
+        (rc = upload(ctx, groups, gp.data(), gp.size() * 4, "tile groups")) != TOS_OK ||
         (rc = upload(ctx, rlos, p->h.row_los.data(), p->h.row_los.size() * 4, "tile rows")) != TOS_OK ||
         (rc = upload(ctx, rptr, p->h.row_ptr.data(), p->h.row_ptr.size() * 8, "tile row offsets")) != TOS_OK ||
         (rc = upload(ctx, state, st, sizeof(st), "tile state")) != TOS_OK)
@@ -193,10 +207,15 @@ int ensure_tile_plan(tos_ctx *ctx, tos_pairs *p)
     a.place = (const LadderLos *)L.place.ptr;
     a.n_rows = p->n_rows;
     a.n_batches = T.n_batches;
-    a.max_batch = (int32_t)q;
+    a.max_batch = q;
+    a.n_groups = (int32_t)gp.size() - 1;
+    a.max_group = max_group;
+    a.group_ptr = (const int32_t *)groups.ptr;
     a.nblk = L.nblk;
     a.batch_ptr = (const int32_t *)T.batch_ptr.ptr;
     a.words = T.words;
+    a.keys = (uint64_t *)keys.ptr;
+    a.keys2 = (uint64_t *)keys2.ptr;
     a.cover = (uint32_t *)cover.ptr;
     a.masks = (uint64_t *)T.masks.ptr;
     a.rec = (uint4 *)T.rec.ptr;
@@ -232,9 +251,9 @@ bool tile_job(const tos_catalog *cat, const tos_pairs *p, const tos_grid &g)
     // beyond 2^31 of them
     auto wraps = [&](double top, int k) { return (top + std::fabs(g.min[k])) / g.width[k] > 1e9; };
     if (g.type == TOS_CARTESIAN) return !wraps(2.0 * cat->dmax, 1);
-    // Polar: |d1 - d2| exact, two bin numbers in one word
+    // Polar: |d1 - d2| exact, a table of the edges in LDS
     if (g.type == TOS_POLAR)
-        return cat->dmax <= 2.0 * cat->dmin && g.nbins[0] < 65000 && g.nbins[1] < 65000 && !wraps(2.0 * cat->dmax, 0) &&
+        return cat->dmax <= 2.0 * cat->dmin && tile_edges(g) <= kTileMaxEdges && !wraps(2.0 * cat->dmax, 0) &&
                !wraps(1.0, 1);
     return true;
 }
@@ -245,7 +264,7 @@ bool tile_args(const tos_pairs *p, const tos_grid &g, XiKernelArgs &a)
     const Ladder &L = cat->ladder;
     const TilePlan &T = p->tiles;
     TileArgs &t = a.tile;
-    t.pix = (const float4 *)L.pix.ptr;
+    t.pix = (const float *)L.pix.ptr;
     t.d = (const float *)L.d.ptr;
     t.l = (const float *)L.l.ptr;
     t.masks = (const uint64_t *)T.masks.ptr;

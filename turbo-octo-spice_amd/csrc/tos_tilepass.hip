@@ -4,7 +4,7 @@
 // sightline pairs of a batch that cover a tile, in ascending K = 2 (1 - c):
 // 256 pixel pairs per step, one running sum per (k1, k2) in registers.
 //   products  one v_mfma_f32_16x16x1_4b per sightline pair: its four blocks
-//             are the outer products w1 w2, (w d)1 (w d)2, 1 1 and 0 0.  With
+//             are the outer products w1 w2, (w d)1 (w d)2, 1 1 and one not used.  With
 //             C = 0 a product rounds once, to the reference's own f32
 //             product (types.h:77-87); the third block is 1 where both
 //             sightlines have the pixel.
@@ -16,26 +16,36 @@
 //             workgroup's LDS histogram.  A pair whose K is within the error
 //             bound of an edge, or whose separation is too small for the
 //             bound, is binned with the reference arithmetic (slow_bin).
-// So 64 pixel pairs cost some 11 VALU instructions (two conversions, two FP64
+// So 64 pixel pairs cost some 9 VALU instructions (two conversions, two FP64
 // additions and one count each, and a share of the scan and the edges) in
-// place of 26 and three LDS atomics (xi_pairs_kernel).  VALU issue bounds the
-// pass (busy 72 %, 46 instructions per visit of 256 pairs of steps; 0.77 of
-// these are pixel pairs, the rest covers ends of sightlines).
+// place of 26 and three LDS atomics (xi_pairs_kernel).  VALU issue and, for
+// large catalogues, L2 misses on the sightlines' blocks bound the pass: 23
+// instructions a visit of 256 pairs of steps and some 115 where an edge is
+// passed.  Sorting larger groups (kMaxGroup) makes edges rarer: 46
+// instructions a visit at 16384 pairs, 39 at 65536 (37 million pairs; Polar
+// 136 and 85).  0.77 of a visit's 256 are pixel pairs, the rest covers ends of
+// sightlines.
+//
+// Polar grids have both their axes move with K, at a K of its own for each
+// pair of steps; the edges come from a table in LDS, so one formula serves
+// both axes.  Where a tile's next pair has passed several edges of a cell the
+// cell moves up again, without the reference arithmetic.
 //
 // 16 x 16 is the matrix instruction's tile and four cells a lane: with the
-// running sums, two visits' operands and the edges it takes 127 vector
+// running sums, two visits' operands and the edges it takes 128 vector
 // registers, which keeps 16 wavefronts on a CU.  Wavefronts draw tiles from
 // one counter; ranges of tiles of equal visits cut beforehand were 20 % slower
 // (8.5 against 7.1 ms for 1.47 million sightline pairs), since the time of a
 // visit varies with the edges it meets.
 //
-// Measured, us per pass, general kernel / this one: 3,450 sightline pairs 551
-// / 273; 1.47 million (1.3e10 pixel pairs) FP64 24620 / 6990; 37 million
-// (3.3e11) 336,000 / 159,000; Observing, 1.3 million pairs 13730 / 5290.
+// Measured, us per pass, general kernel / this one: 3,450 sightline pairs 566
+// / 218; 1.47 million (1.3e10 pixel pairs) FP64 25040 / 5130, Polar 16860 /
+// 4790; 37 million (3.3e11) 335,000 / 115,400; Observing, 1.3 million pairs
+// 13930 / 3690.
 //
 // With seven sums a second instruction forms (w d)1, (w d)2, w1 and w2 as
 // products by 1, exactly; the mean wavelength is one number per cell.  141,344
-// pairs, 50 x 50 x 3 bins in four bands: 65,110 / 5,230 us (the general kernel
+// pairs, 50 x 50 x 3 bins in four bands: 64,240 / 3,390 us (the general kernel
 // makes three full passes with eight atomics per pixel pair; here a band takes
 // the tiles it has cells in).
 #include <hip/hip_runtime.h>
@@ -132,41 +142,43 @@ __device__ __forceinline__ SlowBin slow_cart(const GridExact &ge, uint32_t band_
 
 // Polar: r^2 = K d1 d2 + r_par^2 + base, where base = f32(d1^2) - d1^2 since
 // |d1 - d2| is exact (tile_job asks for dmax <= 2 dmin).  Each (k1, k2) meets
-// the edges of r upwards and those of mu = r_par / r downwards.
+// the edges of r upwards and those of mu = r_par / r downwards: at
+// r^2 = table[e], r edge e <= n0, and r^2 = r_par^2 table[n0 + 1 + j] with
+// 1 / mu^2 of mu edge j (of the bins' lower edges; bin 0 ends at t = -1,
+// where the cast truncates).
 struct PolarStep {
-    double rr, base;                   // r_par^2, base
+    double rr, rrb;                    // r_par^2, r_par^2 + base
     float rpar, inv;                   // inv = (1 - eps) / (d1 d2)
 };
 
-__device__ __forceinline__ PolarStep polar_step(float d1, float d2, float keep)
+__device__ __forceinline__ float polar_inv(float d1, float d2, float keep) { return keep * __builtin_amdgcn_rcpf(d1 * d2); }
+
+__device__ __forceinline__ PolarStep polar_step(float d1, float d2, float inv)
 {
     PolarStep p;
     const float sq = d1 * d1;
-    p.base = (double)-__builtin_fmaf(d1, d1, -sq);
     p.rpar = fabsf(d1 - d2);
     p.rr = (double)p.rpar * (double)p.rpar;
-    p.inv = keep * __builtin_amdgcn_rcpf(d1 * d2);
+    p.rrb = p.rr - (double)__builtin_fmaf(d1, d1, -sq);
+    p.inv = inv;
     return p;
 }
 
-// K of r edge e (in bins), lowered by its error bound
-__device__ __forceinline__ float polar_kr(const GridExact &ge, const PolarStep &p, float e)
+// K at r^2 = f t, lowered by its error bound
+__device__ __forceinline__ float polar_k(const PolarStep &p, double f, double t)
 {
-    const double s = __builtin_fma((double)e, ge.width0, ge.min[0]);
-    return (float)(__builtin_fma(s, s, -p.rr) - p.base) * p.inv;
+    return (float)__builtin_fma(f, t, -p.rrb) * p.inv;
 }
 
-// K of mu edge m (in bins), lowered by its error bound; none below mu = 0,
-// nor for two pixels at one distance (mu = 0)
-__device__ __forceinline__ float polar_km(const GridExact &ge, const PolarStep &p, float m)
+__device__ __forceinline__ double polar_edge(const GridExact &ge, uint32_t i)
 {
-    const double mu = __builtin_fma((double)m, ge.width1, ge.min[1]);
-    if (!(mu > 0.0) || p.rpar == 0.0f) return __builtin_inff();
-    double y = __builtin_amdgcn_rcp(mu);
-    y = __builtin_fma(__builtin_fma(-mu, y, 1.0), y, y);
-    y = __builtin_fma(__builtin_fma(-mu, y, 1.0), y, y);
-    const double r = (double)p.rpar * y;
-    return (float)(__builtin_fma(r, r, -p.rr) - p.base) * p.inv;
+    if (i <= ge.n[0]) {
+        const double r = __builtin_fma((double)i, ge.width0, ge.min[0]);
+        return r * r;
+    }
+    const uint32_t j = i - ge.n[0] - 1;
+    const double mu = __builtin_fma(j > 0 ? (double)j : -1.0, ge.width1, ge.min[1]);
+    return mu > 0.0 ? 1.0 / (mu * mu) : (double)__builtin_inff();
 }
 
 struct SlowPolar {
@@ -174,53 +186,44 @@ struct SlowPolar {
     float kr, km;
 };
 
-// The next edges of a cell: r edge e (in bins) and mu edge m >= -1.
-__device__ __forceinline__ uint32_t polar_pack(float e, float m)
-{
-    return (uint32_t)(int32_t)e | ((uint32_t)((int32_t)m + 1) << 16);
-}
-__device__ __forceinline__ float polar_e(uint32_t edges) { return (float)(edges & 0xffffu); }
-__device__ __forceinline__ float polar_m(uint32_t edges) { return (float)((int32_t)(edges >> 16) - 1); }
-
-__device__ __forceinline__ SlowPolar slow_polar(const GridExact &ge, uint32_t band_lo8, float d1, float l1, float d2,
-                                                float l2, double c, float keep, float K, float k_safe)
+__device__ __forceinline__ SlowPolar slow_polar(const GridExact &ge, const double *table, uint32_t band_lo8, float d1,
+                                                float l1, float d2, float l2, double c, float inv, float K, float k_safe)
 {
     const double d2d = (double)d2;
     const double r1_sq = (double)(d1 * d1), two = (double)(2.0f * d1) * c;
     const uint32_t slot = exact_bin_polar(ge, d1, l1, r1_sq, two, d2, l2, false, 0);
-    const PolarStep p = polar_step(d1, d2, keep);
+    const PolarStep p = polar_step(d1, d2, inv);
     const double r_sq = r1_sq + (d2d - two) * d2d;
     const double r = sqrt_no_tiny(r_sq);
     const double t0 = (r - ge.min[0]) * ge.inv[0], t1 = ((double)p.rpar / r - ge.min[1]) * ge.inv[1];
     const double n0 = (double)ge.n[0], n1 = (double)ge.n[1];
-    // the edges around t0 and t1 (the cast truncates: (-1, 1) is one bin)
-    const double lo0 = t0 >= n0 ? n0 : t0 >= 1.0 ? floor(t0) : -1.0;
-    const double up0 = floor(t0 < 0.0 ? 0.0 : t0) + 1.0;
-    const double lo1 = t1 >= n1 ? n1 : t1 >= 1.0 ? floor(t1) : -1.0;
-    const double up1 = t1 <= -1.0 ? -1.0 : floor(t1 < 0.0 ? 0.0 : t1) + 1.0;
-    const bool no_lo0 = __builtin_fma(lo0, ge.width0, ge.min[0]) <= 0.0;
-    const float k0 = no_lo0 ? -1.0f : polar_kr(ge, p, (float)lo0);
-    const float k1 = t1 >= n1 || p.rpar == 0.0f ? -1.0f : polar_km(ge, p, (float)up1);
-    const float kr = polar_kr(ge, p, (float)up0), km = polar_km(ge, p, (float)lo1);
+    // bins and edges around t0 and t1 (the cast truncates: (-1, 1) is one bin)
+    const uint32_t i0 = t0 >= n0 ? ge.n[0] : t0 >= 1.0 ? (uint32_t)(int32_t)t0 : 0u;
+    const uint32_t i1 = t1 >= n1 ? ge.n[1] : t1 >= 1.0 ? (uint32_t)(int32_t)t1 : 0u;
+    const uint32_t mu0 = ge.n[0] + 1u;
+    const double r_below = ge.min[0] - ge.width0;
+    const float k0 = i0 > 0u ? polar_k(p, 1.0, table[i0]) : r_below > 0.0 ? polar_k(p, r_below, r_below) : -1.0f;
+    const bool no_mu = p.rpar == 0.0f;   // mu = 0 at any K
+    const float k1 = t1 >= n1 || no_mu ? -1.0f : polar_k(p, p.rr, table[mu0 + (t1 <= -1.0 ? 0u : i1 + 1u)]);
+    const float kr = polar_k(p, 1.0, table[min(i0 + 1u, ge.n[0])]);
+    const float km = no_mu ? __builtin_inff() : polar_k(p, p.rr, table[mu0 + i1]);
     const bool dead = t0 >= n0 || t1 <= -1.0;
     const uint32_t iz = z_bin_exact(ge, l1, l2);
     const bool settled = r_sq - p.rr >= 4.0 && t0 > -1.0 && k0 <= k_safe && k1 <= k_safe && iz < ge.n[2] &&
                          (dead || (K < kr && K < km));
     SlowPolar s;
+    s.edges = 0u;                      // in the mu axis
     if (!settled) {
         s.off8 = slot == kReject ? kReject : (slot << 3) - band_lo8;
-        s.edges = 0u;                  // m = -1: in the mu axis
         s.kr = -1.0f;
         s.km = __builtin_inff();
     } else if (dead) {
         s.off8 = kReject;
-        s.edges = 0u;
         s.kr = s.km = __builtin_inff();
     } else {
-        // above the mu axis (lo1 = n1) the slot is that of a bin past the row
-        const uint32_t i1 = t1 >= n1 ? ge.n[1] : (uint32_t)(int32_t)t1;
-        s.off8 = (slot3(ge, (uint32_t)(int32_t)t0, i1, iz) << 3) - band_lo8;
-        s.edges = polar_pack((float)up0, (float)lo1);
+        // above the mu axis (i1 = n1) the slot is that of a bin past the row
+        s.off8 = (slot3(ge, i0, i1, iz) << 3) - band_lo8;
+        s.edges = (i0 + 1u) | (i1 << 16);
         s.kr = kr;
         s.km = km;
     }
@@ -236,11 +239,11 @@ struct Cell {                          // one (k1, k2) of a lane
     float thr;                         // K of the next edge (lower bound; Polar: of r); < 0: bin every pair exactly
     float edge;                        // that edge, in bins
     float km;                          // Polar: K of the next edge of mu
-    uint32_t edges;                    // Polar: the next edges of both axes, in bins
+    uint32_t edges;                    // Polar: the next edges e | j << 16
 
     __device__ __forceinline__ float at() const { return POLAR ? fminf(thr, km) : thr; }
     // the running sums have a slot (Polar: mu is not above its axis)
-    __device__ __forceinline__ bool in_axis(const GridExact &ge) const { return !POLAR || (edges >> 16) <= ge.n[1]; }
+    __device__ __forceinline__ bool in_axis(const GridExact &ge) const { return !POLAR || (edges >> 16) < ge.n[1]; }
 };
 
 template <int COORD, int NSUM, bool FIXED>
@@ -258,6 +261,9 @@ __device__ __forceinline__ void tile_block(const XiKernelArgs &a, size_t part_ro
     TileCtl &ctl = *reinterpret_cast<TileCtl *>(after);
     const int lane = threadIdx.x & (kWave - 1);
     uint4 *queue = reinterpret_cast<uint4 *>(after + kTileCtlBytes) + (threadIdx.x / kWave) * kQueue;
+    double *table = reinterpret_cast<double *>(after + kTileCtlBytes + (blockDim.x / kWave) * (kQueue * sizeof(uint4)));
+    if constexpr (POLAR)
+        for (uint32_t i = threadIdx.x; i < ge.n[0] + ge.n[1] + 2u; i += blockDim.x) table[i] = polar_edge(ge, i);
     {
         const int ns = (int)H.stride();
         for (int b = threadIdx.x; b < ns * NSUM; b += blockDim.x) H.hs[b] = 0.0;
@@ -274,11 +280,12 @@ __device__ __forceinline__ void tile_block(const XiKernelArgs &a, size_t part_ro
     // this lane's operand element: block (channel) g of row / column col;
     // row rho of the A operand is step 4 (rho mod 4) + rho / 4, so that
     // register r of the result holds the steps 4 r + g of its four lane groups
-    const uint32_t lane_a = 16u * (4u * (col & 3) + (col >> 2)) + 4u * g;
-    const uint32_t lane_b = 16u * col + 4u * g;
+    const uint32_t at_a = 4u * col, at_b = 4u * col;
+    // (the fourth block's result is not used)
+    const uint32_t lane_a = at_a + kChannelBytes * min(g, 2), lane_b = at_b + kChannelBytes * min(g, 2);
     // the second instruction's blocks: (w d)1 1, 1 (w d)2, w1 1, 1 w2
-    const uint32_t lane_a2 = lane_a - 4u * g + 4u * (g == 0 ? 1 : g == 2 ? 0 : 2);
-    const uint32_t lane_b2 = lane_b - 4u * g + 4u * (g == 1 ? 1 : g == 3 ? 0 : 2);
+    const uint32_t lane_a2 = at_a + kChannelBytes * (g == 0 ? 1 : g == 2 ? 0 : 2);
+    const uint32_t lane_b2 = at_b + kChannelBytes * (g == 1 ? 1 : g == 3 ? 0 : 2);
     const TOS_GLOBAL char *pixels = global<char>(t.pix);
     const TOS_GLOBAL float *step_d = global<float>(t.d), *step_l = global<float>(t.l);
     const TOS_GLOBAL uint4_v *records = global<uint4_v>(t.rec);
@@ -288,8 +295,8 @@ __device__ __forceinline__ void tile_block(const XiKernelArgs &a, size_t part_ro
 
     const uint32_t n_tiles = (uint32_t)(t.n_batches * t.nblk * wide);
     for (;;) {
-        // the launch's next tile (drawn one at a time: 25.4 ms for 6.2 million
-        // sightline pairs, and no less with draws of 16), unless the
+        // the launch's next tile (drawn one at a time: 6.2 million
+        // sightline pairs took no less with draws of 16), unless the
         // workgroup's u32 counts could overflow: kTileVisits visits of 256
         // pairs, and one tile of at most kMaxBatch visits more for each of its
         // wavefronts
@@ -307,7 +314,7 @@ __device__ __forceinline__ void tile_block(const XiKernelArgs &a, size_t part_ro
         if (visits == 0) continue;
 
         // the lane's four cells
-        const float d2 = step_d[16 * b2 + col], l2 = step_l[16 * b2 + col];
+        const float d2 = step_d[16 * b2 + block_place(col)], l2 = step_l[16 * b2 + block_place(col)];
         float inv_dd[4];               // Cartesian: (1 - eps) / (d1 d2), pair_base
         float base[4];
         float dist1[4];                // Polar: distances of the rows
@@ -322,7 +329,7 @@ __device__ __forceinline__ void tile_block(const XiKernelArgs &a, size_t part_ro
         };
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            const float d1 = step_d[16 * b1 + 4 * r + g], l1 = step_l[16 * b1 + 4 * r + g];
+            const float d1 = step_d[16 * b1 + block_place(4 * g + r)], l1 = step_l[16 * b1 + block_place(4 * g + r)];
             clear(cell[r]);
             if constexpr (NSUM == 7) lsum[r] = l1 + l2;
             cell[r].off8 = kReject;
@@ -330,6 +337,7 @@ __device__ __forceinline__ void tile_block(const XiKernelArgs &a, size_t part_ro
             if constexpr (POLAR) {
                 // r >= r_par, up to rounding: past the window none is in range
                 dist1[r] = d1;
+                inv_dd[r] = polar_inv(d1, d2, keep);
                 const bool live = !a.window || (double)fabsf(d1 - d2) < a.win_half;
                 cell[r].edges = 0u;
                 cell[r].thr = live ? -1.0f : __builtin_inff();
@@ -380,44 +388,44 @@ __device__ __forceinline__ void tile_block(const XiKernelArgs &a, size_t part_ro
         auto cross = [&](float K, uint32_t p) {
             const uint32_t kb = __float_as_uint(K);
             const uint32_t kb_safe = kb > t.ulps ? kb - t.ulps : 0u;
+            bool again;
+            do {
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                CellT &c = cell[r];
-                // as unsigned bits a negative thr is above every K
-                if (c.at() <= K && __float_as_uint(c.at()) <= kb_safe) {
-                    const uint32_t n = (uint32_t)c.n;
-                    // (a band of a larger grid holds a part of the slots)
-                    if ((FIXED || c.off8 < a.band_len8) && c.in_axis(ge)) add(c, n, lsum[r]);
-                    empty(c, n);
-                    if constexpr (POLAR) {
-                        float d1 = dist1[r];
-                        asm volatile("" : "+v"(d1));   // its terms are formed here, not kept
-                        const PolarStep p = polar_step(d1, d2, keep);
-                        if (c.thr <= c.km) {
-                            const bool out = (c.edges & 0xffffu) >= ge.n[0];
-                            c.off8 = out ? kReject : c.off8 + ge.row8;
-                            c.edges += 1u;
-                            c.thr = out ? __builtin_inff() : polar_kr(ge, p, polar_e(c.edges));
-                            c.km = out ? __builtin_inff() : c.km;
-                        } else {
-                            // bin m - 1; below bin 0 the next edge is at -1
-                            const bool out = c.edges < 0x10000u;
-                            c.off8 = out ? kReject : c.off8 - ge.nz8;
-                            c.edges -= out ? 0u : c.edges < 0x30000u ? (c.edges & 0xffff0000u) : 0x10000u;
-                            c.thr = out ? __builtin_inff() : c.thr;
-                            c.km = out ? __builtin_inff() : polar_km(ge, p, polar_m(c.edges));
+                for (int r = 0; r < 4; ++r) {
+                    CellT &c = cell[r];
+                    // as unsigned bits a negative thr is above every K
+                    if (c.at() <= K && __float_as_uint(c.at()) <= kb_safe) {
+                        const uint32_t n = (uint32_t)c.n;
+                        // (a band of a larger grid holds a part of the slots)
+                        if ((FIXED || c.off8 < a.band_len8) && c.in_axis(ge)) add(c, n, lsum[r]);
+                        empty(c, n);
+                        if constexpr (POLAR) {
+                            float d1 = dist1[r];
+                            asm volatile("" : "+v"(d1));   // its terms are formed here, not kept
+                            const PolarStep p = polar_step(d1, d2, inv_dd[r]);
+                            const bool of_r = !(c.km < c.thr);
+                            // past the last r bin, or mu below its axis: for good
+                            const bool out = of_r ? (c.edges & 0xffffu) >= ge.n[0] : c.edges < 0x10000u;
+                            c.edges += of_r ? 1u : 0xffff0000u;
+                            const uint32_t i = of_r ? c.edges & 0xffffu : ge.n[0] + 1u + (c.edges >> 16);
+                            const float k = polar_k(p, of_r ? 1.0 : p.rr, table[out ? 0u : i]);
+                            c.off8 = out ? kReject : c.off8 + (of_r ? ge.row8 : 0u - ge.nz8);
+                            c.thr = out ? __builtin_inff() : of_r ? k : c.thr;
+                            c.km = out ? __builtin_inff() : of_r ? c.km : k;
+                            continue;
                         }
-                        continue;
+                        const bool out = c.edge >= (float)ge.n[1];
+                        c.off8 = out ? kReject : c.off8 + ge.nz8;
+                        c.edge += 1.0f;
+                        float bs = base[r];
+                        asm volatile("" : "+v"(bs));   // converted here, not kept as a double
+                        c.thr = out ? __builtin_inff() : edge_k(ge.min[1], ge.width1, c.edge, bs, inv_dd[r]);
                     }
-                    const bool out = c.edge >= (float)ge.n[1];
-                    c.off8 = out ? kReject : c.off8 + ge.nz8;
-                    c.edge += 1.0f;
-                    float bs = base[r];
-                    asm volatile("" : "+v"(bs));   // converted here, not kept as a double
-                    c.thr = out ? __builtin_inff() : edge_k(ge.min[1], ge.width1, c.edge, bs, inv_dd[r]);
                 }
-            }
-            next = fminf(fminf(cell[0].at(), cell[1].at()), fminf(cell[2].at(), cell[3].at()));
+                next = fminf(fminf(cell[0].at(), cell[1].at()), fminf(cell[2].at(), cell[3].at()));
+                // several edges passed since the tile's last pair: once more
+                again = next <= K && __float_as_uint(next) <= kb_safe;
+            } while (__any(again));
             if (__any(next <= K)) {
                 const double cs = global<double>(a.csep)[p];
                 uint32_t slow = 0;
@@ -431,10 +439,11 @@ __device__ __forceinline__ void tile_block(const XiKernelArgs &a, size_t part_ro
 #pragma unroll 1
                 for (int r = 0; r < 4; ++r) {
                     if ((slow >> r) & 1u) {
-                        const int k1 = 16 * b1 + 4 * r + g;
+                        const int k1 = 16 * b1 + block_place(4 * g + r);
                         if constexpr (POLAR) {
-                            const SlowPolar s = slow_polar(ge, a.band_lo8, step_d[k1], step_l[k1], d2, l2, cs, keep, K,
-                                                           __uint_as_float(kb_safe));
+                            const float d1 = step_d[k1];
+                            const SlowPolar s = slow_polar(ge, table, a.band_lo8, d1, step_l[k1], d2, l2, cs,
+                                                           polar_inv(d1, d2, keep), K, __uint_as_float(kb_safe));
                             nre += s.kr < 0.0f ? 1u : 0u;
 #pragma unroll
                             for (int q = 0; q < 4; ++q) {
@@ -500,7 +509,7 @@ __device__ __forceinline__ void tile_block(const XiKernelArgs &a, size_t part_ro
         const int n_words = (global<int32_t>(t.batch_ptr)[batch + 1] - p0 + kWave - 1) / kWave;
         const TOS_GLOBAL uint64_t *mask1 = global<uint64_t>(t.masks) + ((size_t)(2 * batch) * t.nblk + b1) * t.words;
         const TOS_GLOBAL uint64_t *mask2 = global<uint64_t>(t.masks) + ((size_t)(2 * batch + 1) * t.nblk + b2) * t.words;
-        const uint32_t add1 = 256u * (uint32_t)b1, add2 = 256u * (uint32_t)b2;
+        const uint32_t add1 = kBlockBytes * (uint32_t)b1, add2 = kBlockBytes * (uint32_t)b2;
         int w0 = -kWave;               // first word of the lanes' words
         uint64_t word = 0, left = 0;   // the lane's word; words still to queue
         int fill = 0;                  // queued entries (wave-uniform)
@@ -658,13 +667,15 @@ int tile_threads_per_cu(int nsum) { return nsum == 7 ? 512 : 1024; }
 // wavefronts per CU either way (128 vector registers); 512 with seven sums.
 int tile_block_size(int nsum, int nslots) { return nsum == 7 || tile_fixed(nslots) ? 512 : 1024; }
 
-size_t tile_lds_bytes(int nsum, int nslots)
+// n_edges: bins of both axes of a Polar grid, 0 on the others
+size_t tile_lds_bytes(int nsum, int nslots, int n_edges)
 {
     const size_t hist = nsum == 7           ? hist_bytes<7, false>(nslots)
                         : tile_fixed(nslots) ? hist_bytes<2, true>(nslots)
                                              : hist_bytes<2, false>(nslots);
     return ((hist + 15) & ~(size_t)15) + kTileCtlBytes +
-           (size_t)(tile_block_size(nsum, nslots) / kWave) * kQueue * sizeof(uint4);
+           (size_t)(tile_block_size(nsum, nslots) / kWave) * kQueue * sizeof(uint4) +
+           (n_edges > 0 ? (size_t)(n_edges + 2) * sizeof(double) : 0);
 }
 
 int launch_tile_pass(int coord, int nsum, const XiKernelArgs &a, int n_wg, int block, size_t lds, void *stream)

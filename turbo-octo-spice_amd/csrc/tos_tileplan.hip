@@ -8,6 +8,10 @@
 // sightlines, and its axis-1 bin rises with the separation measure
 // K = 2 (1 - c) of the sightline pair; tos_tilepass.hip walks the pairs of a
 // batch in ascending K and keeps one running sum per pair of steps.
+//
+// A group of neighbouring pairs is sorted by K and cut into batches, so that
+// a batch spans a part of the K range only: its tiles meet fewer bin edges
+// than those of a batch of as many pairs cut out of the list.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -146,7 +150,7 @@ __global__ void __launch_bounds__(256) ladder_fill(LadderArgs a)
     const LosInfo li = a.los[s];
     const uint32_t b0 = a.place[s].b0_nb & 255u, nb = a.place[s].b0_nb >> 8;
     const uint32_t first = a.nblk_of[s];
-    if (lane == 0) a.place[s].off = 256u * (first - b0);
+    if (lane == 0) a.place[s].off = kBlockBytes * (first - b0);
     int prev = -1;   // wave-uniform: the last step of the pixels before
     for (int32_t p0 = 0; p0 < li.n; p0 += kWave) {
         const int32_t p = p0 + lane;
@@ -164,27 +168,53 @@ __global__ void __launch_bounds__(256) ladder_fill(LadderArgs a)
         const bool ok = !in || (st > before && at < nb * kBlockSteps && __builtin_isfinite(v.z) &&
                                 __builtin_isfinite(v.w));
         if (!ok) a.state[0] = 1;
-        if (in && ok) a.out[(size_t)first * kBlockSteps + at] = make_float4(v.z, v.w, 1.0f, 0.0f);
+        if (in && ok) {
+            constexpr uint32_t ch = kChannelBytes / 4;
+            float *o = a.out + (size_t)(first + at / kBlockSteps) * (3 * ch) + block_place(at % kBlockSteps);
+            o[0] = v.z;
+            o[ch] = v.w;
+            o[2 * ch] = 1.0f;
+        }
         prev = __shfl(st, kWave - 1);
     }
 }
 
-// One workgroup per batch: the batch's pairs sorted by K = f32(2 (1 - c))
-// (a bitonic network over {K, index} in LDS), then their records.  A
-// coincident pair's c may exceed 1 by a rounding; its K is taken as 0.
+// The record of the group's pair `key` (K bits << 32 | index in the group) at
+// its place `at` in ascending K.
+__device__ __forceinline__ void put_record(const TilePlanArgs &a, int32_t p0, int32_t at, uint64_t key, int64_t r0,
+                                           int64_t r1)
+{
+    const int32_t p = p0 + (int32_t)(uint32_t)key;
+    while (r0 < r1) {   // last row with row_ptr <= p
+        const int64_t mid = r0 + (r1 - r0 + 1) / 2;
+        if (a.row_ptr[mid] <= p) r0 = mid;
+        else r1 = mid - 1;
+    }
+    const LadderLos li = a.place[a.row_los[r0]], lj = a.place[a.other[p]];
+    a.rec[p0 + at] = make_uint4(li.off, lj.off, (uint32_t)(key >> 32), (uint32_t)p);
+    a.cover[p0 + at] = (li.b0_nb & 0xffffu) | (lj.b0_nb << 16);
+}
+
+// One workgroup per run of kSortRun pairs of a group: the run sorted by
+// K = f32(2 (1 - c)) (a bitonic network over {K, index} in LDS).  A group of
+// one run gets its records at once, the runs of a longer one go to a.keys.
+// A coincident pair's c may exceed 1 by a rounding; its K is taken as 0.
 __global__ void __launch_bounds__(1024) tile_sort(TilePlanArgs a)
 {
     extern __shared__ uint64_t key[];
-    const int32_t p0 = a.batch_ptr[blockIdx.x], n = a.batch_ptr[blockIdx.x + 1] - p0;
+    const int32_t p0 = a.group_ptr[blockIdx.x], p1 = a.group_ptr[blockIdx.x + 1];
+    const int32_t s0 = p0 + (int32_t)blockIdx.y * kSortRun;
+    if (s0 >= p1) return;
+    const int32_t n = min(p1 - s0, kSortRun);
     int32_t m = 2;
     while (m < n) m <<= 1;
     for (int32_t t = threadIdx.x; t < m; t += blockDim.x) {
         uint64_t k = kEmpty;
         if (t < n) {
-            const double kd = 2.0 * (1.0 - a.csep[p0 + t]);
+            const double kd = 2.0 * (1.0 - a.csep[s0 + t]);
             if (!(kd > -1e-9 && kd < 4.5)) a.state[0] = 1;
             const float kf = kd > 0.0 ? (float)kd : 0.0f;
-            k = ((uint64_t)__float_as_uint(kf) << 32) | (uint32_t)t;
+            k = ((uint64_t)__float_as_uint(kf) << 32) | (uint32_t)(s0 - p0 + t);
         }
         key[t] = k;
     }
@@ -202,24 +232,35 @@ __global__ void __launch_bounds__(1024) tile_sort(TilePlanArgs a)
             __syncthreads();
         }
     }
-    // rows of the batch: [lo, hi] hold its pairs
-    auto row_of = [&](int64_t p, int64_t lo, int64_t hi) {
-        while (lo < hi) {   // last row with row_ptr <= p
-            const int64_t mid = lo + (hi - lo + 1) / 2;
-            if (a.row_ptr[mid] <= p) lo = mid;
-            else hi = mid - 1;
-        }
-        return lo;
-    };
-    const int64_t r0 = row_of(p0, 0, a.n_rows - 1);
-    const int64_t r1 = row_of((int64_t)p0 + n - 1, r0, a.n_rows - 1);
+    const bool whole = p1 - p0 <= kSortRun;
     for (int32_t t = threadIdx.x; t < n; t += blockDim.x) {
-        const uint64_t k = key[t];
-        const int32_t p = p0 + (int32_t)(uint32_t)k;
-        const LadderLos li = a.place[a.row_los[row_of(p, r0, r1)]], lj = a.place[a.other[p]];
-        a.rec[p0 + t] = make_uint4(li.off, lj.off, (uint32_t)(k >> 32), (uint32_t)p);
-        a.cover[p0 + t] = (li.b0_nb & 0xffffu) | (lj.b0_nb << 16);
+        if (whole) put_record(a, p0, t, key[t], 0, a.n_rows - 1);
+        else a.keys[s0 + t] = key[t];
     }
+}
+
+// Merges neighbouring runs of `width` keys of each group, from `src` to `dst`:
+// a key's place is its index in its own run plus the number of smaller keys in
+// the other (keys differ).  The last merge, of a whole group, writes the
+// records.
+__global__ void __launch_bounds__(256) tile_merge(TilePlanArgs a, const uint64_t *src, uint64_t *dst, int32_t width)
+{
+    const int32_t p0 = a.group_ptr[blockIdx.x], n = a.group_ptr[blockIdx.x + 1] - p0;
+    const int32_t t = (int32_t)(blockIdx.y * blockDim.x + threadIdx.x);
+    if (n <= kSortRun || t >= n) return;
+    const uint64_t *keys = src + p0;
+    const uint64_t mine = keys[t];
+    const int32_t run = t / width, other = run ^ 1;
+    const int32_t first = min(n, other * width);
+    int32_t lo = first, hi = min(n, first + width);
+    while (lo < hi) {
+        const int32_t mid = lo + (hi - lo) / 2;
+        if (keys[mid] < mine) lo = mid + 1;
+        else hi = mid;
+    }
+    const int32_t at = min(run, other) * width + (t - run * width) + (lo - first);
+    if (dst) dst[p0 + at] = mine;
+    else put_record(a, p0, at, mine, 0, a.n_rows - 1);
 }
 
 // Pairs covering each tile of a batch: corner counts of the covered
@@ -304,8 +345,8 @@ int launch_ladder_fill(const LadderArgs &a, int64_t n_blocks, void *stream)
 {
     hipStream_t st = (hipStream_t)stream;
     if (a.n_los <= 0) return 0;
-    const int64_t n = n_blocks * kBlockSteps;
-    hipLaunchKernelGGL(zero_f4, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, a.out, n);
+    const int64_t n = n_blocks * (kBlockBytes / sizeof(float4));
+    hipLaunchKernelGGL(zero_f4, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, (float4 *)a.out, n);
     hipLaunchKernelGGL(ladder_fill, dim3((unsigned)((a.n_los + 3) / 4)), dim3(256), 0, st, a);
     return (int)hipGetLastError();
 }
@@ -315,14 +356,25 @@ int launch_tile_plan(const TilePlanArgs &a, void *stream)
     hipStream_t st = (hipStream_t)stream;
     if (a.n_batches <= 0) return 0;
     int32_t m = 2;
-    while (m < a.max_batch) m <<= 1;
+    while (m < a.max_group && m < kSortRun) m <<= 1;
     const size_t lds_sort = (size_t)m * 8, lds_cnt = (size_t)(a.nblk + 1) * (a.nblk + 1) * 4;
     hipError_t e = hipFuncSetAttribute((const void *)tile_sort, hipFuncAttributeMaxDynamicSharedMemorySize,
                                        (int)lds_sort);
     if (e == hipSuccess)
         e = hipFuncSetAttribute((const void *)tile_visits, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_cnt);
     if (e != hipSuccess) return (int)e;
-    hipLaunchKernelGGL(tile_sort, dim3((unsigned)a.n_batches), dim3(1024), lds_sort, st, a);
+    const unsigned ng = (unsigned)a.n_groups, runs = (unsigned)((a.max_group + kSortRun - 1) / kSortRun);
+    hipLaunchKernelGGL(tile_sort, dim3(ng, runs), dim3(1024), lds_sort, st, a);
+    const uint64_t *src = a.keys;
+    uint64_t *dst = a.keys2;
+    for (int32_t width = kSortRun; width < a.max_group; width *= 2) {
+        const bool last = 2 * width >= a.max_group;
+        hipLaunchKernelGGL(tile_merge, dim3(ng, (unsigned)((a.max_group + 255) / 256)), dim3(256), 0, st, a, src,
+                           last ? nullptr : dst, width);
+        uint64_t *const t = dst;
+        dst = const_cast<uint64_t *>(src);
+        src = t;
+    }
     hipLaunchKernelGGL(tile_masks, dim3((unsigned)a.n_batches, (unsigned)((a.words + 3) / 4)), dim3(256), 0, st, a);
     hipLaunchKernelGGL(tile_visits, dim3((unsigned)a.n_batches), dim3(256), lds_cnt, st, a);
     return (int)hipGetLastError();

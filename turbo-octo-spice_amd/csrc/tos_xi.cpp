@@ -235,7 +235,7 @@ bool plan_tiles(tos_ctx *ctx, const tos_pairs *p, int accum, const tos_grid &g, 
     const int slots = banded ? (int)(band_rows * (ge.rowlen + ge.pad)) : (int)ge.nslots;
     L.nbins = banded ? (int)(band_rows * ge.rowlen) : (int)ge.ntot;
     L.nsum = xi_nsum(accum);
-    L.lds = tile_lds_bytes(L.nsum, slots);
+    L.lds = tile_lds_bytes(L.nsum, slots, tile_edges(g));
     L.block = tile_block_size(L.nsum, slots);
     L.n_wg = tile_workgroups(p, a.tile, ctx->ncu * tile_threads_per_cu(L.nsum) / L.block, L.block);
     L.n_seg = std::min(32, L.n_wg);
@@ -249,7 +249,7 @@ uint32_t band_rows_for(const tos_ctx *ctx, int accum, const tos_grid &g, bool ti
     const uint32_t rowslots = ge.rowlen + ge.pad;
     auto fits = [&](uint32_t rows) {
         const int slots = (int)(rows * rowslots);
-        return (int64_t)(tiles ? tile_lds_bytes(xi_nsum(accum), slots) : xi_lds_bytes(accum, slots)) + 64 <= ctx->max_lds_block;
+        return (int64_t)(tiles ? tile_lds_bytes(xi_nsum(accum), slots, tile_edges(g)) : xi_lds_bytes(accum, slots)) + 64 <= ctx->max_lds_block;
     };
     if (fits(ge.n[0])) return ge.n[0];
     uint32_t lo = 0, hi = ge.n[0];   // the most rows that fit
