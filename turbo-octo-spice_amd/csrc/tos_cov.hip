@@ -47,18 +47,32 @@ __global__ void __launch_bounds__(256) cov_samples(const double *didj, const dou
     if (threadIdx.x == 0) w[k] = part[0];
 }
 
-// mean over samples per bin, in sample order; wsum[0] = W (same order)
-__global__ void __launch_bounds__(256) cov_mean(const double *x, const double *w, int64_t k_n, int32_t n, double *mu,
-                                                double *wsum)
+// mean over samples per bin; wsum[0] = W.  64 bins a workgroup; wavefront g
+// adds every kMeanWaves-th sample, the partial sums are added in order (one
+// thread a bin walking all samples took 579 us for 1900 samples of 2500 bins,
+// this 40).
+constexpr int kMeanWaves = 16;
+__global__ void __launch_bounds__(64 * kMeanWaves) cov_mean(const double *x, const double *w, int64_t k_n, int32_t n,
+                                                            double *mu, double *wsum)
 {
-    const int32_t b = blockIdx.x * blockDim.x + threadIdx.x;
-    double W = 0.0;
-    for (int64_t k = 0; k < k_n; ++k) W += w[k];
+    __shared__ double part[2][kMeanWaves][64];
+    const int lane = threadIdx.x & 63, g = threadIdx.x >> 6;
+    const int32_t b = blockIdx.x * 64 + lane;
+    double s = 0.0, W = 0.0;
+    for (int64_t k = g; k < k_n; k += kMeanWaves) {
+        W += w[k];
+        if (b < n) s += w[k] * x[k * n + b];
+    }
+    part[0][g][lane] = s;
+    part[1][g][lane] = W;
+    __syncthreads();
+    if (g > 0) return;
+    for (int q = 1; q < kMeanWaves; ++q) {
+        s += part[0][q][lane];
+        W += part[1][q][lane];
+    }
     if (b == 0) wsum[0] = W;
-    if (b >= n) return;
-    double s = 0.0;
-    for (int64_t k = 0; k < k_n; ++k) s += w[k] * x[k * n + b];
-    mu[b] = W > 0 ? s / W : 0.0;
+    if (b < n) mu[b] = W > 0 ? s / W : 0.0;
 }
 
 // operands: A_kb = w_k (x_kb - mu_b), B_kb = x_kb - mu_b (B in place of x)
@@ -75,13 +89,16 @@ __global__ void __launch_bounds__(256) cov_center(double *x, const double *w, co
 }
 
 // C = A^T B / W on the matrix cores.  Block (bx, by): C rows [32 bx, +32),
-// columns [32 by, +32); wavefront q owns the 16x16 quadrant (q / 2, q % 2).
+// columns [32 by, +32), for by >= bx only: C is symmetric, and the other half
+// is written as its mirror image (half the products of the full square, which
+// took 1003 us for 1900 samples of 2500 bins, this 643); wavefront q owns the 16x16 quadrant (q / 2, q % 2).
 // v_mfma_f64_16x16x4f64: lane l supplies A[k + l/16][i0 + l%16] and
 // B[k + l/16][j0 + l%16]; it holds D[l/16 + 4 r][l%16], r = 0..3 (lane
 // layout checked on the device: tests/test_gpu_covariance.py).
 __global__ void __launch_bounds__(256) cov_gemm(const double *A, const double *B, const double *wsum, int64_t k_n,
                                                 int32_t n, double *C)
 {
+    if (blockIdx.y < blockIdx.x) return;
     const int lane = threadIdx.x & 63;
     const int q = threadIdx.x >> 6;
     const int32_t i0 = blockIdx.x * 32 + 16 * (q >> 1);
@@ -114,7 +131,11 @@ __global__ void __launch_bounds__(256) cov_gemm(const double *A, const double *B
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
         const int32_t oi = i0 + kk + 4 * r;
-        if (oi < n && jok) C[(int64_t)oi * n + cj] = acc[r] * inv;
+        if (oi < n && jok) {
+            const double v = acc[r] * inv;
+            C[(int64_t)oi * n + cj] = v;
+            if (blockIdx.y > blockIdx.x) C[(int64_t)cj * n + oi] = v;
+        }
     }
 }
 
@@ -126,7 +147,7 @@ int launch_covariance(const double *didj, const double *wgt, int64_t k_n, int32_
     hipStream_t st = (hipStream_t)stream;
     if (k_n <= 0 || n <= 0) return 0;
     hipLaunchKernelGGL(cov_samples, dim3((unsigned)k_n), dim3(256), 0, st, didj, wgt, k_n, n, x, w);
-    hipLaunchKernelGGL(cov_mean, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, x, w, k_n, n, mu, wsum);
+    hipLaunchKernelGGL(cov_mean, dim3((unsigned)((n + 63) / 64)), dim3(64 * kMeanWaves), 0, st, x, w, k_n, n, mu, wsum);
     const int64_t tot = k_n * n;
     hipLaunchKernelGGL(cov_center, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, st, x, w, mu, k_n, n, a);
     const unsigned tiles = (unsigned)((n + 31) / 32);
