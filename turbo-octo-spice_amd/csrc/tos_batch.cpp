@@ -80,7 +80,7 @@ static void release_state(BatchState *&b)
 {
     if (!b) return;
     b->drop_graph();
-    for (DevBuf *d : {&b->args, &b->tasks, &b->red, &b->parts_cnt, &b->parts_sum, &b->res}) d->release();
+    for (DevBuf *d : {&b->args, &b->tile_args, &b->tasks, &b->red, &b->parts_cnt, &b->parts_sum, &b->res}) d->release();
     if (b->host_res) (void)hipHostFree(b->host_res);
     if (b->ev0) (void)hipEventDestroy(b->ev0);
     if (b->ev1) (void)hipEventDestroy(b->ev1);
@@ -146,8 +146,8 @@ void add_buffer_key(std::vector<uint64_t> &k, int32_t n, const tos_batch_job *jo
 constexpr int kTileRounds = 4;
 
 void plan_tile_group(const tos_ctx *ctx, BatchGroup &G, int max_slots, const tos_batch_job *jobs,
-                     std::vector<XiKernelArgs> &args, std::vector<XiWgTask> &tasks, std::vector<uint64_t> &task_cost,
-                     std::vector<int> &job_nwg)
+                     const std::vector<TileArgs> &targs, std::vector<XiWgTask> &tasks,
+                     std::vector<uint64_t> &task_cost, std::vector<int> &job_nwg)
 {
     int max_edges = 0;
     for (int j : G.jobs) max_edges = std::max(max_edges, tile_edges(jobs[j].grid));
@@ -163,7 +163,7 @@ void plan_tile_group(const tos_ctx *ctx, BatchGroup &G, int max_slots, const tos
     for (int j : order) {
         const double share = total > 0 ? (double)jobs[j].pairs->tiles.total / total : 0.0;
         const int want = std::min(resident, std::max(1, (int)std::ceil(kTileRounds * resident * share)));
-        const int nwg = tile_workgroups(jobs[j].pairs, args[(size_t)j].tile, want, G.block);
+        const int nwg = tile_workgroups(jobs[j].pairs, targs[(size_t)j], want, G.block);
         job_nwg[(size_t)j] = nwg;
         for (int w = 0; w < nwg; ++w) tasks.push_back(XiWgTask{j, 0, 0, w});
     }
@@ -180,6 +180,7 @@ int batch_prepare(tos_ctx *ctx, int32_t n, const tos_batch_job *jobs, BatchState
     std::map<VariantKey, std::vector<int>> by;
     B.nbins.assign((size_t)n, 0);
     std::vector<XiKernelArgs> args((size_t)n);
+    std::vector<TileArgs> targs((size_t)n);
     for (int32_t j = 0; j < n; ++j) {
         fill_args(jobs[j].cat, jobs[j].pairs, jobs[j].grid, true, args[(size_t)j]);
         bool fixed, simple;
@@ -187,7 +188,7 @@ int batch_prepare(tos_ctx *ctx, int32_t n, const tos_batch_job *jobs, BatchState
         // jobs of the tile path: the precision and `simple` make no difference
         const tos_batch_job &J = jobs[j];
         const bool tile = tiles && tile_job(J.cat, J.pairs, J.grid) && J.pairs->tiles.state == 1 &&
-                          tile_args(J.pairs, J.grid, args[(size_t)j]) &&
+                          tile_args(J.pairs, J.grid, targs[(size_t)j]) &&
                           (int64_t)tile_lds_bytes(2, (int)args[(size_t)j].ge.nslots, kTileMaxEdges) + 64 <= ctx->max_lds_block &&
                           J.pairs->tiles.total / kTileVisits < (uint64_t)kMaxTasks;
         if (tile)
@@ -220,7 +221,7 @@ int batch_prepare(tos_ctx *ctx, int32_t n, const tos_batch_job *jobs, BatchState
             max_slots = std::max(max_slots, (int)ge.nslots);
         }
         if (G.key.tile) {
-            plan_tile_group(ctx, G, max_slots, jobs, args, tasks, task_cost, job_nwg);
+            plan_tile_group(ctx, G, max_slots, jobs, targs, tasks, task_cost, job_nwg);
             B.groups.push_back(G);
             continue;
         }
@@ -336,14 +337,17 @@ int batch_prepare(tos_ctx *ctx, int32_t n, const tos_batch_job *jobs, BatchState
         a.part_cnt = (uint32_t *)B.parts_cnt.ptr + co;
         a.part_sum = (double *)B.parts_sum.ptr + so;
         a.n_recheck = (unsigned long long *)(res + 2 * j);
-        a.tile.next = (uint32_t *)(res + 2 * n + j);
+        targs[(size_t)j].next = (uint32_t *)(res + 2 * n + j);
         red[(size_t)j].part_cnt = a.part_cnt;
         red[(size_t)j].part_sum = a.part_sum;
         red[(size_t)j].out_cnt = res + B.out_off[(size_t)j];
         red[(size_t)j].out_sum = (double *)(res + B.out_off[(size_t)j] + B.nbins[(size_t)j]);
     }
+    std::vector<TileKernelArgs> tile;   // every job's, if any takes the tile path
+    if (std::any_of(B.groups.begin(), B.groups.end(), [](const BatchGroup &G) { return G.key.tile; }))
+        for (int32_t j = 0; j < n; ++j) tile.push_back(TileKernelArgs{args[(size_t)j], targs[(size_t)j]});
     for (const BatchGroup &G : B.groups) {
-        const int e = G.key.tile ? launch_tile_batch(G.key.coord, G.key.fixed, XiBatchArgs{}, 0, G.block, G.lds,
+        const int e = G.key.tile ? launch_tile_batch(G.key.coord, G.key.fixed, TileBatchArgs{}, 0, G.block, G.lds,
                                                      ctx->stream)
                                  : launch_xi_batch(G.key.coord, G.key.prec, G.key.fixed, G.key.simple, XiBatchArgs{},
                                                    0, G.block, G.lds, ctx->stream);
@@ -353,7 +357,9 @@ int batch_prepare(tos_ctx *ctx, int32_t n, const tos_batch_job *jobs, BatchState
     if ((rc = upload(ctx, B.args, args.data(), args.size() * sizeof(XiKernelArgs), "batch job table")) != TOS_OK ||
         (rc = upload(ctx, B.tasks, tasks.data(), tasks.size() * sizeof(XiWgTask), "batch workgroup tasks")) !=
             TOS_OK ||
-        (rc = upload(ctx, B.red, red.data(), red.size() * sizeof(XiReduceJob), "batch reduction table")) != TOS_OK)
+        (rc = upload(ctx, B.red, red.data(), red.size() * sizeof(XiReduceJob), "batch reduction table")) != TOS_OK ||
+        (rc = upload(ctx, B.tile_args, tile.data(), tile.size() * sizeof(TileKernelArgs), "batch tile table")) !=
+            TOS_OK)
         return rc;
     hipError_t e = hipStreamSynchronize(ctx->stream);
     if (e != hipSuccess) return hip_fail(ctx, e, "tos_batch_run upload");
@@ -372,7 +378,8 @@ int batch_enqueue(tos_ctx *ctx, BatchState &B, int32_t n, hipStream_t stream)
         XiBatchArgs ba;
         ba.jobs = (const XiKernelArgs *)B.args.ptr;
         ba.wg = (const XiWgTask *)B.tasks.ptr + G.task_begin;
-        e = G.key.tile ? launch_tile_batch(G.key.coord, G.key.fixed, ba, G.n_wg, G.block, G.lds, stream)
+        const TileBatchArgs ta{(const TileKernelArgs *)B.tile_args.ptr, ba.wg};
+        e = G.key.tile ? launch_tile_batch(G.key.coord, G.key.fixed, ta, G.n_wg, G.block, G.lds, stream)
                        : launch_xi_batch(G.key.coord, G.key.prec, G.key.fixed, G.key.simple, ba, G.n_wg, G.block,
                                          G.lds, stream);
         if (e != hipSuccess) return hip_fail(ctx, (hipError_t)e, "batched pair kernel launch");

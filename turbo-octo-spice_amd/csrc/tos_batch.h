@@ -44,7 +44,7 @@ struct BatchState {
     std::vector<size_t> out_off;       // per job, in uint64 words of `res`
     size_t res_words = 0;
     int64_t max_fields = 0;
-    DevBuf args, tasks, red, parts_cnt, parts_sum, res;
+    DevBuf args, tile_args, tasks, red, parts_cnt, parts_sum, res;
     void *host_res = nullptr;          // pinned copy of `res`
     size_t host_res_bytes = 0;
     hipGraph_t graph = nullptr;

@@ -172,7 +172,7 @@ int plan_launch(tos_ctx *ctx, const tos_xi_opts *opts, int prec, int accum, cons
 uint32_t band_rows_for(const tos_ctx *ctx, int accum, const tos_grid &g, bool tiles = false);
 // The tile path's launch: LDS, partial rows and workgroups (false: more
 // partial rows than allowed).
-bool plan_tiles(tos_ctx *ctx, const tos_pairs *p, int accum, const tos_grid &g, XiKernelArgs &a, XiLaunch &L,
+bool plan_tiles(tos_ctx *ctx, const tos_pairs *p, int accum, const tos_grid &g, const TileArgs &t, XiLaunch &L,
                 uint32_t band_rows);
 // The tile path (tos_tile.cpp): whether a job may take it, its plan
 // (tiles.state 1 when built; 2: the general path), its kernel arguments
@@ -180,7 +180,7 @@ bool plan_tiles(tos_ctx *ctx, const tos_pairs *p, int accum, const tos_grid &g, 
 bool tile_job(const tos_catalog *cat, const tos_pairs *p, const tos_grid &g);
 int ensure_ladder(tos_ctx *ctx, tos_catalog *cat);
 int ensure_tile_plan(tos_ctx *ctx, tos_pairs *p);
-bool tile_args(const tos_pairs *p, const tos_grid &g, XiKernelArgs &a);
+bool tile_args(const tos_pairs *p, const tos_grid &g, TileArgs &t);
 // Workgroups of a tile pass that should have `want` of them.
 int tile_workgroups(const tos_pairs *p, const TileArgs &a, int want, int block);
 // Resolves this device's static scratch array of tos_xi_run_noalloc

@@ -436,8 +436,6 @@ void grid_exact_consts(const tos_grid &g, GridExact &ge)
     ge.nslots = (uint32_t)g.nbins[0] * (ge.rowlen + ge.pad);
     ge.row8 = 8u * (ge.rowlen + ge.pad);
     ge.nz8 = 8u * ge.n[2];
-    ge.width0 = g.width[0];
-    ge.width1 = g.width[1];
 }
 
 static bool is_pow2(double x)

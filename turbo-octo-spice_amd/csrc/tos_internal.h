@@ -56,7 +56,6 @@ struct GridExact {
     uint32_t nslots;      // n0 * (rowlen + pad)
     uint32_t row8;        // 8 (rowlen + pad): byte stride of an axis-0 row of FP64 sums
     uint32_t nz8;         // 8 n2
-    double width0, width1;   // bin widths of axes 0 and 1
 };
 
 // Constants of the FP32 fast path with its guard band.  The kernel forms
@@ -128,6 +127,7 @@ struct TileArgs {
     // `ulps` float steps below a pair's value is certainly below it
     uint32_t ulps;
     double eps;
+    double width0, width1;        // bin widths of axes 0 and 1
 };
 
 struct XiKernelArgs {
@@ -168,7 +168,15 @@ struct XiKernelArgs {
     uint32_t band_len8;
     int32_t band_bin0;
     int32_t banded;
-    TileArgs tile;                // tile path only
+};
+
+// Arguments of the tile path's kernels.  The plan's stay out of XiKernelArgs:
+// with them in it (384 bytes) the general kernels got other code around their
+// argument loads and more spilled scalar registers.
+static_assert(sizeof(XiKernelArgs) == 272, "the general kernels' code depends on the size of their arguments");
+struct TileKernelArgs {
+    XiKernelArgs xi;
+    TileArgs tile;
 };
 
 // One workgroup's task in a batched launch: items [begin, end) of job
@@ -185,6 +193,12 @@ struct XiWgTask {
 // launch uses the same kernel variant (coordinates, precision, layout).
 struct XiBatchArgs {
     const XiKernelArgs *jobs;
+    const XiWgTask *wg;
+};
+
+// The same of the tile path.
+struct TileBatchArgs {
+    const TileKernelArgs *jobs;
     const XiWgTask *wg;
 };
 
@@ -312,8 +326,9 @@ int tile_block_size(int nsum, int nslots);
 size_t tile_lds_bytes(int nsum, int nslots, int n_edges);
 inline int tile_edges(const tos_grid &g) { return g.type == TOS_POLAR ? g.nbins[0] + g.nbins[1] : 0; }
 constexpr int kTileMaxEdges = 512;     // 4 KiB: two workgroups of the fixed layout still share a CU's LDS
-int launch_tile_pass(int coord, int nsum, const XiKernelArgs &a, int n_wg, int block, size_t lds_bytes, void *stream);
-int launch_tile_batch(int coord, bool fixed, const XiBatchArgs &b, int n_wg, int block, size_t lds_bytes,
+int launch_tile_pass(int coord, int nsum, const TileKernelArgs &a, int n_wg, int block, size_t lds_bytes,
+                     void *stream);
+int launch_tile_batch(int coord, bool fixed, const TileBatchArgs &b, int n_wg, int block, size_t lds_bytes,
                       void *stream);
 
 // Zero n 64-bit words with a kernel (safe inside a captured graph).

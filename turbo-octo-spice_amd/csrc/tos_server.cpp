@@ -755,7 +755,7 @@ extern "C" int tos_server_stop(tos_server *S)
     for (Slot &sl : S->slots) {
         (void)hipStreamSynchronize(sl.stream);
         sl.B.drop_graph();
-        for (DevBuf *d : {&sl.B.args, &sl.B.tasks, &sl.B.red, &sl.B.parts_cnt, &sl.B.parts_sum, &sl.B.res})
+        for (DevBuf *d : {&sl.B.args, &sl.B.tile_args, &sl.B.tasks, &sl.B.red, &sl.B.parts_cnt, &sl.B.parts_sum, &sl.B.res})
             d->release();
         if (sl.B.host_res) (void)hipHostFree(sl.B.host_res);
         (void)hipStreamDestroy(sl.stream);

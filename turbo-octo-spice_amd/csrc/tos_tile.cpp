@@ -258,12 +258,12 @@ bool tile_job(const tos_catalog *cat, const tos_pairs *p, const tos_grid &g)
     return true;
 }
 
-bool tile_args(const tos_pairs *p, const tos_grid &g, XiKernelArgs &a)
+bool tile_args(const tos_pairs *p, const tos_grid &g, TileArgs &t)
 {
     const tos_catalog *cat = p->cat;
     const Ladder &L = cat->ladder;
     const TilePlan &T = p->tiles;
-    TileArgs &t = a.tile;
+    t = TileArgs{};
     t.pix = (const float *)L.pix.ptr;
     t.d = (const float *)L.d.ptr;
     t.l = (const float *)L.l.ptr;
@@ -274,6 +274,8 @@ bool tile_args(const tos_pairs *p, const tos_grid &g, XiKernelArgs &a)
     t.visits = (const uint32_t *)T.visits.ptr;
     t.nblk = L.nblk;
     t.n_batches = T.n_batches;
+    t.width0 = g.width[0];
+    t.width1 = g.width[1];
     // tiles whose steps all differ by less than the axis-0 window
     const std::vector<float> &key = g.type == TOS_OBSERVING ? L.h_l : L.h_d;
     const double X = grid_window_half(g, cat->dmax, g.type == TOS_OBSERVING ? cat->lmax_abs : cat->dmax);

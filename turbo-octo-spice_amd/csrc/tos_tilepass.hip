@@ -114,7 +114,7 @@ struct SlowBin {
 // The reference's bin of one pixel pair, and the K up to which it holds for
 // its pair of steps (thr < 0: this pair only).  Out of line: it runs for a
 // tile's first pair and for the rare pairs next to an edge.
-__device__ __forceinline__ SlowBin slow_cart(const GridExact &ge, uint32_t band_lo8, float d1, float l1, float d2,
+__device__ __forceinline__ SlowBin slow_cart(const GridExact &ge, double width1, uint32_t band_lo8, float d1, float l1, float d2,
                                              float l2, double c, double eps, float K, float k_safe)
 {
     const double d2d = (double)d2;
@@ -129,9 +129,9 @@ __device__ __forceinline__ SlowBin slow_cart(const GridExact &ge, uint32_t band_
     // the edges around t (the cast truncates: (-1, 1) is one bin)
     const double lo = t >= n1 ? n1 : t >= 1.0 ? floor(t) : -1.0;
     const double up = t <= -1.0 ? -1.0 : floor(t < 0.0 ? 0.0 : t) + 1.0;
-    const float k_up = edge_k(ge.min[1], ge.width1, (float)up, base, inv);
-    const bool no_lo = t <= -1.0 || __builtin_fma(lo, ge.width1, ge.min[1]) <= 0.0;
-    const float k_lo = no_lo ? -1.0f : edge_k(ge.min[1], ge.width1, (float)lo, base, inv);
+    const float k_up = edge_k(ge.min[1], width1, (float)up, base, inv);
+    const bool no_lo = t <= -1.0 || __builtin_fma(lo, width1, ge.min[1]) <= 0.0;
+    const float k_lo = no_lo ? -1.0f : edge_k(ge.min[1], width1, (float)lo, base, inv);
     const bool settled = rp2 >= 4.0 && k_lo <= k_safe && (t >= n1 || K < k_up) && z_bin_exact(ge, l1, l2) < ge.n[2];
     SlowBin s;
     s.off8 = slot == kReject ? kReject : (slot << 3) - band_lo8;
@@ -170,14 +170,14 @@ __device__ __forceinline__ float polar_k(const PolarStep &p, double f, double t)
     return (float)__builtin_fma(f, t, -p.rrb) * p.inv;
 }
 
-__device__ __forceinline__ double polar_edge(const GridExact &ge, uint32_t i)
+__device__ __forceinline__ double polar_edge(const GridExact &ge, const TileArgs &w, uint32_t i)
 {
     if (i <= ge.n[0]) {
-        const double r = __builtin_fma((double)i, ge.width0, ge.min[0]);
+        const double r = __builtin_fma((double)i, w.width0, ge.min[0]);
         return r * r;
     }
     const uint32_t j = i - ge.n[0] - 1;
-    const double mu = __builtin_fma(j > 0 ? (double)j : -1.0, ge.width1, ge.min[1]);
+    const double mu = __builtin_fma(j > 0 ? (double)j : -1.0, w.width1, ge.min[1]);
     return mu > 0.0 ? 1.0 / (mu * mu) : (double)__builtin_inff();
 }
 
@@ -186,8 +186,8 @@ struct SlowPolar {
     float kr, km;
 };
 
-__device__ __forceinline__ SlowPolar slow_polar(const GridExact &ge, const double *table, uint32_t band_lo8, float d1,
-                                                float l1, float d2, float l2, double c, float inv, float K, float k_safe)
+__device__ __forceinline__ SlowPolar slow_polar(const GridExact &ge, double width0, const double *table, uint32_t band_lo8,
+                                                float d1, float l1, float d2, float l2, double c, float inv, float K, float k_safe)
 {
     const double d2d = (double)d2;
     const double r1_sq = (double)(d1 * d1), two = (double)(2.0f * d1) * c;
@@ -201,7 +201,7 @@ __device__ __forceinline__ SlowPolar slow_polar(const GridExact &ge, const doubl
     const uint32_t i0 = t0 >= n0 ? ge.n[0] : t0 >= 1.0 ? (uint32_t)(int32_t)t0 : 0u;
     const uint32_t i1 = t1 >= n1 ? ge.n[1] : t1 >= 1.0 ? (uint32_t)(int32_t)t1 : 0u;
     const uint32_t mu0 = ge.n[0] + 1u;
-    const double r_below = ge.min[0] - ge.width0;
+    const double r_below = ge.min[0] - width0;
     const float k0 = i0 > 0u ? polar_k(p, 1.0, table[i0]) : r_below > 0.0 ? polar_k(p, r_below, r_below) : -1.0f;
     const bool no_mu = p.rpar == 0.0f;   // mu = 0 at any K
     const float k1 = t1 >= n1 || no_mu ? -1.0f : polar_k(p, p.rr, table[mu0 + (t1 <= -1.0 ? 0u : i1 + 1u)]);
@@ -247,12 +247,11 @@ struct Cell {                          // one (k1, k2) of a lane
 };
 
 template <int COORD, int NSUM, bool FIXED>
-__device__ __forceinline__ void tile_block(const XiKernelArgs &a, size_t part_row)
+__device__ __forceinline__ void tile_block(const XiKernelArgs &a, const TileArgs &t, size_t part_row)
 {
     constexpr bool POLAR = COORD == TOS_POLAR;
     using CellT = Cell<NSUM, POLAR>;
     const GridExact &ge = a.ge;
-    const TileArgs &t = a.tile;
     const float keep = (float)(1.0 - t.eps);
     extern __shared__ double lds_tile[];
     const uint32_t nslots = FIXED ? ge.nslots : a.band_len8 / 8u;
@@ -263,7 +262,7 @@ __device__ __forceinline__ void tile_block(const XiKernelArgs &a, size_t part_ro
     uint4 *queue = reinterpret_cast<uint4 *>(after + kTileCtlBytes) + (threadIdx.x / kWave) * kQueue;
     double *table = reinterpret_cast<double *>(after + kTileCtlBytes + (blockDim.x / kWave) * (kQueue * sizeof(uint4)));
     if constexpr (POLAR)
-        for (uint32_t i = threadIdx.x; i < ge.n[0] + ge.n[1] + 2u; i += blockDim.x) table[i] = polar_edge(ge, i);
+        for (uint32_t i = threadIdx.x; i < ge.n[0] + ge.n[1] + 2u; i += blockDim.x) table[i] = polar_edge(ge, t, i);
     {
         const int ns = (int)H.stride();
         for (int b = threadIdx.x; b < ns * NSUM; b += blockDim.x) H.hs[b] = 0.0;
@@ -419,7 +418,7 @@ __device__ __forceinline__ void tile_block(const XiKernelArgs &a, size_t part_ro
                         c.edge += 1.0f;
                         float bs = base[r];
                         asm volatile("" : "+v"(bs));   // converted here, not kept as a double
-                        c.thr = out ? __builtin_inff() : edge_k(ge.min[1], ge.width1, c.edge, bs, inv_dd[r]);
+                        c.thr = out ? __builtin_inff() : edge_k(ge.min[1], t.width1, c.edge, bs, inv_dd[r]);
                     }
                 }
                 next = fminf(fminf(cell[0].at(), cell[1].at()), fminf(cell[2].at(), cell[3].at()));
@@ -442,7 +441,7 @@ __device__ __forceinline__ void tile_block(const XiKernelArgs &a, size_t part_ro
                         const int k1 = 16 * b1 + block_place(4 * g + r);
                         if constexpr (POLAR) {
                             const float d1 = step_d[k1];
-                            const SlowPolar s = slow_polar(ge, table, a.band_lo8, d1, step_l[k1], d2, l2, cs,
+                            const SlowPolar s = slow_polar(ge, t.width0, table, a.band_lo8, d1, step_l[k1], d2, l2, cs,
                                                            polar_inv(d1, d2, keep), K, __uint_as_float(kb_safe));
                             nre += s.kr < 0.0f ? 1u : 0u;
 #pragma unroll
@@ -454,7 +453,7 @@ __device__ __forceinline__ void tile_block(const XiKernelArgs &a, size_t part_ro
                             }
                             continue;
                         }
-                        const SlowBin s = slow_cart(ge, a.band_lo8, step_d[k1], step_l[k1], d2, l2, cs, t.eps, K,
+                        const SlowBin s = slow_cart(ge, t.width1, a.band_lo8, step_d[k1], step_l[k1], d2, l2, cs, t.eps, K,
                                                     __uint_as_float(kb_safe));
                         nre += s.thr < 0.0f ? 1u : 0u;
 #pragma unroll
@@ -630,21 +629,21 @@ __device__ __forceinline__ void tile_block(const XiKernelArgs &a, size_t part_ro
 // room for one workgroup of eight wavefronts on a CU.
 template <int COORD, int NSUM, bool FIXED>
 __global__ void __launch_bounds__(NSUM == 7 ? 512 : kTileBlockMax)
-__attribute__((amdgpu_waves_per_eu(NSUM == 7 ? 2 : 4, NSUM == 7 ? 2 : 4))) tile_pass_kernel(XiKernelArgs a)
+__attribute__((amdgpu_waves_per_eu(NSUM == 7 ? 2 : 4, NSUM == 7 ? 2 : 4))) tile_pass_kernel(TileKernelArgs a)
 {
-    tile_block<COORD, NSUM, FIXED>(a, blockIdx.x);
+    tile_block<COORD, NSUM, FIXED>(a.xi, a.tile, blockIdx.x);
 }
 
 // Many jobs in one launch: workgroup w serves job b.wg[w].job and writes its
 // partial row b.wg[w].row.
 template <int COORD, int NSUM, bool FIXED>
 __global__ void __launch_bounds__(kTileBlockMax) __attribute__((amdgpu_waves_per_eu(4, 4)))
-tile_batch_kernel(XiBatchArgs b)
+tile_batch_kernel(TileBatchArgs b)
 {
     const XiWgTask w = b.wg[blockIdx.x];
     // a copy taken before the kernel writes anything: scalar loads
-    const XiKernelArgs a = b.jobs[w.job];
-    tile_block<COORD, NSUM, FIXED>(a, (size_t)w.row);
+    const TileKernelArgs a = b.jobs[w.job];
+    tile_block<COORD, NSUM, FIXED>(a.xi, a.tile, (size_t)w.row);
 }
 
 // n_wg == 0 only raises the kernel's dynamic LDS limit.
@@ -678,11 +677,11 @@ size_t tile_lds_bytes(int nsum, int nslots, int n_edges)
            (n_edges > 0 ? (size_t)(n_edges + 2) * sizeof(double) : 0);
 }
 
-int launch_tile_pass(int coord, int nsum, const XiKernelArgs &a, int n_wg, int block, size_t lds, void *stream)
+int launch_tile_pass(int coord, int nsum, const TileKernelArgs &a, int n_wg, int block, size_t lds, void *stream)
 {
     hipStream_t st = (hipStream_t)stream;
-    const bool fixed = !a.banded && tile_fixed((int)a.ge.nslots);
-    void (*fn)(XiKernelArgs);
+    const bool fixed = !a.xi.banded && tile_fixed((int)a.xi.ge.nslots);
+    void (*fn)(TileKernelArgs);
     if (nsum == 7)
         fn = coord == TOS_OBSERVING ? tile_pass_kernel<TOS_OBSERVING, 7, false>
              : coord == TOS_POLAR   ? tile_pass_kernel<TOS_POLAR, 7, false>
@@ -696,7 +695,7 @@ int launch_tile_pass(int coord, int nsum, const XiKernelArgs &a, int n_wg, int b
     return (int)launch_one(fn, a, n_wg, block, lds, st);
 }
 
-int launch_tile_batch(int coord, bool fixed, const XiBatchArgs &b, int n_wg, int block, size_t lds, void *stream)
+int launch_tile_batch(int coord, bool fixed, const TileBatchArgs &b, int n_wg, int block, size_t lds, void *stream)
 {
     hipStream_t st = (hipStream_t)stream;
     if (coord == TOS_OBSERVING)

@@ -226,7 +226,7 @@ int plan_launch(tos_ctx *ctx, const tos_xi_opts *opts, int prec, int accum, cons
     return TOS_OK;
 }
 
-bool plan_tiles(tos_ctx *ctx, const tos_pairs *p, int accum, const tos_grid &g, XiKernelArgs &a, XiLaunch &L,
+bool plan_tiles(tos_ctx *ctx, const tos_pairs *p, int accum, const tos_grid &g, const TileArgs &t, XiLaunch &L,
                 uint32_t band_rows)
 {
     GridExact ge;
@@ -237,7 +237,7 @@ bool plan_tiles(tos_ctx *ctx, const tos_pairs *p, int accum, const tos_grid &g, 
     L.nsum = xi_nsum(accum);
     L.lds = tile_lds_bytes(L.nsum, slots, tile_edges(g));
     L.block = tile_block_size(L.nsum, slots);
-    L.n_wg = tile_workgroups(p, a.tile, ctx->ncu * tile_threads_per_cu(L.nsum) / L.block, L.block);
+    L.n_wg = tile_workgroups(p, t, ctx->ncu * tile_threads_per_cu(L.nsum) / L.block, L.block);
     L.n_seg = std::min(32, L.n_wg);
     return (int64_t)L.n_wg * L.nbins * (4 + 8 * L.nsum) <= kMaxPartialBytes;
 }
@@ -358,7 +358,7 @@ extern "C" int tos_xi_run(tos_ctx *ctx, const tos_catalog *cat, const tos_pairs 
     // no launch shape asked for
     bool tiles = flags == 0 && (!opts || (opts->block_size == 0 && opts->blocks_per_cu == 0 && opts->wg_per_slot == 0)) &&
                  tile_job(cat, p, g);
-    XiKernelArgs a;
+    TileArgs t;
     if (tiles) {
         if ((rc = ensure_tile_plan(ctx, p)) != TOS_OK) return rc;
         tiles = p->tiles.state == 1;
@@ -378,15 +378,12 @@ extern "C" int tos_xi_run(tos_ctx *ctx, const tos_catalog *cat, const tos_pairs 
     }
     // the theta bins before the kernel arguments, which hold their address
     if (g.type == TOS_OBSERVING && (rc = ensure_theta(ctx, p, g)) != TOS_OK) return rc;
-    if (tiles) {
-        fill_args(cat, p, g, true, a);
-        tiles = tile_args(p, g, a);
-    }
+    tiles = tiles && tile_args(p, g, t);
     // a grid too large for one LDS histogram runs in bands of axis-0 rows,
     // one full pass over the pairs per band
     uint32_t rows = band_rows_for(ctx, accum, g, tiles);
     XiLaunch L;
-    if (tiles && (rows == 0 || !plan_tiles(ctx, p, accum, g, a, L, rows))) {
+    if (tiles && (rows == 0 || !plan_tiles(ctx, p, accum, g, t, L, rows))) {
         tiles = false;
         rows = band_rows_for(ctx, accum, g);
     }
@@ -399,8 +396,10 @@ extern "C" int tos_xi_run(tos_ctx *ctx, const tos_catalog *cat, const tos_pairs 
     const bool banded = rows < ge.n[0];
     if (!tiles && (rc = plan_launch(ctx, opts, prec, accum, g, n_items, L, banded ? rows : 0)) != TOS_OK) return rc;
     if ((rc = reserve_scratch(ctx, L, nbins)) != TOS_OK) return rc;
+    XiKernelArgs a;
     if (tiles) {
-        a.tile.next = (uint32_t *)((unsigned long long *)ctx->recheck.ptr + 2);
+        fill_args(cat, p, g, true, a);
+        t.next = (uint32_t *)((unsigned long long *)ctx->recheck.ptr + 2);
     } else {
         std::vector<int32_t> wgp;
         balance_items(p->item_cost, L.n_wg, wgp);
@@ -441,7 +440,7 @@ extern "C" int tos_xi_run(tos_ctx *ctx, const tos_catalog *cat, const tos_pairs 
         }
         if (tiles && r0 > 0 && (e = launch_zero_u64(a.n_recheck + 2, 1, ctx->stream)) != hipSuccess)
             return hip_fail(ctx, (hipError_t)e, "tile counter clear");
-        e = tiles ? launch_tile_pass(g.type, L.nsum, a, L.n_wg, L.block, L.lds, ctx->stream)
+        e = tiles ? launch_tile_pass(g.type, L.nsum, TileKernelArgs{a, t}, L.n_wg, L.block, L.lds, ctx->stream)
                   : launch_xi(g.type, prec, accum, a, L.n_wg, L.block, L.lds, ctx->stream);
         if (e != hipSuccess) return hip_fail(ctx, (hipError_t)e, "xi kernel launch");
         if (!banded) hipEventRecord(ctx->ev1, ctx->stream);   // the pair kernel alone
