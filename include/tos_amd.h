@@ -170,6 +170,15 @@ int tos_pairs_upload(tos_ctx *ctx, const tos_catalog *cat, const tos_pair_csr *c
                      tos_pairs **out);
 int tos_pairs_free(tos_ctx *ctx, tos_pairs *p);
 int tos_pairs_stats(const tos_pairs *p, tos_pair_stats *out);
+/* The kernel that the last tos_xi_run or tos_batch_run over this list took:
+ * the general pair kernel, or the pass on the wavelength ladder that the
+ * spectra of a catalogue share.  No counterpart in the reference. */
+enum tos_pass {
+    TOS_PASS_NONE = 0,       /* no pass yet, or one without work items */
+    TOS_PASS_GENERAL = 1,
+    TOS_PASS_LADDER = 2
+};
+int tos_pairs_last_pass(const tos_pairs *p, int32_t *pass);
 /* Copy the CSR back (arrays sized from tos_pairs_stats; any may be NULL). */
 int tos_pairs_download(tos_ctx *ctx, const tos_pairs *p, int32_t *row_los,
                        int32_t *row_skybin, int64_t *row_ptr, int32_t *other,

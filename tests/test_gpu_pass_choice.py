@@ -1,0 +1,91 @@
+"""Which kernel a pass takes (tos_pairs_last_pass): the comparisons of
+test_gpu_tile.py hold the pass on the ladder against the general kernel, so
+the default run has to be on the ladder there, and off it where a catalogue
+has none."""
+import ctypes
+
+import numpy as np
+import pytest
+
+import tos_amd
+from tos_amd import GridSpec, _lib, synth
+from test_gpu_tile import CART, GRIDS, OBS, POLAR_GRIDS, masked
+
+ALL = GRIDS + [(tos_amd.POLAR,) + s for s in POLAR_GRIDS]
+
+
+def test_last_pass_refuses_invalid_arguments():
+    k = ctypes.c_int32(0)
+    assert _lib.lib().tos_pairs_last_pass(None, ctypes.byref(k)) == 1
+
+
+@pytest.fixture(scope="module")
+def lists(dev):
+    """The catalogue of test_gpu_tile.py and its pair list for each grid type."""
+    cat = masked(synth.lya_catalog(520, area_deg2=40.0, seed=71), 0.05)
+    dcat = dev.upload(cat)
+    wide = {CART: GridSpec.cartesian(), OBS: GridSpec.observing(), tos_amd.POLAR: GridSpec.polar()}
+    out = {t: dcat.pairs(g.max_angular_scale(cat.scale), order=3, nthreads=8) for t, g in wide.items()}
+    yield cat, dcat, out
+    for p in out.values():
+        p.free()
+    dcat.free()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("spec", ALL, ids=[f"{s[0]}-{s[1]}-{s[2]}-{s[3][-1]}" for s in ALL])
+def test_survey_catalogues_take_the_ladder(dev, lists, spec):
+    pairs, grid = lists[2][spec[0]], GridSpec.from_specs(*spec)
+    print(f"case: grid {grid.specs} type {grid.type}", flush=True)
+    for prec in (tos_amd.FP64, tos_amd.FP32C):
+        pairs.run(grid, precision=prec, flags=tos_amd.XI_NO_ZCONST)
+        assert pairs.last_pass() == tos_amd.PASS_GENERAL
+        pairs.run(grid, precision=prec)
+        assert pairs.last_pass() == tos_amd.PASS_LADDER
+    pairs.run(grid, precision=tos_amd.FP64, accum=tos_amd.ACC_ALL)
+    assert pairs.last_pass() == tos_amd.PASS_LADDER
+
+
+@pytest.mark.gpu
+def test_batches_and_sky_bins(dev, lists):
+    pairs, grid = lists[2][CART], GridSpec.cartesian()
+    pairs.run_per_skybin(grid, precision=tos_amd.FP32C)
+    assert pairs.last_pass() == tos_amd.PASS_GENERAL
+    jobs = [(lists[2][t], g, p) for t, g, p in ((CART, grid, tos_amd.FP64), (OBS, GridSpec.observing(), tos_amd.FP32C),
+                                                 (tos_amd.POLAR, GridSpec.polar(), tos_amd.FP32C))]
+    dev.batch_run(jobs)
+    assert [p.last_pass() for p, _, _ in jobs] == [tos_amd.PASS_LADDER] * 3
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("change", ["off_ladder", "two_wavelengths", "descending", "overflow", "few_pairs", "shape"])
+def test_passes_without_a_ladder(dev, lists, change):
+    cat = lists[0]
+    kw = {k: getattr(cat, k).copy() for k in ("value", "loglam", "weight", "distance")}
+    n, a, b = cat.n_pix, cat.offsets[40], cat.offsets[41]
+    if change == "off_ladder":
+        kw["distance"] += np.repeat(np.arange(cat.n_los), cat.counts()).astype(np.float32) * np.float32(1e-2)
+    elif change == "two_wavelengths":
+        kw["loglam"][n // 2] += np.float32(1e-5)
+    elif change == "descending":
+        for k in ("distance", "loglam"):
+            kw[k][a:b] = kw[k][a:b][::-1]
+    elif change == "overflow":
+        kw["weight"][n // 3] = kw["value"][n // 3] = 1e30
+    c = synth.Catalog(cat.ra, cat.dec, cat.offsets, kw["value"], kw["loglam"], kw["weight"], kw["distance"], cat.zq,
+                      cat.scale)
+    if change == "few_pairs":
+        c = c.subset(np.arange(20))
+    grid = GridSpec.cartesian()
+    dcat = dev.upload(c)
+    pairs = dcat.pairs(grid.max_angular_scale(c.scale), order=3, nthreads=8)
+    assert pairs.last_pass() == tos_amd.PASS_NONE
+    print(f"case: {change}", flush=True)
+    for _ in range(2):
+        pairs.run(grid, precision=tos_amd.FP32C, block_size=512 if change == "shape" else 0)
+        assert pairs.last_pass() == tos_amd.PASS_GENERAL
+    if change != "shape":
+        dev.batch_run([(pairs, grid, tos_amd.FP32C)])
+        assert pairs.last_pass() == tos_amd.PASS_GENERAL
+    pairs.free()
+    dcat.free()

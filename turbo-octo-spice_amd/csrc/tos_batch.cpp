@@ -604,6 +604,7 @@ int xi_run_per_skybin(tos_ctx *ctx, const tos_catalog *cat, tos_pairs *p, const 
     out->num_guard_rechecks = rechecks;
     out->num_pairs_evaluated = evaluated;
     out->kernel_ms = ms;
+    p->last_pass = TOS_PASS_GENERAL;
     return TOS_OK;
 }
 
@@ -694,6 +695,10 @@ extern "C" int tos_batch_run(tos_ctx *ctx, int32_t n, const tos_batch_job *jobs,
     batch_collect(B, n, ms, out);
     for (int32_t j = 0; j < n; ++j)
         if (jobs[j].precision == TOS_FP64) out[j].num_guard_rechecks = 0;
+    for (const BatchGroup &G : B.groups)
+        for (int j : G.jobs)
+            const_cast<tos_pairs *>(jobs[j].pairs)->last_pass =
+                jobs[j].pairs->n_items == 0 ? TOS_PASS_NONE : G.key.tile ? TOS_PASS_LADDER : TOS_PASS_GENERAL;
     return TOS_OK;
 }
 

@@ -637,6 +637,13 @@ extern "C" int tos_pairs_stats(const tos_pairs *p, tos_pair_stats *out)
     return TOS_OK;
 }
 
+extern "C" int tos_pairs_last_pass(const tos_pairs *p, int32_t *pass)
+{
+    if (!p || !pass) return TOS_ERR_INVALID;
+    *pass = p->last_pass;
+    return TOS_OK;
+}
+
 extern "C" int tos_pairs_download(tos_ctx *ctx, const tos_pairs *p, int32_t *row_los, int32_t *row_skybin,
                                   int64_t *row_ptr, int32_t *other, double *cos_sep)
 {

@@ -133,6 +133,7 @@ struct tos_pairs {
     double theta_key[3] = {0, 0, 0};
     int32_t theta_n = -1;
     tos::TilePlan tiles;
+    int32_t last_pass = TOS_PASS_NONE;   // of tos_xi_run / tos_batch_run
 };
 
 namespace tos {

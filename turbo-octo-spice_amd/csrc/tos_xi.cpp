@@ -368,6 +368,7 @@ extern "C" int tos_xi_run(tos_ctx *ctx, const tos_catalog *cat, const tos_pairs 
     if ((rc = ensure_items(ctx, p, !(flags & TOS_XI_NO_TRANSPOSE), nullptr, tuned_step_cap(ctx, g, prec))) != TOS_OK)
         return rc;
     const size_t n_items = (size_t)p->n_items;
+    p->last_pass = TOS_PASS_NONE;
     if (n_items == 0) {
         std::memset(out->num_pairs, 0, sizeof(uint64_t) * nbins);
         std::memset(out->didj, 0, sizeof(double) * nbins);
@@ -462,6 +463,7 @@ extern "C" int tos_xi_run(tos_ctx *ctx, const tos_catalog *cat, const tos_pairs 
     out->kernel_ms = ms;
     out->num_guard_rechecks = prec == TOS_FP32C ? nre[0] : 0;
     out->num_pairs_evaluated = nre[1];
+    p->last_pass = tiles ? TOS_PASS_LADDER : TOS_PASS_GENERAL;
     uint64_t used = 0;
     for (int b = 0; b < nbins; ++b) {
         const double *s = &sums[(size_t)b * L.nsum];

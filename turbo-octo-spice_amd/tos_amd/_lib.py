@@ -23,6 +23,7 @@ SKY_HEALPIX, SKY_PLATES = 0, 1
 FP64, FP32C = 0, 1
 ACC_CORE, ACC_ALL = 0, 1
 BRUTE_FP64, BRUTE_FP32 = 0, 1
+PASS_NONE, PASS_GENERAL, PASS_LADDER = 0, 1, 2
 XI_NO_WINDOW, XI_NO_TRANSPOSE, XI_NO_INTERLEAVE, XI_NO_ZCONST = 1, 2, 4, 8
 
 
@@ -126,6 +127,7 @@ SIGNATURES = {
     "tos_pairs_upload": (C.c_int, [_P, _P, C.POINTER(PairCSR), C.POINTER(_P)]),
     "tos_pairs_free": (C.c_int, [_P, _P]),
     "tos_pairs_stats": (C.c_int, [_P, C.POINTER(PairStats)]),
+    "tos_pairs_last_pass": (C.c_int, [_P, C.POINTER(C.c_int32)]),
     "tos_pairs_download": (C.c_int, [_P, _P, _P, _P, _P, _P, _P]),
     "tos_xi_run": (C.c_int, [_P, _P, _P, C.POINTER(Grid), C.POINTER(XiOpts),
                              C.POINTER(XiResult)]),

@@ -228,6 +228,13 @@ class DevicePairs:
         check(lib().tos_pairs_stats(self.h, C.byref(s)))
         return s.as_dict()
 
+    def last_pass(self) -> int:
+        """PASS_LADDER, PASS_GENERAL or PASS_NONE: the kernel of the list's
+        last run or batched run (tos_pairs_last_pass)."""
+        k = C.c_int32(0)
+        check(lib().tos_pairs_last_pass(self.h, C.byref(k)))
+        return int(k.value)
+
     def download(self):
         st = self.stats()
         nr = st["n_rows"]
