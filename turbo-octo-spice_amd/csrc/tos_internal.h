@@ -283,7 +283,7 @@ struct LadderArgs {
     const LosInfo *los;
     int64_t n_los, n_pix;
     uint64_t *table;              // [kLadderTable] {loglam bits << 32 | distance bits}, all ones: empty
-    uint32_t *state;              // [0] not a ladder, [1] entries, [2] blocks in all
+    uint32_t *state;              // [0] not a ladder, [1] entries, [2] blocks in all (the survey sets all three)
     const uint16_t *step;         // [kLadderTable] ladder step of each table entry
     LadderLos *place;             // [n_los]
     uint32_t *nblk_of;            // [n_los] blocks of each sightline, then their exclusive prefix

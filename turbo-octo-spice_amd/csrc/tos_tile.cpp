@@ -49,39 +49,35 @@ int ensure_ladder(tos_ctx *ctx, tos_catalog *cat)
     if (L.state) return TOS_OK;
     L.state = 2;
     if (cat->n_los == 0 || cat->n_pix == 0 || !(cat->dmin > 1e-3) || !cat->d_sorted || !cat->l_sorted) return TOS_OK;
-    Scratch sc;
-    DevBuf &table = sc.b[0], &state = sc.b[1], &step = sc.b[2], &nblk_of = sc.b[3];
-    int rc;
-    std::vector<uint64_t> tab(kLadderTable, ~0ull);
+    // the table and the state in the context's scratch: a catalogue without a
+    // ladder costs no allocation
+    constexpr size_t kTableBytes = (size_t)kLadderTable * 8;
     uint32_t st[3] = {0, 0, 0};
-    if (table.reserve(tab.size() * 8) != TOS_OK || state.reserve(sizeof(st)) != TOS_OK ||
-        step.reserve(kLadderTable * 2) != TOS_OK || nblk_of.reserve((size_t)cat->n_los * 4) != TOS_OK ||
-        L.place.reserve((size_t)cat->n_los * sizeof(LadderLos)) != TOS_OK) {
-        L.release();
-        return TOS_OK;
-    }
-    if ((rc = upload(ctx, table, tab.data(), tab.size() * 8, "ladder table")) != TOS_OK ||
-        (rc = upload(ctx, state, st, sizeof(st), "ladder state")) != TOS_OK)
-        return rc;
+    if (ctx->scratch_a.reserve(kTableBytes + sizeof(st)) != TOS_OK) return TOS_OK;
+    int rc;
     LadderArgs a{};
     a.pix = (const float4 *)cat->pix.ptr;
     a.los = (const LosInfo *)cat->los.ptr;
     a.n_los = cat->n_los;
     a.n_pix = cat->n_pix;
-    a.table = (uint64_t *)table.ptr;
-    a.state = (uint32_t *)state.ptr;
-    a.step = (const uint16_t *)step.ptr;
-    a.place = (LadderLos *)L.place.ptr;
-    a.nblk_of = (uint32_t *)nblk_of.ptr;
+    a.table = (uint64_t *)ctx->scratch_a.ptr;
+    a.state = (uint32_t *)((char *)ctx->scratch_a.ptr + kTableBytes);
     int e = launch_ladder_collect(a, ctx->stream);
     if (e != hipSuccess) return hip_fail(ctx, (hipError_t)e, "ladder collection");
-    hipError_t he = hipMemcpyAsync(tab.data(), table.ptr, tab.size() * 8, hipMemcpyDeviceToHost, ctx->stream);
-    if (he != hipSuccess) return hip_fail(ctx, he, "ladder table copy");
-    if ((rc = copy_back(ctx, st, state.ptr, sizeof(st), "ladder state copy")) != TOS_OK) return rc;
-    if (st[0]) {
+    if ((rc = copy_back(ctx, st, a.state, sizeof(st), "ladder state copy")) != TOS_OK) return rc;
+    if (st[0]) return TOS_OK;
+    std::vector<uint64_t> tab(kLadderTable);
+    if ((rc = copy_back(ctx, tab.data(), a.table, kTableBytes, "ladder table copy")) != TOS_OK) return rc;
+    Scratch sc;
+    DevBuf &step = sc.b[0], &nblk_of = sc.b[1];
+    if (step.reserve(kLadderTable * 2) != TOS_OK || nblk_of.reserve((size_t)cat->n_los * 4) != TOS_OK ||
+        L.place.reserve((size_t)cat->n_los * sizeof(LadderLos)) != TOS_OK) {
         L.release();
         return TOS_OK;
     }
+    a.step = (const uint16_t *)step.ptr;
+    a.place = (LadderLos *)L.place.ptr;
+    a.nblk_of = (uint32_t *)nblk_of.ptr;
     // the steps in ascending distance; wavelengths must ascend with them
     struct Step {
         float d, l;
@@ -119,7 +115,7 @@ int ensure_ladder(tos_ctx *ctx, tos_catalog *cat)
         return rc;
     e = launch_ladder_place(a, ctx->stream);
     if (e != hipSuccess) return hip_fail(ctx, (hipError_t)e, "ladder placement");
-    if ((rc = copy_back(ctx, st, state.ptr, sizeof(st), "ladder block count")) != TOS_OK) return rc;
+    if ((rc = copy_back(ctx, st, a.state, sizeof(st), "ladder block count")) != TOS_OK) return rc;
     if (st[0] || st[2] >= (1u << 24) ||   // 32-bit byte offsets
         L.pix.reserve((size_t)st[2] * kBlockBytes) != TOS_OK) {
         L.release();
@@ -128,7 +124,7 @@ int ensure_ladder(tos_ctx *ctx, tos_catalog *cat)
     a.out = (float *)L.pix.ptr;
     e = launch_ladder_fill(a, st[2], ctx->stream);
     if (e != hipSuccess) return hip_fail(ctx, (hipError_t)e, "ladder fill");
-    if ((rc = copy_back(ctx, st, state.ptr, sizeof(st), "ladder state copy")) != TOS_OK) return rc;
+    if ((rc = copy_back(ctx, st, a.state, sizeof(st), "ladder state copy")) != TOS_OK) return rc;
     if (st[0]) {
         L.release();
         return TOS_OK;

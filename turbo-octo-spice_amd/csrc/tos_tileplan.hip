@@ -47,6 +47,50 @@ __device__ __forceinline__ int find_step(const uint64_t *table, uint64_t key)
     return -1;
 }
 
+// Clears the table.  The last workgroup looks at kSample pixels spread over
+// the catalogue: a distance with two wavelengths, or more than kMaxLadder
+// distances, and there is no ladder (state[0]).  Finding that out by filling
+// the table took 2 ms for 16,000 pixels off any ladder and 14 ms for 440,000
+// (every thread of the device inserts, and probes an overfull table); this
+// and its read-back take 20 to 30 us.
+constexpr uint32_t kSample = 4096;
+constexpr int kMaxProbe = 64;   // the tables are a quarter and half full at most
+static_assert(kSample >= 2 * kMaxLadder && (kSample & (kSample - 1)) == 0, "slots of the sample's table");
+__global__ void __launch_bounds__(1024) ladder_clear(LadderArgs a)
+{
+    __shared__ unsigned long long seen[kSample];
+    __shared__ uint32_t distinct, bad;
+    const int32_t i = (int32_t)(blockIdx.x * 1024 + threadIdx.x);
+    if (i < kLadderTable) {   // whole workgroups: kLadderTable is a multiple of 1024
+        a.table[i] = kEmpty;
+        return;
+    }
+    for (uint32_t q = threadIdx.x; q < kSample; q += 1024) seen[q] = kEmpty;
+    if (threadIdx.x == 0) distinct = bad = 0;
+    __syncthreads();
+    const int64_t n = min(a.n_pix, (int64_t)kSample), step = a.n_pix / n;
+    for (uint32_t q = threadIdx.x; q < n; q += 1024) {
+        const uint64_t key = step_key(a.pix[q * step]);
+        uint32_t h = slot_hash((uint32_t)key) & (kSample - 1);
+        for (int probe = 0; probe < kMaxProbe; ++probe) {
+            // decided: no more of the probes, which get long
+            if (__hip_atomic_load(&distinct, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) > (uint32_t)kMaxLadder) break;
+            const uint64_t k = atomicCAS(&seen[h], (unsigned long long)kEmpty, (unsigned long long)key);
+            if (k == kEmpty) atomicAdd(&distinct, 1u);
+            else if (k != key && (uint32_t)k == (uint32_t)key) bad = 1;
+            if (k == kEmpty || (uint32_t)k == (uint32_t)key) break;
+            if (probe + 1 == kMaxProbe) bad = 1;
+            h = (h + 1) & (kSample - 1);
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        a.state[0] = bad || distinct > (uint32_t)kMaxLadder ? 1u : 0u;
+        a.state[1] = a.state[2] = 0u;
+    }
+}
+static_assert(kLadderTable % 1024 == 0, "ladder_clear's workgroups clear or sample as a whole");
+
 // Every distinct (distance, loglam) of the catalogue into the hash table; a
 // distance with two wavelengths, or more than kMaxLadder of them, ends the
 // collection (state[0]).  The table is read before it is written, and almost
@@ -63,7 +107,7 @@ __global__ void __launch_bounds__(256) ladder_collect(LadderArgs a)
         last = key;
         uint32_t h = slot_hash((uint32_t)key);
         for (int probe = 0;; ++probe) {
-            if (probe == kLadderTable) {
+            if (probe == kMaxProbe) {
                 a.state[0] = 1;
                 break;
             }
@@ -326,6 +370,7 @@ int launch_ladder_collect(const LadderArgs &a, void *stream)
 {
     if (a.n_pix <= 0) return 0;
     const int64_t blocks = (a.n_pix + 255) / 256;
+    hipLaunchKernelGGL(ladder_clear, dim3(kLadderTable / 1024 + 1), dim3(1024), 0, (hipStream_t)stream, a);
     hipLaunchKernelGGL(ladder_collect, dim3((unsigned)(blocks < 4096 ? blocks : 4096)), dim3(256), 0,
                        (hipStream_t)stream, a);
     return (int)hipGetLastError();
