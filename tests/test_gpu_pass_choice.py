@@ -9,7 +9,7 @@ import pytest
 
 import tos_amd
 from tos_amd import GridSpec, _lib, synth
-from test_gpu_tile import CART, GRIDS, OBS, POLAR_GRIDS, masked
+from test_gpu_tile import CART, GRIDS, OBS, POLAR_GRIDS, close, masked
 
 ALL = GRIDS + [(tos_amd.POLAR,) + s for s in POLAR_GRIDS]
 
@@ -87,5 +87,31 @@ def test_passes_without_a_ladder(dev, lists, change):
     if change != "shape":
         dev.batch_run([(pairs, grid, tos_amd.FP32C)])
         assert pairs.last_pass() == tos_amd.PASS_GENERAL
+    pairs.free()
+    dcat.free()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("unit", [1e-3, 0.05, 1.0, 10.0])
+@pytest.mark.parametrize("polar", [False, True], ids=["cartesian", "polar"])
+def test_distances_in_other_units(dev, lists, unit, polar):
+    """Edges are tracked from a squared separation on that scales with the
+    distances: few pixel pairs take the reference arithmetic in any unit."""
+    cat, u = lists[0], np.float32(unit)
+    c = synth.Catalog(cat.ra, cat.dec, cat.offsets, cat.value, cat.loglam, cat.weight, cat.distance * u, cat.zq,
+                      cat.scale * float(u))
+    top = 200.0 * float(u)
+    grid = GridSpec.from_specs(tos_amd.POLAR if polar else CART, f"[0:{top!r}]*50",
+                               "[0:1]*20" if polar else f"[0:{top!r}]*50", "[3.556:3.735]*1")
+    dcat = dev.upload(c)
+    pairs = dcat.pairs(grid.max_angular_scale(c.scale), order=3, nthreads=8)
+    print(f"case: unit {unit} polar {polar}", flush=True)
+    h = pairs.run(grid, precision=tos_amd.FP32C)
+    assert pairs.last_pass() == tos_amd.PASS_LADDER
+    close(h, *(lambda r: (r.num_pairs, {"didj": r.didj, "wgt": r.wgt}))(
+        pairs.run(grid, precision=tos_amd.FP64, flags=tos_amd.XI_NO_ZCONST)))
+    # r < 2 Mpc/h of 200 is 1e-4 of the pairs of a uniform sky, and some 1e-4
+    # of the rest lie within the error bound of an edge
+    assert h.num_guard_rechecks < 0.01 * h.num_pairs_evaluated
     pairs.free()
     dcat.free()

@@ -127,6 +127,7 @@ struct TileArgs {
     // `ulps` float steps below a pair's value is certainly below it
     uint32_t ulps;
     double eps;
+    double s_min;                 // from this squared separation up
     double width0, width1;        // bin widths of axes 0 and 1
 };
 

@@ -285,15 +285,21 @@ bool tile_args(const tos_pairs *p, const tos_grid &g, TileArgs &t)
             }
     }
     t.band = band;
-    // K of an edge at squared separation s >= 4 is known within a relative
+    // K of an edge at squared separation s >= s_min is known within a relative
     //   2^-24 (f32 K) + 3 2^-24 (f32 threshold: the squared edge, 1 / (d1 d2)
     //   and their product)
-    //   + (7e-15 dmax^2 (the reference's FP64 rounding of r^2) + 2^-24 base) / 4,
+    //   + (7e-15 dmax^2 (the reference's FP64 rounding of r^2) + 2^-24 base) / s_min,
     // base <= ulp32(dmax^2) + 2 * 2^-24 dmax * axis-0 range; doubled
     // (Polar: base <= ulp32(dmax^2), six more roundings in the threshold, and
     // r^2 = r_par^2 / mu^2 as the reference's rounded mu, of at least (smallest
-    // step) / R, has it)
+    // step) / R, has it).
+    // s_min is 4 (Mpc/h)^2 for the distances of a survey and goes down with
+    // dmax^2, like the errors: in Gpc/h every pair would lie below 4, and each
+    // takes the reference arithmetic there (400,000 sightline pairs 29 ms, the
+    // general kernel 23, this 1.9).
     const double u = std::ldexp(1.0, -24);
+    const double scale = std::min(1.0, cat->dmax / 5000.0);
+    t.s_min = 4.0 * scale * scale;
     double base = 2.0 * u * cat->dmax * cat->dmax + 4.0 * u * cat->dmax * std::fabs(g.max[0]);
     double ops = 4.0, abs_err = 7e-15 * cat->dmax * cat->dmax;
     if (g.type == TOS_POLAR) {
@@ -306,7 +312,7 @@ bool tile_args(const tos_pairs *p, const tos_grid &g, TileArgs &t)
         const double M = 1.0 + std::fabs(g.min[1]) + g.nbins[1] * g.width[1];
         abs_err += 1e-15 * R * R * (4.0 + M * R / step);
     }
-    t.eps = 2.0 * (ops * u + (abs_err + u * base) / 4.0);
+    t.eps = 2.0 * (ops * u + (abs_err + u * base) / t.s_min);
     t.ulps = (uint32_t)std::ceil(2.2 * t.eps / u) + 2;
     return t.eps < 1e-4;
 }

@@ -115,7 +115,7 @@ struct SlowBin {
 // its pair of steps (thr < 0: this pair only).  Out of line: it runs for a
 // tile's first pair and for the rare pairs next to an edge.
 __device__ __forceinline__ SlowBin slow_cart(const GridExact &ge, double width1, uint32_t band_lo8, float d1, float l1, float d2,
-                                             float l2, double c, double eps, float K, float k_safe)
+                                             float l2, double c, double eps, double s_min, float K, float k_safe)
 {
     const double d2d = (double)d2;
     const double r1_sq = (double)(d1 * d1), two = (double)(2.0f * d1) * c;
@@ -132,7 +132,7 @@ __device__ __forceinline__ SlowBin slow_cart(const GridExact &ge, double width1,
     const float k_up = edge_k(ge.min[1], width1, (float)up, base, inv);
     const bool no_lo = t <= -1.0 || __builtin_fma(lo, width1, ge.min[1]) <= 0.0;
     const float k_lo = no_lo ? -1.0f : edge_k(ge.min[1], width1, (float)lo, base, inv);
-    const bool settled = rp2 >= 4.0 && k_lo <= k_safe && (t >= n1 || K < k_up) && z_bin_exact(ge, l1, l2) < ge.n[2];
+    const bool settled = rp2 >= s_min && k_lo <= k_safe && (t >= n1 || K < k_up) && z_bin_exact(ge, l1, l2) < ge.n[2];
     SlowBin s;
     s.off8 = slot == kReject ? kReject : (slot << 3) - band_lo8;
     s.edge = (float)up;
@@ -187,7 +187,8 @@ struct SlowPolar {
 };
 
 __device__ __forceinline__ SlowPolar slow_polar(const GridExact &ge, double width0, const double *table, uint32_t band_lo8,
-                                                float d1, float l1, float d2, float l2, double c, float inv, float K, float k_safe)
+                                                float d1, float l1, float d2, float l2, double c, float inv,
+                                                double s_min, float K, float k_safe)
 {
     const double d2d = (double)d2;
     const double r1_sq = (double)(d1 * d1), two = (double)(2.0f * d1) * c;
@@ -209,7 +210,7 @@ __device__ __forceinline__ SlowPolar slow_polar(const GridExact &ge, double widt
     const float km = no_mu ? __builtin_inff() : polar_k(p, p.rr, table[mu0 + i1]);
     const bool dead = t0 >= n0 || t1 <= -1.0;
     const uint32_t iz = z_bin_exact(ge, l1, l2);
-    const bool settled = r_sq - p.rr >= 4.0 && t0 > -1.0 && k0 <= k_safe && k1 <= k_safe && iz < ge.n[2] &&
+    const bool settled = r_sq - p.rr >= s_min && t0 > -1.0 && k0 <= k_safe && k1 <= k_safe && iz < ge.n[2] &&
                          (dead || (K < kr && K < km));
     SlowPolar s;
     s.edges = 0u;                      // in the mu axis
@@ -442,7 +443,8 @@ __device__ __forceinline__ void tile_block(const XiKernelArgs &a, const TileArgs
                         if constexpr (POLAR) {
                             const float d1 = step_d[k1];
                             const SlowPolar s = slow_polar(ge, t.width0, table, a.band_lo8, d1, step_l[k1], d2, l2, cs,
-                                                           polar_inv(d1, d2, keep), K, __uint_as_float(kb_safe));
+                                                           polar_inv(d1, d2, keep), t.s_min, K,
+                                                           __uint_as_float(kb_safe));
                             nre += s.kr < 0.0f ? 1u : 0u;
 #pragma unroll
                             for (int q = 0; q < 4; ++q) {
@@ -453,8 +455,8 @@ __device__ __forceinline__ void tile_block(const XiKernelArgs &a, const TileArgs
                             }
                             continue;
                         }
-                        const SlowBin s = slow_cart(ge, t.width1, a.band_lo8, step_d[k1], step_l[k1], d2, l2, cs, t.eps, K,
-                                                    __uint_as_float(kb_safe));
+                        const SlowBin s = slow_cart(ge, t.width1, a.band_lo8, step_d[k1], step_l[k1], d2, l2, cs, t.eps,
+                                                    t.s_min, K, __uint_as_float(kb_safe));
                         nre += s.thr < 0.0f ? 1u : 0u;
 #pragma unroll
                         for (int q = 0; q < 4; ++q) {
