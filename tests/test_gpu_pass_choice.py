@@ -115,3 +115,87 @@ def test_distances_in_other_units(dev, lists, unit, polar):
     assert h.num_guard_rechecks < 0.01 * h.num_pairs_evaluated
     pairs.free()
     dcat.free()
+
+
+def thinned(cat, keep):
+    owner = np.repeat(np.arange(cat.n_los), cat.counts())
+    off = np.zeros(cat.n_los + 1, np.int64)
+    np.cumsum(np.bincount(owner[keep], minlength=cat.n_los), out=off[1:])
+    return synth.Catalog(cat.ra, cat.dec, off, cat.value[keep], cat.loglam[keep], cat.weight[keep],
+                         cat.distance[keep], cat.zq, cat.scale)
+
+
+def passes(dev, cat, grid, n, prec=tos_amd.FP32C):
+    """The kernels of n passes over a new pair list, whose results must agree
+    with the general kernel's."""
+    dcat = dev.upload(cat)
+    pairs = dcat.pairs(grid.max_angular_scale(cat.scale), order=3, nthreads=8)
+    assert pairs.stats()["num_sightline_pairs_used"] >= 400
+    out = []
+    for k in range(n):
+        print(f"case: {cat.n_los} sightlines {cat.n_pix} pixels grid {grid.specs} pass {k}", flush=True)
+        h = pairs.run(grid, precision=prec)
+        out.append(pairs.last_pass())
+        if k in (0, n - 1):
+            ref = pairs.run(grid, precision=tos_amd.FP64, flags=tos_amd.XI_NO_ZCONST)
+            close(h, ref.num_pairs, {"didj": ref.didj, "wgt": ref.wgt})
+    pairs.free()
+    dcat.free()
+    return out
+
+
+# Forms whose visits cost more than the pixel pairs they hold: thinned spectra,
+# bins far narrower than the pairs' separations differ, pairs too close to track
+COSTLY = {
+    "masked": lambda: (thinned(c := synth.lya_catalog(400, area_deg2=130.0, seed=3),
+                               np.random.default_rng(5).random(c.n_pix) < 0.03), GridSpec.cartesian()),
+    "every_25th": lambda: (thinned(c := synth.lya_catalog(700, area_deg2=100.0, seed=3),
+                                   (np.arange(c.n_pix) - np.repeat(c.offsets[:-1], c.counts())) % 25 == 0),
+                           GridSpec.cartesian()),
+    "narrow_bins": lambda: (synth.lya_catalog(120, area_deg2=40.0, seed=3),
+                            GridSpec.from_specs(CART, "[0:200]*2", "[0:200]*4000", "[3.556:3.735]*1")),
+    "close_pairs": lambda: (synth.lya_catalog(800, area_deg2=0.2, seed=3),
+                            GridSpec.from_specs(CART, "[0:2]*10", "[0:2]*10", "[3.556:3.735]*1")),
+}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("form", list(COSTLY))
+def test_forms_that_the_ladder_makes_slower(dev, form):
+    cat, grid = COSTLY[form]()
+    assert passes(dev, cat, grid, 8) == [tos_amd.PASS_GENERAL] * 8
+
+
+@pytest.mark.gpu
+def test_a_small_list_gets_its_plan_once_it_has_paid(dev):
+    """The plan of a small, thinned list costs more than a pass gains: the
+    first passes go without, later ones have it, for good."""
+    cat = synth.lya_catalog(60, area_deg2=5.0, seed=3)
+    cat = thinned(cat, np.random.default_rng(5).random(cat.n_pix) < 0.3)
+    p = passes(dev, cat, GridSpec.cartesian(), 12)
+    assert p[0] == tos_amd.PASS_GENERAL and p[-1] == tos_amd.PASS_LADDER
+    assert p == sorted(p)
+
+
+@pytest.mark.gpu
+def test_batches_choose_as_a_whole(dev):
+    """Jobs too small for a plan each share the launch's verdict, and a sparse
+    job stays on the general kernel among full ones."""
+    grid = GridSpec.cartesian()
+    full = synth.lya_catalog(700, area_deg2=100.0, seed=4)
+    sparse = thinned(full, (np.arange(full.n_pix) - np.repeat(full.offsets[:-1], full.counts())) % 25 == 0)
+    made = []
+    for cat in (full, sparse, synth.lya_catalog(30, area_deg2=3.0, seed=5)):
+        dcat = dev.upload(cat)
+        made.append((dcat, dcat.pairs(grid.max_angular_scale(cat.scale), order=3, nthreads=8)))
+    jobs = [(p, grid, tos_amd.FP32C) for _, p in made]
+    for graph in (False, True, True):
+        res = dev.batch_run(jobs, use_graph=graph)[0]
+        assert [p.last_pass() for _, p in made][:2] == [tos_amd.PASS_LADDER, tos_amd.PASS_GENERAL]
+        for (_, p), h in zip(made, res):
+            ref = p.run(grid, precision=tos_amd.FP64, flags=tos_amd.XI_NO_ZCONST)
+            close(h, ref.num_pairs, {"didj": ref.didj, "wgt": ref.wgt})
+            p.run(grid, precision=tos_amd.FP32C)
+    for dcat, p in made:
+        p.free()
+        dcat.free()

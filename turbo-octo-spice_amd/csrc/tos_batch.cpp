@@ -134,7 +134,6 @@ void add_buffer_key(std::vector<uint64_t> &k, int32_t n, const tos_batch_job *jo
         put(k, p->other.ptr);
         put(k, p->csep.ptr);
         put(k, jobs[j].cat->pix.ptr);
-        k.push_back((uint64_t)p->tiles.state);
     }
     for (const TuneEntry &t : ctx->tuned) k.push_back(((uint64_t)t.block << 32) | (uint32_t)t.blocks_per_cu);
 }
@@ -174,7 +173,7 @@ void plan_tile_group(const tos_ctx *ctx, BatchGroup &G, int max_slots, const tos
 }  // namespace
 
 int batch_prepare(tos_ctx *ctx, int32_t n, const tos_batch_job *jobs, BatchState &B, const ItemSlice *slices,
-                  bool tiles)
+                  const char *tiles)
 {
     // group jobs by kernel variant, decided from each job's own constants
     std::map<VariantKey, std::vector<int>> by;
@@ -187,8 +186,7 @@ int batch_prepare(tos_ctx *ctx, int32_t n, const tos_batch_job *jobs, BatchState
         xi_variant(jobs[j].grid.type, args[(size_t)j].ge, args[(size_t)j].gf, fixed, simple);
         // jobs of the tile path: the precision and `simple` make no difference
         const tos_batch_job &J = jobs[j];
-        const bool tile = tiles && tile_job(J.cat, J.pairs, J.grid) && J.pairs->tiles.state == 1 &&
-                          tile_args(J.pairs, J.grid, targs[(size_t)j]) &&
+        const bool tile = tiles && tiles[j] && tile_args(J.pairs, J.grid, targs[(size_t)j]) &&
                           (int64_t)tile_lds_bytes(2, (int)args[(size_t)j].ge.nslots, kTileMaxEdges) + 64 <= ctx->max_lds_block &&
                           J.pairs->tiles.total / kTileVisits < (uint64_t)kMaxTasks;
         if (tile)
@@ -641,9 +639,13 @@ extern "C" int tos_batch_run(tos_ctx *ctx, int32_t n, const tos_batch_job *jobs,
         if ((rc = ensure_items(ctx, p, true, nullptr, tuned_step_cap(ctx, jobs[j].grid, jobs[j].precision))) !=
             TOS_OK)
             return rc;
-        if (tile_job(jobs[j].cat, p, jobs[j].grid) && (rc = ensure_tile_plan(ctx, p)) != TOS_OK) return rc;
         if (jobs[j].grid.type == TOS_OBSERVING && (rc = ensure_theta(ctx, p, jobs[j].grid)) != TOS_OK) return rc;
     }
+    std::vector<TileJob> tj;
+    std::vector<char> tiles((size_t)n, 0);
+    for (int32_t j = 0; j < n; ++j)
+        tj.push_back(TileJob{const_cast<tos_pairs *>(jobs[j].pairs), &jobs[j].grid, jobs[j].precision, TOS_ACC_CORE});
+    if ((rc = choose_tiles(ctx, n, tj.data(), tiles.data())) != TOS_OK) return rc;
     if (!ctx->batch) {
         ctx->batch = new BatchState();
         if (hipEventCreate(&ctx->batch->ev0) != hipSuccess || hipEventCreate(&ctx->batch->ev1) != hipSuccess) {
@@ -654,10 +656,11 @@ extern "C" int tos_batch_run(tos_ctx *ctx, int32_t n, const tos_batch_job *jobs,
     BatchState &B = *ctx->batch;
     std::vector<uint64_t> key = job_key(n, jobs);
     add_buffer_key(key, n, jobs, ctx);
+    key.insert(key.end(), tiles.begin(), tiles.end());
     if (key != B.key) {
         B.drop_graph();
         B.key.clear();
-        if ((rc = batch_prepare(ctx, n, jobs, B, nullptr, true)) != TOS_OK) return rc;
+        if ((rc = batch_prepare(ctx, n, jobs, B, nullptr, tiles.data())) != TOS_OK) return rc;
         B.key = key;
     }
     hipError_t he;

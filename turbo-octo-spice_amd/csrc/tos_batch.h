@@ -74,10 +74,10 @@ struct ItemSlice {
 // Plan the batch (variant groups, workgroups per job, item ranges), size
 // its buffers and upload the tables; synchronises ctx->stream.  slices:
 // when given, job j covers only its items slices[j] (its result is then the
-// histogram of those items).  tiles: jobs with a tile plan take the tile
-// pass.
+// histogram of those items).  tiles: when given, the jobs with tiles[j] take
+// the tile pass.
 int batch_prepare(tos_ctx *ctx, int32_t n, const tos_batch_job *jobs, BatchState &B,
-                  const ItemSlice *slices = nullptr, bool tiles = false);
+                  const ItemSlice *slices = nullptr, const char *tiles = nullptr);
 // Enqueue the device work of a prepared batch on `stream`.
 int batch_enqueue(tos_ctx *ctx, BatchState &B, int32_t n, hipStream_t stream);
 // Copy the results of a completed batch out of its pinned buffer.

@@ -276,6 +276,7 @@ extern "C" int tos_catalog_upload(tos_ctx *ctx, const tos_sightlines *s, tos_cat
     struct LosScan {
         float lmin, lmax;
         double dmin, dmax, labs;
+        float step;   // smallest loglam step
         bool d_sorted, l_sorted, finite;
     };
     std::vector<LosScan> scan((size_t)bad_off);
@@ -283,11 +284,13 @@ extern "C" int tos_catalog_upload(tos_ctx *ctx, const tos_sightlines *s, tos_cat
     // its scan
     auto pack = [&](int64_t k, float4 *dst) {
         const int64_t a = s->offsets[k], b = s->offsets[k + 1];
-        LosScan r{INFINITY, -INFINITY, INFINITY, 0.0, 0.0, true, true, true};
+        LosScan r{INFINITY, -INFINITY, INFINITY, 0.0, 0.0, INFINITY, true, true, true};
         for (int64_t p = a; p < b; ++p) {
             if (p > a) {
                 if (!(s->distance[p] >= s->distance[p - 1])) r.d_sorted = false;
                 if (!(s->loglam[p] >= s->loglam[p - 1])) r.l_sorted = false;
+                const float up = s->loglam[p] - s->loglam[p - 1];
+                if (up > 0.0f) r.step = std::min(r.step, up);
             }
             const float d = s->distance[p], l = s->loglam[p], w = s->weight[p], v = s->value[p];
             // {distance, loglam, weight, f32(weight * value)} (types.h:78)
@@ -399,6 +402,26 @@ extern "C" int tos_catalog_upload(tos_ctx *ctx, const tos_sightlines *s, tos_cat
     }
     c->dmin = np > 0 ? dmin : 0;
     c->dmax = np > 0 ? dmax : 0;
+    // sampled wavelength geometry: the step is the one that a tenth of the
+    // sightlines undercut (the smallest might be an odd pixel's)
+    double l_lo = INFINITY, l_hi = -INFINITY, span = 0;
+    std::vector<float> steps;
+    const int64_t every = std::max<int64_t>(1, nl / 1024);
+    for (int64_t k = 0; k < nl; k += every) {
+        if (c->h_los[(size_t)k].n < 2) continue;
+        const LosScan &r = scan[(size_t)k];
+        l_lo = std::min(l_lo, (double)r.lmin);
+        l_hi = std::max(l_hi, (double)r.lmax);
+        span += (double)r.lmax - (double)r.lmin;
+        steps.push_back(r.step);
+    }
+    if (!steps.empty()) {
+        std::nth_element(steps.begin(), steps.begin() + (std::ptrdiff_t)(steps.size() / 10), steps.end());
+        const float step = steps[steps.size() / 10];
+        c->l_step = std::isfinite(step) ? (double)step : 0.0;
+        c->l_range = l_hi - l_lo;
+        c->l_span = span / (double)steps.size();
+    }
     rc = upload(ctx, c->los, c->h_los.data(), c->h_los.size() * sizeof(LosInfo), "catalog sightlines");
     if (rc == TOS_OK) {
         hipError_t e = hipStreamSynchronize(ctx->stream);
@@ -477,6 +500,7 @@ extern "C" int tos_pairs_build(tos_ctx *ctx, const tos_catalog *cat, const tos_s
     }
     tos_pairs *p = new (std::nothrow) tos_pairs();
     if (!p) return TOS_ERR_NOMEM;
+    p->max_ang = max_ang;
     int rc = TOS_OK;
     bool undecided = false, done = false;
     if (on_device) {
@@ -486,6 +510,7 @@ extern "C" int tos_pairs_build(tos_ctx *ctx, const tos_catalog *cat, const tos_s
             tos_pairs_free(ctx, p);
             p = new (std::nothrow) tos_pairs();
             if (!p) return TOS_ERR_NOMEM;
+            p->max_ang = max_ang;
         }
     }
     if (!done) {
@@ -531,6 +556,10 @@ extern "C" int tos_pairs_upload(tos_ctx *ctx, const tos_catalog *cat, const tos_
     if (nr == 0) h.row_ptr.assign(1, 0);
     h.other.assign(csr->other, csr->other + np);
     h.cos_sep.assign(csr->cos_sep, csr->cos_sep + np);
+    if (np > 0) {
+        const double c = *std::min_element(h.cos_sep.begin(), h.cos_sep.end());
+        p->max_ang = std::acos(std::max(-1.0, std::min(1.0, c)));
+    }
     // validate and fill stats
     std::vector<int32_t> keys(h.row_skybin);
     std::sort(keys.begin(), keys.end());

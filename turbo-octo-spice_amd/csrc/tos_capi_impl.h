@@ -43,10 +43,14 @@ struct TuneEntry {
 
 // A catalogue on its ladder (tos_tile.cpp).
 struct Ladder {
-    int state = 0;                // 0: not looked for, 1: built, 2: none
+    int state = 0;                // 0: not looked for, 1: built, 2: none, 3: found, its pixels not laid out yet
     int nblk = 0;
+    int n_steps = 0;
+    double mean_nb = 0;           // blocks a sightline covers
     DevBuf pix, d, l, place;
     std::vector<float> h_d, h_l;  // [16 nblk]
+    std::vector<uint64_t> table;  // state 3: the survey's hash table and the step of each slot
+    std::vector<uint16_t> step_of;
     void release();
 };
 
@@ -97,6 +101,9 @@ struct tos_catalog {
     int64_t n_los = 0, n_pix = 0;
     double dmin = 0, dmax = 0;
     double lmax_abs = 0;   // largest |loglam|
+    // loglam of the catalogue, of a sightline, and between neighbouring pixels
+    // (0: no sightline has two pixels); estimates from some of the sightlines
+    double l_range = 0, l_span = 0, l_step = 0;
     bool d_sorted = true, l_sorted = true;   // pixels ascending in every sightline
     tos::DevBuf pix;    // float4 {distance, loglam, weight, weight*value}
     tos::DevBuf los;    // LosInfo
@@ -111,6 +118,7 @@ struct tos_pairs {
     uint64_t uid = tos::next_uid();
     const tos_catalog *cat = nullptr;
     int64_t n_rows = 0, n_pairs = 0;
+    double max_ang = 0;                  // no pair of the list is farther apart than about this
     tos::HostPairs h;
     tos::DevBuf other, csep;
     // false after a device search: h.other / h.cos_sep are copied back only
@@ -133,6 +141,7 @@ struct tos_pairs {
     double theta_key[3] = {0, 0, 0};
     int32_t theta_n = -1;
     tos::TilePlan tiles;
+    int32_t passes_before_plan = 0;      // that took the general path for the plan's cost
     int32_t last_pass = TOS_PASS_NONE;   // of tos_xi_run / tos_batch_run
 };
 
@@ -175,12 +184,15 @@ uint32_t band_rows_for(const tos_ctx *ctx, int accum, const tos_grid &g, bool ti
 // partial rows than allowed).
 bool plan_tiles(tos_ctx *ctx, const tos_pairs *p, int accum, const tos_grid &g, const TileArgs &t, XiLaunch &L,
                 uint32_t band_rows);
-// The tile path (tos_tile.cpp): whether a job may take it, its plan
-// (tiles.state 1 when built; 2: the general path), its kernel arguments
+// The tile path (tos_tile.cpp): which of the jobs of a launch take it
+// (take[j] = 1; their plans are built), the kernel arguments of one that does
 // (false: the edge bound is too wide).
-bool tile_job(const tos_catalog *cat, const tos_pairs *p, const tos_grid &g);
-int ensure_ladder(tos_ctx *ctx, tos_catalog *cat);
-int ensure_tile_plan(tos_ctx *ctx, tos_pairs *p);
+struct TileJob {
+    tos_pairs *p;
+    const tos_grid *g;
+    int prec, accum;
+};
+int choose_tiles(tos_ctx *ctx, int n, const TileJob *jobs, char *take);
 bool tile_args(const tos_pairs *p, const tos_grid &g, TileArgs &t);
 // Workgroups of a tile pass that should have `want` of them.
 int tile_workgroups(const tos_pairs *p, const TileArgs &a, int want, int block);

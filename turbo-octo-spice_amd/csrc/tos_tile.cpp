@@ -42,8 +42,21 @@ void TilePlan::release()
     state = 0;
 }
 
-// The catalogue on its ladder, or state 2 when it has none (or no memory).
-int ensure_ladder(tos_ctx *ctx, tos_catalog *cat)
+constexpr size_t kTableBytes = (size_t)kLadderTable * 8;
+
+static LadderArgs ladder_args(const tos_catalog *cat)
+{
+    LadderArgs a{};
+    a.pix = (const float4 *)cat->pix.ptr;
+    a.los = (const LosInfo *)cat->los.ptr;
+    a.n_los = cat->n_los;
+    a.n_pix = cat->n_pix;
+    return a;
+}
+
+// Looks for the catalogue's ladder: state 3 (its steps are known) or 2 (none,
+// or no memory).
+static int survey_ladder(tos_ctx *ctx, tos_catalog *cat)
 {
     Ladder &L = cat->ladder;
     if (L.state) return TOS_OK;
@@ -51,15 +64,10 @@ int ensure_ladder(tos_ctx *ctx, tos_catalog *cat)
     if (cat->n_los == 0 || cat->n_pix == 0 || !(cat->dmin > 1e-3) || !cat->d_sorted || !cat->l_sorted) return TOS_OK;
     // the table and the state in the context's scratch: a catalogue without a
     // ladder costs no allocation
-    constexpr size_t kTableBytes = (size_t)kLadderTable * 8;
     uint32_t st[3] = {0, 0, 0};
-    if (ctx->scratch_a.reserve(kTableBytes + sizeof(st)) != TOS_OK) return TOS_OK;
+    if (ctx->scratch_a.reserve(kTableBytes + 16) != TOS_OK) return TOS_OK;
     int rc;
-    LadderArgs a{};
-    a.pix = (const float4 *)cat->pix.ptr;
-    a.los = (const LosInfo *)cat->los.ptr;
-    a.n_los = cat->n_los;
-    a.n_pix = cat->n_pix;
+    LadderArgs a = ladder_args(cat);
     a.table = (uint64_t *)ctx->scratch_a.ptr;
     a.state = (uint32_t *)((char *)ctx->scratch_a.ptr + kTableBytes);
     int e = launch_ladder_collect(a, ctx->stream);
@@ -68,16 +76,6 @@ int ensure_ladder(tos_ctx *ctx, tos_catalog *cat)
     if (st[0]) return TOS_OK;
     std::vector<uint64_t> tab(kLadderTable);
     if ((rc = copy_back(ctx, tab.data(), a.table, kTableBytes, "ladder table copy")) != TOS_OK) return rc;
-    Scratch sc;
-    DevBuf &step = sc.b[0], &nblk_of = sc.b[1];
-    if (step.reserve(kLadderTable * 2) != TOS_OK || nblk_of.reserve((size_t)cat->n_los * 4) != TOS_OK ||
-        L.place.reserve((size_t)cat->n_los * sizeof(LadderLos)) != TOS_OK) {
-        L.release();
-        return TOS_OK;
-    }
-    a.step = (const uint16_t *)step.ptr;
-    a.place = (LadderLos *)L.place.ptr;
-    a.nblk_of = (uint32_t *)nblk_of.ptr;
     // the steps in ascending distance; wavelengths must ascend with them
     struct Step {
         float d, l;
@@ -96,24 +94,61 @@ int ensure_ladder(tos_ctx *ctx, tos_catalog *cat)
     std::sort(steps.begin(), steps.end(), [](const Step &x, const Step &y) { return x.d < y.d; });
     bool ok = !steps.empty() && steps.size() <= (size_t)kMaxLadder;
     for (size_t k = 1; ok && k < steps.size(); ++k) ok = steps[k].d > steps[k - 1].d && steps[k].l > steps[k - 1].l;
-    if (!ok) {
-        L.release();
-        return TOS_OK;
-    }
+    if (!ok) return TOS_OK;
+    L.n_steps = (int)steps.size();
     L.nblk = (int)((steps.size() + kBlockSteps - 1) / kBlockSteps);
-    std::vector<uint16_t> step_of(kLadderTable, 0);
+    L.step_of.assign(kLadderTable, 0);
     L.h_d.assign((size_t)L.nblk * kBlockSteps, steps.back().d);
     L.h_l.assign((size_t)L.nblk * kBlockSteps, steps.back().l);
     for (size_t k = 0; k < steps.size(); ++k) {
-        step_of[(size_t)steps[k].slot] = (uint16_t)k;
+        L.step_of[(size_t)steps[k].slot] = (uint16_t)k;
         L.h_d[k] = steps[k].d;
         L.h_l[k] = steps[k].l;
     }
-    if ((rc = upload(ctx, step, step_of.data(), step_of.size() * 2, "ladder steps")) != TOS_OK ||
+    L.table.swap(tab);
+    // mean blocks of a sightline, from some of them
+    const int64_t every = std::max<int64_t>(1, cat->n_los / 512);
+    int64_t n = 0, blocks = 0;
+    for (int64_t k = 0; k < cat->n_los; k += every) {
+        const LosInfo &li = cat->h_los[(size_t)k];
+        if (li.n == 0) continue;
+        auto at = [&](float l) { return (std::lower_bound(L.h_l.begin(), L.h_l.begin() + L.n_steps, l) - L.h_l.begin()) / kBlockSteps; };
+        blocks += at(li.lmax) - at(li.lmin) + 1;
+        ++n;
+    }
+    L.mean_nb = n > 0 ? (double)blocks / (double)n : 0.0;
+    L.state = 3;
+    return TOS_OK;
+}
+
+// A surveyed catalogue's pixels laid out on the ladder (state 1; 2: none, or
+// no memory).
+static int build_ladder(tos_ctx *ctx, tos_catalog *cat)
+{
+    Ladder &L = cat->ladder;
+    if (L.state != 3) return TOS_OK;
+    L.state = 2;
+    constexpr size_t kStepBytes = (size_t)kLadderTable * 2;
+    uint32_t st[3] = {0, 0, 0};
+    int rc;
+    if (ctx->scratch_b.reserve(kStepBytes + (size_t)cat->n_los * 4) != TOS_OK ||
+        L.place.reserve((size_t)cat->n_los * sizeof(LadderLos)) != TOS_OK) {
+        L.release();
+        return TOS_OK;
+    }
+    L.table.resize(kLadderTable + 2, 0);   // and the state, cleared
+    if ((rc = upload(ctx, ctx->scratch_a, L.table.data(), L.table.size() * 8, "ladder table")) != TOS_OK ||
+        (rc = upload(ctx, ctx->scratch_b, L.step_of.data(), kStepBytes, "ladder steps")) != TOS_OK ||
         (rc = upload(ctx, L.d, L.h_d.data(), L.h_d.size() * 4, "ladder distances")) != TOS_OK ||
         (rc = upload(ctx, L.l, L.h_l.data(), L.h_l.size() * 4, "ladder wavelengths")) != TOS_OK)
         return rc;
-    e = launch_ladder_place(a, ctx->stream);
+    LadderArgs a = ladder_args(cat);
+    a.table = (uint64_t *)ctx->scratch_a.ptr;
+    a.state = (uint32_t *)((char *)ctx->scratch_a.ptr + kTableBytes);
+    a.step = (const uint16_t *)ctx->scratch_b.ptr;
+    a.place = (LadderLos *)L.place.ptr;
+    a.nblk_of = (uint32_t *)((char *)ctx->scratch_b.ptr + kStepBytes);
+    int e = launch_ladder_place(a, ctx->stream);
     if (e != hipSuccess) return hip_fail(ctx, (hipError_t)e, "ladder placement");
     if ((rc = copy_back(ctx, st, a.state, sizeof(st), "ladder block count")) != TOS_OK) return rc;
     if (st[0] || st[2] >= (1u << 24) ||   // 32-bit byte offsets
@@ -130,6 +165,8 @@ int ensure_ladder(tos_ctx *ctx, tos_catalog *cat)
         return TOS_OK;
     }
     L.state = 1;
+    L.table = std::vector<uint64_t>();
+    L.step_of = std::vector<uint16_t>();
     return TOS_OK;
 }
 
@@ -154,13 +191,14 @@ static void cut_equal(std::vector<int32_t> &ptr, int64_t first, int64_t n, int64
     for (int64_t k = 0; k < parts; ++k) ptr.push_back((int32_t)(first + n * k / parts));
 }
 
-int ensure_tile_plan(tos_ctx *ctx, tos_pairs *p)
+// The list's tile plan: T.state 1, or 2 (none, or no memory).
+static int ensure_tile_plan(tos_ctx *ctx, tos_pairs *p)
 {
     TilePlan &T = p->tiles;
     if (T.state) return TOS_OK;
     T.state = 2;
     tos_catalog *cat = const_cast<tos_catalog *>(p->cat);
-    int rc = ensure_ladder(ctx, cat);
+    int rc = build_ladder(ctx, cat);
     if (rc != TOS_OK) return rc;
     const Ladder &L = cat->ladder;
     if (L.state != 1 || p->n_pairs == 0) return TOS_OK;
@@ -232,15 +270,15 @@ int ensure_tile_plan(tos_ctx *ctx, tos_pairs *p)
 
 // Fewer candidate pairs than this take the general path.  Measured, general
 // / tile, us per pass on a 200 x 200 Mpc/h grid of 50 x 50 bins: 426 pairs
-// 535 / 260; 1,259 pairs 547 / 257; 9,061 pairs 770 / 383; 6.2 million pairs
-// 53,500 / 25,400.  Below, a launch is a few tiles and the plan of a first
-// pass costs what it saves.
+// 535 / 260; 1,259 pairs 547 / 257; 9,061 pairs 770 / 383.  Below, a launch is
+// a few tiles.
 constexpr int64_t kTileMinPairs = 400;
 
-bool tile_job(const tos_catalog *cat, const tos_pairs *p, const tos_grid &g)
+// Whether the tile path can do a job of the list at all.
+static bool tile_able(const tos_pairs *p, const tos_grid &g)
 {
-    if (p->n_pairs < kTileMinPairs) return false;
-    if (cat->ladder.state == 2 || p->tiles.state == 2) return false;
+    const tos_catalog *cat = p->cat;
+    if (p->n_pairs < kTileMinPairs || cat->ladder.state == 2 || p->tiles.state == 2 || !(cat->l_step > 0)) return false;
     // the edge bound needs squared separations well above their rounding
     if (!(cat->dmin > 1e-3) || cat->dmax > 1e5) return false;
     // bins far past an axis stay there: the reference's cast wraps only
@@ -252,6 +290,167 @@ bool tile_job(const tos_catalog *cat, const tos_pairs *p, const tos_grid &g)
         return cat->dmax <= 2.0 * cat->dmin && tile_edges(g) <= kTileMaxEdges && !wraps(2.0 * cat->dmax, 0) &&
                !wraps(1.0, 1);
     return true;
+}
+
+// Blocks apart that two steps inside the axis-0 window can lie (all, without
+// a window).
+static int tile_band(const tos_catalog *cat, const tos_grid &g)
+{
+    const Ladder &L = cat->ladder;
+    const std::vector<float> &key = g.type == TOS_OBSERVING ? L.h_l : L.h_d;
+    const double X = grid_window_half(g, cat->dmax, g.type == TOS_OBSERVING ? cat->lmax_abs : cat->dmax);
+    if (!(X > 0)) return L.nblk - 1;
+    int band = 0;
+    for (int b1 = 0; b1 < L.nblk; ++b1)
+        for (int b2 = b1 + band + 1; b2 < L.nblk; ++b2) {
+            if (!((double)key[(size_t)b2 * kBlockSteps] - (double)key[(size_t)b1 * kBlockSteps + kBlockSteps - 1] < X)) break;
+            band = b2 - b1;
+        }
+    return band;
+}
+
+// From this squared separation up the edges are tracked (see tile_args).
+static double tile_s_min(const tos_catalog *cat)
+{
+    const double scale = std::min(1.0, cat->dmax / 5000.0);
+    return 4.0 * scale * scale;
+}
+
+// What the passes of a launch's jobs are expected to take, in us.
+struct PassCost {
+    // general path: the longest chain of one work item, and the pairs' work
+    double gen_lat = 0, gen = 0;
+    // tile path: start, the visits' work, the longest chain of edges, of close
+    // pairs; the plan
+    double base = 140, tile = 0, edges = 0, near = 0, plan = 0;
+    double general() const { return 150 + std::hypot(gen_lat, gen); }
+    double tiles() const { return base + std::max(tile, edges) + near; }
+    void add(const PassCost &o)
+    {
+        gen_lat = std::max(gen_lat, o.gen_lat);
+        gen += o.gen;
+        base = std::max(base, o.base);
+        tile += o.tile;
+        edges = std::max(edges, o.edges);
+        near = std::max(near, o.near);
+        plan += o.plan;
+    }
+};
+
+// A visit costs the same whether its 256 pixel pairs exist or not, so sparse
+// sightlines make the tile path the slower one; bins that are narrow for the
+// pairs there are, and pairs too close to track, cost it as much; and a first
+// pass pays for the plan.  The coefficients are a fit to 594 measured forms:
+// 40 to 12,000 sightlines; 2 to 95 % of the pixels masked, sightlines cut to 3,
+// 12 and 40 pixels or thinned 8 and 25 times; all grids, windows of 2 to 200
+// Mpc/h, 50 to 4000 axis-1 bins; both precisions, two and seven sums.  Of
+// the forms that the tile path makes slower by a tenth or more (780 pairs with
+// 4000 bins 1.4 / 9.4 ms, 144,000 pairs thinned 25 times 0.67 / 0.78, 4,700
+// pairs within 2 Mpc/h 0.58 / 0.87) the rule takes none.  Before the ladder is
+// surveyed its size is that of the sampled spectra.
+static PassCost pass_cost(const tos_ctx *ctx, const tos_pairs *p, const tos_grid &g, int prec, int accum)
+{
+    const tos_catalog *cat = p->cat;
+    const Ladder &L = cat->ladder;
+    const bool all = accum == TOS_ACC_ALL, polar = g.type == TOS_POLAR, obs = g.type == TOS_OBSERVING;
+    const double P = (double)p->n_pairs, N = (double)p->h.stats.num_pixel_pairs;
+    GridExact ge;
+    grid_exact_consts(g, ge);
+    const bool fixed = tile_fixed((int)ge.nslots);
+    // the ladder's blocks, those of a sightline, the axis-0 band, and the share
+    // of a pair's pixel pairs inside the axis-0 window
+    const double X = grid_window_half(g, cat->dmax, obs ? cat->lmax_abs : cat->dmax);
+    const double key_range = obs ? cat->l_range : cat->dmax - cat->dmin;
+    const double steps = L.state ? (double)L.n_steps : cat->l_range / cat->l_step + 1.0;
+    const double nblk = std::ceil(steps / kBlockSteps);
+    const double nb = L.state ? L.mean_nb : std::min(nblk, cat->l_span / (cat->l_step * kBlockSteps) + 1.0);
+    const double block = std::max(1e-300, key_range / std::max(1.0, nblk));
+    const double band = X > 0 ? std::min(nblk - 1.0, std::floor(X / block) + 1.0) : nblk - 1.0;
+    const double w = X > 0 ? std::min(1.0, 2.0 * X / (nb * block)) : 1.0;
+    PassCost c;
+    // general path; beyond the fixed layout LDS holds fewer wavefronts, and
+    // too large a grid takes a pass for each band
+    double f = all ? 3.5 : prec == TOS_FP64 ? 1.6 : 1.0;
+    if (g.type != TOS_CARTESIAN) f *= 1.15;
+    const uint32_t rows = std::max(1u, band_rows_for(ctx, accum, g));
+    const double bands = (double)((ge.n[0] + rows - 1) / rows);
+    const double Nw = N * (0.3 + 0.7 * w);
+    const double partners = P / (double)std::max<int64_t>(1, p->n_rows), pix = std::sqrt(N / P);
+    const double item = std::max(pix * std::sqrt(partners), partners * std::min(4.8, 0.25 * pix));
+    c.gen_lat = (all ? 2.0 : f) * (fixed ? 1.0 : 1.6 * bands) * std::min(380.0, item) * (0.2 + 0.75 * w);
+    c.gen = f * bands * (fixed ? 1.0 : prec == TOS_FP64 ? 1.9 : 3.5) * (2e-3 * P + std::min(2e-6 * Nw, 3000.0 + 3e-7 * Nw));
+    // tile path
+    if (polar) c.base = 245;
+    if (p->tiles.state == 0) c.plan = 240 + 11e-3 * std::min(P, 16384.0) + 0.6e-3 * P;
+    const double all_visits = p->tiles.state == 1 ? (double)p->tiles.total : P * nb * nb;
+    const double visits = std::max(1.0, all_visits * std::min(1.0, (2.0 * band + 1.0) / std::max(1.0, nb)));
+    const double tiles = nblk * (2.0 * band + 1.0), bins = polar ? (double)tile_edges(g) : (double)ge.n[1];
+    const double batch = (double)std::min<int64_t>(batch_pairs(p->n_pairs), p->n_pairs), batches = P / batch;
+    // edges a cell passes per visit: each group of pairs takes a tile's cells
+    // through all bins
+    const double e = bins * tiles * std::ceil(P / kMaxGroup) / visits;
+    c.tile = 0.8e-3 * P + visits * 1e-3 * (0.02 + 0.7 * std::max(std::sqrt(e), 2.0 * e)) * (all ? 2.5 : fixed ? 1.0 : P < 3e5 ? 1.25 : 2.7);
+    if (obs) return c;
+    c.edges = std::max(0.0, (polar ? 9.0 : 5.0) * (bins / std::sqrt(batches) - 30.0));
+    // pairs too close to track, in one batch or a few
+    const double reach = std::max(p->max_ang, 1e-9);
+    const double close = std::min(1.0, tile_s_min(cat) / (cat->dmin * cat->dmin * reach * reach));
+    const double cover = std::min(1.0, nb / nblk);
+    c.near = (polar ? 25.0 : 17.0) * std::min(close * P, batch) * cover * cover + 0.75e-3 * close * visits;
+    return c;
+}
+
+// The plan must pay for itself on this pass, or have paid on the passes that
+// went without it: a list that is used again and again gets one at last.
+static bool tiles_pay(const PassCost &c, int32_t passes_before)
+{
+    return (c.general() - c.tiles()) * (passes_before + 1.0) >= c.plan;
+}
+
+int choose_tiles(tos_ctx *ctx, int n, const TileJob *jobs, char *take)
+{
+    int rc;
+    std::vector<PassCost> cost((size_t)n);
+    auto price = [&](int j) { cost[(size_t)j] = pass_cost(ctx, jobs[j].p, *jobs[j].g, jobs[j].prec, jobs[j].accum); };
+    auto pays = [&] {
+        PassCost c;
+        int32_t before = INT32_MAX;
+        for (int j = 0; j < n; ++j) {
+            if (!take[j]) continue;
+            c.add(cost[(size_t)j]);
+            if (jobs[j].p->tiles.state == 0) before = std::min(before, jobs[j].p->passes_before_plan);
+        }
+        return tiles_pay(c, before);
+    };
+    bool any = false;
+    for (int j = 0; j < n; ++j) {
+        if (!(take[j] = tile_able(jobs[j].p, *jobs[j].g))) continue;
+        any = true;
+        price(j);
+    }
+    if (!any) return TOS_OK;
+    bool pay = pays();
+    if (pay) {
+        for (int j = 0; j < n; ++j) {
+            if (!take[j]) continue;
+            const int known = jobs[j].p->cat->ladder.state;
+            if ((rc = survey_ladder(ctx, const_cast<tos_catalog *>(jobs[j].p->cat))) != TOS_OK) return rc;
+            if (!(take[j] = jobs[j].p->cat->ladder.state != 2)) continue;
+            if (known == 0) price(j);
+            take[j] = cost[(size_t)j].tiles() < cost[(size_t)j].general();
+        }
+        pay = pays();
+    }
+    for (int j = 0; j < n; ++j) {
+        if (!take[j]) continue;
+        if (!pay) {
+            if (jobs[j].p->passes_before_plan < 1000) ++jobs[j].p->passes_before_plan;
+        } else if ((rc = ensure_tile_plan(ctx, jobs[j].p)) != TOS_OK) {
+            return rc;
+        }
+        take[j] = pay && jobs[j].p->tiles.state == 1;
+    }
+    return TOS_OK;
 }
 
 bool tile_args(const tos_pairs *p, const tos_grid &g, TileArgs &t)
@@ -272,19 +471,7 @@ bool tile_args(const tos_pairs *p, const tos_grid &g, TileArgs &t)
     t.n_batches = T.n_batches;
     t.width0 = g.width[0];
     t.width1 = g.width[1];
-    // tiles whose steps all differ by less than the axis-0 window
-    const std::vector<float> &key = g.type == TOS_OBSERVING ? L.h_l : L.h_d;
-    const double X = grid_window_half(g, cat->dmax, g.type == TOS_OBSERVING ? cat->lmax_abs : cat->dmax);
-    int band = L.nblk - 1;
-    if (X > 0) {
-        band = 0;
-        for (int b1 = 0; b1 < L.nblk; ++b1)
-            for (int b2 = b1 + band + 1; b2 < L.nblk; ++b2) {
-                if (!((double)key[(size_t)b2 * kBlockSteps] - (double)key[(size_t)b1 * kBlockSteps + kBlockSteps - 1] < X)) break;
-                band = b2 - b1;
-            }
-    }
-    t.band = band;
+    t.band = tile_band(cat, g);
     // K of an edge at squared separation s >= s_min is known within a relative
     //   2^-24 (f32 K) + 3 2^-24 (f32 threshold: the squared edge, 1 / (d1 d2)
     //   and their product)
@@ -298,8 +485,7 @@ bool tile_args(const tos_pairs *p, const tos_grid &g, TileArgs &t)
     // takes the reference arithmetic there (400,000 sightline pairs 29 ms, the
     // general kernel 23, this 1.9).
     const double u = std::ldexp(1.0, -24);
-    const double scale = std::min(1.0, cat->dmax / 5000.0);
-    t.s_min = 4.0 * scale * scale;
+    t.s_min = tile_s_min(cat);
     double base = 2.0 * u * cat->dmax * cat->dmax + 4.0 * u * cat->dmax * std::fabs(g.max[0]);
     double ops = 4.0, abs_err = 7e-15 * cat->dmax * cat->dmax;
     if (g.type == TOS_POLAR) {

@@ -354,14 +354,16 @@ extern "C" int tos_xi_run(tos_ctx *ctx, const tos_catalog *cat, const tos_pairs 
 
     const int flags = opts ? opts->flags : 0;
     int rc;
-    // the tile path: catalogues on a ladder, no work scheme switched off and
-    // no launch shape asked for
+    // the tile path: catalogues on a ladder where it pays, no work scheme
+    // switched off and no launch shape asked for
     bool tiles = flags == 0 && (!opts || (opts->block_size == 0 && opts->blocks_per_cu == 0 && opts->wg_per_slot == 0)) &&
-                 tile_job(cat, p, g);
+                 p->n_pairs > 0;
     TileArgs t;
     if (tiles) {
-        if ((rc = ensure_tile_plan(ctx, p)) != TOS_OK) return rc;
-        tiles = p->tiles.state == 1;
+        const TileJob job{p, &g, prec, accum};
+        char take = 0;
+        if ((rc = choose_tiles(ctx, 1, &job, &take)) != TOS_OK) return rc;
+        tiles = take != 0;
     }
     // the work items in either case: tos_xi_run_noalloc takes them up on any
     // grid
