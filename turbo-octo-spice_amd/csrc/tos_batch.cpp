@@ -608,31 +608,12 @@ int xi_run_per_skybin(tos_ctx *ctx, const tos_catalog *cat, tos_pairs *p, const 
 
 }  // namespace tos
 
-extern "C" int tos_batch_run(tos_ctx *ctx, int32_t n, const tos_batch_job *jobs, int use_graph, tos_xi_result *out,
-                             double *batch_ms)
+namespace tos {
+
+// tos_batch_run, checked arguments; may_tile: the tile path is open.
+static int run_batch(tos_ctx *ctx, int32_t n, const tos_batch_job *jobs, int use_graph, bool may_tile,
+                     tos_xi_result *out, double *batch_ms)
 {
-    if (!ctx || n < 0 || (n > 0 && (!jobs || !out))) return TOS_ERR_INVALID;
-    if (n == 0) {
-        if (batch_ms) *batch_ms = 0;
-        return TOS_OK;
-    }
-    for (int32_t j = 0; j < n; ++j) {
-        const tos_batch_job &J = jobs[j];
-        if (!J.cat || !J.pairs || J.pairs->cat != J.cat) {
-            set_err(ctx, "tos_batch_run: job " + std::to_string(j) + " has no catalogue or a pair list of another");
-            return TOS_ERR_INVALID;
-        }
-        if (!grid_ok(ctx, &J.grid)) return TOS_ERR_INVALID;
-        if ((J.precision != TOS_FP64 && J.precision != TOS_FP32C) || J.accum != TOS_ACC_CORE) {
-            set_err(ctx, "tos_batch_run: jobs take TOS_FP64 or TOS_FP32C with TOS_ACC_CORE");
-            return TOS_ERR_INVALID;
-        }
-        if (!out[j].num_pairs || !out[j].didj || !out[j].wgt) {
-            set_err(ctx, "tos_batch_run: result arrays missing for job " + std::to_string(j));
-            return TOS_ERR_INVALID;
-        }
-    }
-    hipSetDevice(ctx->device);
     int rc;
     for (int32_t j = 0; j < n; ++j) {
         tos_pairs *p = const_cast<tos_pairs *>(jobs[j].pairs);
@@ -645,7 +626,7 @@ extern "C" int tos_batch_run(tos_ctx *ctx, int32_t n, const tos_batch_job *jobs,
     std::vector<char> tiles((size_t)n, 0);
     for (int32_t j = 0; j < n; ++j)
         tj.push_back(TileJob{const_cast<tos_pairs *>(jobs[j].pairs), &jobs[j].grid, jobs[j].precision, TOS_ACC_CORE});
-    if ((rc = choose_tiles(ctx, n, tj.data(), tiles.data())) != TOS_OK) return rc;
+    if (may_tile && (rc = choose_tiles(ctx, n, tj.data(), tiles.data())) != TOS_OK) return rc;
     if (!ctx->batch) {
         ctx->batch = new BatchState();
         if (hipEventCreate(&ctx->batch->ev0) != hipSuccess || hipEventCreate(&ctx->batch->ev1) != hipSuccess) {
@@ -703,6 +684,42 @@ extern "C" int tos_batch_run(tos_ctx *ctx, int32_t n, const tos_batch_job *jobs,
             const_cast<tos_pairs *>(jobs[j].pairs)->last_pass =
                 jobs[j].pairs->n_items == 0 ? TOS_PASS_NONE : G.key.tile ? TOS_PASS_LADDER : TOS_PASS_GENERAL;
     return TOS_OK;
+}
+
+}  // namespace tos
+
+extern "C" int tos_batch_run(tos_ctx *ctx, int32_t n, const tos_batch_job *jobs, int use_graph, tos_xi_result *out,
+                             double *batch_ms)
+{
+    if (!ctx || n < 0 || (n > 0 && (!jobs || !out))) return TOS_ERR_INVALID;
+    if (n == 0) {
+        if (batch_ms) *batch_ms = 0;
+        return TOS_OK;
+    }
+    for (int32_t j = 0; j < n; ++j) {
+        const tos_batch_job &J = jobs[j];
+        if (!J.cat || !J.pairs || J.pairs->cat != J.cat) {
+            set_err(ctx, "tos_batch_run: job " + std::to_string(j) + " has no catalogue or a pair list of another");
+            return TOS_ERR_INVALID;
+        }
+        if (!grid_ok(ctx, &J.grid)) return TOS_ERR_INVALID;
+        if ((J.precision != TOS_FP64 && J.precision != TOS_FP32C) || J.accum != TOS_ACC_CORE) {
+            set_err(ctx, "tos_batch_run: jobs take TOS_FP64 or TOS_FP32C with TOS_ACC_CORE");
+            return TOS_ERR_INVALID;
+        }
+        if (!out[j].num_pairs || !out[j].didj || !out[j].wgt) {
+            set_err(ctx, "tos_batch_run: result arrays missing for job " + std::to_string(j));
+            return TOS_ERR_INVALID;
+        }
+    }
+    hipSetDevice(ctx->device);
+    // without memory for the batch beside its lists' tile plans, the general
+    // path
+    int rc = run_batch(ctx, n, jobs, use_graph, true, out, batch_ms);
+    if (rc != TOS_ERR_NOMEM) return rc;
+    bool dropped = false;
+    for (int32_t j = 0; j < n; ++j) dropped |= drop_tiles(ctx, const_cast<tos_pairs *>(jobs[j].pairs));
+    return dropped ? run_batch(ctx, n, jobs, use_graph, false, out, batch_ms) : rc;
 }
 
 extern "C" int tos_xi_autotune(tos_ctx *ctx, const tos_catalog *cat, const tos_pairs *pairs, const tos_grid *grid,

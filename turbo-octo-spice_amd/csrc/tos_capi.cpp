@@ -41,6 +41,7 @@ int DevBuf::reserve(size_t n)
     if (n == 0) return TOS_OK;
     if (hipMalloc(&ptr, n) != hipSuccess) {
         ptr = nullptr;
+        (void)hipGetLastError();   // not the next launch's
         return TOS_ERR_NOMEM;
     }
     bytes = n;

@@ -193,6 +193,9 @@ struct TileJob {
     int prec, accum;
 };
 int choose_tiles(tos_ctx *ctx, int n, const TileJob *jobs, char *take);
+// Gives the plan's and the ladder's memory back for good (a later allocation
+// has failed); false: there was none.
+bool drop_tiles(tos_ctx *ctx, tos_pairs *p);
 bool tile_args(const tos_pairs *p, const tos_grid &g, TileArgs &t);
 // Workgroups of a tile pass that should have `want` of them.
 int tile_workgroups(const tos_pairs *p, const TileArgs &a, int want, int block);

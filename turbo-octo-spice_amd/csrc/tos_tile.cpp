@@ -121,27 +121,34 @@ static int survey_ladder(tos_ctx *ctx, tos_catalog *cat)
     return TOS_OK;
 }
 
+// What a step of building a ladder or a plan left undone: its memory is given
+// back, and a lack of memory is no error, the job takes the general path.
+template <typename T>
+static int give_up(T &built, int rc)
+{
+    built.release();
+    built.state = 2;
+    return rc == TOS_ERR_NOMEM ? TOS_OK : rc;
+}
+
 // A surveyed catalogue's pixels laid out on the ladder (state 1; 2: none, or
 // no memory).
 static int build_ladder(tos_ctx *ctx, tos_catalog *cat)
 {
     Ladder &L = cat->ladder;
     if (L.state != 3) return TOS_OK;
-    L.state = 2;
     constexpr size_t kStepBytes = (size_t)kLadderTable * 2;
     uint32_t st[3] = {0, 0, 0};
     int rc;
     if (ctx->scratch_b.reserve(kStepBytes + (size_t)cat->n_los * 4) != TOS_OK ||
-        L.place.reserve((size_t)cat->n_los * sizeof(LadderLos)) != TOS_OK) {
-        L.release();
-        return TOS_OK;
-    }
+        L.place.reserve((size_t)cat->n_los * sizeof(LadderLos)) != TOS_OK)
+        return give_up(L, TOS_ERR_NOMEM);
     L.table.resize(kLadderTable + 2, 0);   // and the state, cleared
     if ((rc = upload(ctx, ctx->scratch_a, L.table.data(), L.table.size() * 8, "ladder table")) != TOS_OK ||
         (rc = upload(ctx, ctx->scratch_b, L.step_of.data(), kStepBytes, "ladder steps")) != TOS_OK ||
         (rc = upload(ctx, L.d, L.h_d.data(), L.h_d.size() * 4, "ladder distances")) != TOS_OK ||
         (rc = upload(ctx, L.l, L.h_l.data(), L.h_l.size() * 4, "ladder wavelengths")) != TOS_OK)
-        return rc;
+        return give_up(L, rc);
     LadderArgs a = ladder_args(cat);
     a.table = (uint64_t *)ctx->scratch_a.ptr;
     a.state = (uint32_t *)((char *)ctx->scratch_a.ptr + kTableBytes);
@@ -149,21 +156,16 @@ static int build_ladder(tos_ctx *ctx, tos_catalog *cat)
     a.place = (LadderLos *)L.place.ptr;
     a.nblk_of = (uint32_t *)((char *)ctx->scratch_b.ptr + kStepBytes);
     int e = launch_ladder_place(a, ctx->stream);
-    if (e != hipSuccess) return hip_fail(ctx, (hipError_t)e, "ladder placement");
-    if ((rc = copy_back(ctx, st, a.state, sizeof(st), "ladder block count")) != TOS_OK) return rc;
+    if (e != hipSuccess) return give_up(L, hip_fail(ctx, (hipError_t)e, "ladder placement"));
+    if ((rc = copy_back(ctx, st, a.state, sizeof(st), "ladder block count")) != TOS_OK) return give_up(L, rc);
     if (st[0] || st[2] >= (1u << 24) ||   // 32-bit byte offsets
-        L.pix.reserve((size_t)st[2] * kBlockBytes) != TOS_OK) {
-        L.release();
-        return TOS_OK;
-    }
+        L.pix.reserve((size_t)st[2] * kBlockBytes) != TOS_OK)
+        return give_up(L, TOS_ERR_NOMEM);
     a.out = (float *)L.pix.ptr;
     e = launch_ladder_fill(a, st[2], ctx->stream);
-    if (e != hipSuccess) return hip_fail(ctx, (hipError_t)e, "ladder fill");
-    if ((rc = copy_back(ctx, st, a.state, sizeof(st), "ladder state copy")) != TOS_OK) return rc;
-    if (st[0]) {
-        L.release();
-        return TOS_OK;
-    }
+    if (e != hipSuccess) return give_up(L, hip_fail(ctx, (hipError_t)e, "ladder fill"));
+    if ((rc = copy_back(ctx, st, a.state, sizeof(st), "ladder state copy")) != TOS_OK) return give_up(L, rc);
+    if (st[0]) return give_up(L, TOS_OK);
     L.state = 1;
     L.table = std::vector<uint64_t>();
     L.step_of = std::vector<uint16_t>();
@@ -219,20 +221,17 @@ static int ensure_tile_plan(tos_ctx *ctx, tos_pairs *p)
     DevBuf &rlos = sc.b[0], &rptr = sc.b[1], &state = sc.b[2], &cover = sc.b[3], &keys = sc.b[4], &groups = sc.b[5], &keys2 = sc.b[6];
     T.words = (int)((q + 63) / 64);
     const size_t np = (size_t)p->n_pairs, rows = (size_t)T.n_batches * L.nblk;
-    if (cover.reserve(np * 4) != TOS_OK || T.masks.reserve(rows * 2 * T.words * 8) != TOS_OK || T.rec.reserve(np * 16) != TOS_OK ||
-        T.visits.reserve(rows * L.nblk * 4) != TOS_OK ||
-        state.reserve(16) != TOS_OK || (max_group > kSortRun && (keys.reserve(np * 8) != TOS_OK || keys2.reserve(np * 8) != TOS_OK))) {
-        T.release();
-        T.state = 2;
-        return TOS_OK;
-    }
+    if (cover.reserve(np * 4) != TOS_OK || T.masks.reserve(rows * 2 * T.words * 8) != TOS_OK ||
+        T.rec.reserve(np * 16) != TOS_OK || T.visits.reserve(rows * L.nblk * 4) != TOS_OK ||
+        (max_group > kSortRun && (keys.reserve(np * 8) != TOS_OK || keys2.reserve(np * 8) != TOS_OK)))
+        return give_up(T, TOS_ERR_NOMEM);
     uint64_t st[2] = {0, 0};
     if ((rc = upload(ctx, T.batch_ptr, bp.data(), bp.size() * 4, "tile batches")) != TOS_OK ||
         (rc = upload(ctx, groups, gp.data(), gp.size() * 4, "tile groups")) != TOS_OK ||
         (rc = upload(ctx, rlos, p->h.row_los.data(), p->h.row_los.size() * 4, "tile rows")) != TOS_OK ||
         (rc = upload(ctx, rptr, p->h.row_ptr.data(), p->h.row_ptr.size() * 8, "tile row offsets")) != TOS_OK ||
         (rc = upload(ctx, state, st, sizeof(st), "tile state")) != TOS_OK)
-        return rc;
+        return give_up(T, rc);
     TilePlanArgs a{};
     a.row_los = (const int32_t *)rlos.ptr;
     a.row_ptr = (const int64_t *)rptr.ptr;
@@ -256,13 +255,9 @@ static int ensure_tile_plan(tos_ctx *ctx, tos_pairs *p)
     a.visits = (uint32_t *)T.visits.ptr;
     a.state = (unsigned long long *)state.ptr;
     const int e = launch_tile_plan(a, ctx->stream);
-    if (e != hipSuccess) return hip_fail(ctx, (hipError_t)e, "tile plan");
-    if ((rc = copy_back(ctx, st, state.ptr, sizeof(st), "tile state copy")) != TOS_OK) return rc;
-    if (st[0]) {
-        T.release();
-        T.state = 2;
-        return TOS_OK;
-    }
+    if (e != hipSuccess) return give_up(T, hip_fail(ctx, (hipError_t)e, "tile plan"));
+    if ((rc = copy_back(ctx, st, state.ptr, sizeof(st), "tile state copy")) != TOS_OK) return give_up(T, rc);
+    if (st[0]) return give_up(T, TOS_OK);
     T.total = st[1];
     T.state = 1;
     return TOS_OK;
@@ -451,6 +446,16 @@ int choose_tiles(tos_ctx *ctx, int n, const TileJob *jobs, char *take)
         take[j] = pay && jobs[j].p->tiles.state == 1;
     }
     return TOS_OK;
+}
+
+bool drop_tiles(tos_ctx *ctx, tos_pairs *p)
+{
+    Ladder &L = const_cast<tos_catalog *>(p->cat)->ladder;
+    if (p->tiles.state != 1 && L.state != 1) return false;
+    (void)hipStreamSynchronize(ctx->stream);
+    (void)give_up(p->tiles, TOS_OK);
+    (void)give_up(L, TOS_OK);   // other lists of the catalogue: see tile_able
+    return true;
 }
 
 bool tile_args(const tos_pairs *p, const tos_grid &g, TileArgs &t)

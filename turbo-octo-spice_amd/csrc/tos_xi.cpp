@@ -311,41 +311,10 @@ void fill_args(const tos_catalog *cat, const tos_pairs *p, const tos_grid &g, bo
     }
 }
 
-}  // namespace tos
-
-extern "C" int tos_xi_run(tos_ctx *ctx, const tos_catalog *cat, const tos_pairs *pairs_c, const tos_grid *grid,
-                          const tos_xi_opts *opts, tos_xi_result *out)
+// One pass of tos_xi_run, checked arguments; may_tile: the tile path is open.
+static int run_pass(tos_ctx *ctx, const tos_catalog *cat, tos_pairs *p, const tos_grid &g, const tos_xi_opts *opts,
+                    int prec, int accum, bool may_tile, tos_xi_result *out)
 {
-    if (!ctx || !cat || !pairs_c || !out) return TOS_ERR_INVALID;
-    if (!grid_ok(ctx, grid)) return TOS_ERR_INVALID;
-    tos_pairs *p = const_cast<tos_pairs *>(pairs_c);
-    if (p->cat != cat) {
-        set_err(ctx, "tos_xi_run: the pair list was built for another catalogue");
-        return TOS_ERR_INVALID;
-    }
-    const int prec = opts ? opts->precision : TOS_FP64;
-    const int accum = opts ? opts->accum : TOS_ACC_CORE;
-    if ((prec != TOS_FP64 && prec != TOS_FP32C) || (accum != TOS_ACC_CORE && accum != TOS_ACC_ALL)) {
-        set_err(ctx, "tos_xi_run: unknown precision or accumulator set");
-        return TOS_ERR_INVALID;
-    }
-    if (opts && opts->per_skybin) {
-        const bool subs = p->h.stats.n_skybins > 0;
-        if (accum != TOS_ACC_CORE || !out->num_pairs || !out->didj || !out->wgt ||
-            (subs && (!out->skybin_keys || !out->sub_num_pairs || !out->sub_didj || !out->sub_wgt))) {
-            set_err(ctx, "tos_xi_run: per-sky-bin subsamples take TOS_ACC_CORE and every subsample array");
-            return TOS_ERR_INVALID;
-        }
-        hipSetDevice(ctx->device);
-        return xi_run_per_skybin(ctx, cat, p, *grid, prec, opts->flags, out);
-    }
-    if (!out->num_pairs || !out->didj || !out->wgt ||
-        (accum == TOS_ACC_ALL && (!out->di || !out->dj || !out->wi || !out->wj || !out->z))) {
-        set_err(ctx, "tos_xi_run: result arrays missing");
-        return TOS_ERR_INVALID;
-    }
-    hipSetDevice(ctx->device);
-    const tos_grid g = *grid;
     const int nbins = g.nbins[0] * g.nbins[1] * g.nbins[2];
     out->num_pixel_pairs_used = 0;
     out->num_guard_rechecks = 0;
@@ -356,7 +325,7 @@ extern "C" int tos_xi_run(tos_ctx *ctx, const tos_catalog *cat, const tos_pairs 
     int rc;
     // the tile path: catalogues on a ladder where it pays, no work scheme
     // switched off and no launch shape asked for
-    bool tiles = flags == 0 && (!opts || (opts->block_size == 0 && opts->blocks_per_cu == 0 && opts->wg_per_slot == 0)) &&
+    bool tiles = may_tile && flags == 0 && (!opts || (opts->block_size == 0 && opts->blocks_per_cu == 0 && opts->wg_per_slot == 0)) &&
                  p->n_pairs > 0;
     TileArgs t;
     if (tiles) {
@@ -484,4 +453,44 @@ extern "C" int tos_xi_run(tos_ctx *ctx, const tos_catalog *cat, const tos_pairs 
     return TOS_OK;
 }
 
+}  // namespace tos
 
+extern "C" int tos_xi_run(tos_ctx *ctx, const tos_catalog *cat, const tos_pairs *pairs_c, const tos_grid *grid,
+                          const tos_xi_opts *opts, tos_xi_result *out)
+{
+    if (!ctx || !cat || !pairs_c || !out) return TOS_ERR_INVALID;
+    if (!grid_ok(ctx, grid)) return TOS_ERR_INVALID;
+    tos_pairs *p = const_cast<tos_pairs *>(pairs_c);
+    if (p->cat != cat) {
+        set_err(ctx, "tos_xi_run: the pair list was built for another catalogue");
+        return TOS_ERR_INVALID;
+    }
+    const int prec = opts ? opts->precision : TOS_FP64;
+    const int accum = opts ? opts->accum : TOS_ACC_CORE;
+    if ((prec != TOS_FP64 && prec != TOS_FP32C) || (accum != TOS_ACC_CORE && accum != TOS_ACC_ALL)) {
+        set_err(ctx, "tos_xi_run: unknown precision or accumulator set");
+        return TOS_ERR_INVALID;
+    }
+    if (opts && opts->per_skybin) {
+        const bool subs = p->h.stats.n_skybins > 0;
+        if (accum != TOS_ACC_CORE || !out->num_pairs || !out->didj || !out->wgt ||
+            (subs && (!out->skybin_keys || !out->sub_num_pairs || !out->sub_didj || !out->sub_wgt))) {
+            set_err(ctx, "tos_xi_run: per-sky-bin subsamples take TOS_ACC_CORE and every subsample array");
+            return TOS_ERR_INVALID;
+        }
+        hipSetDevice(ctx->device);
+        int rc = xi_run_per_skybin(ctx, cat, p, *grid, prec, opts->flags, out);
+        if (rc == TOS_ERR_NOMEM && drop_tiles(ctx, p)) rc = xi_run_per_skybin(ctx, cat, p, *grid, prec, opts->flags, out);
+        return rc;
+    }
+    if (!out->num_pairs || !out->didj || !out->wgt ||
+        (accum == TOS_ACC_ALL && (!out->di || !out->dj || !out->wi || !out->wj || !out->z))) {
+        set_err(ctx, "tos_xi_run: result arrays missing");
+        return TOS_ERR_INVALID;
+    }
+    hipSetDevice(ctx->device);
+    // without memory for the pass beside the list's tile plan, the general path
+    int rc = run_pass(ctx, cat, p, *grid, opts, prec, accum, true, out);
+    if (rc == TOS_ERR_NOMEM && drop_tiles(ctx, p)) rc = run_pass(ctx, cat, p, *grid, opts, prec, accum, false, out);
+    return rc;
+}
