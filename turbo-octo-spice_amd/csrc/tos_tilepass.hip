@@ -76,6 +76,16 @@ __device__ __forceinline__ const TOS_GLOBAL T *global(const void *p)
     return (const TOS_GLOBAL T *)p;
 }
 
+// Orders a wavefront's LDS accesses before and after it, for its queue, which
+// other lanes read than wrote it.  LDS serves a wavefront's accesses in order,
+// so this holds the compiler only.
+__device__ __forceinline__ void wave_lds_fence()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // The workgroup's control words, after its histogram in LDS.
 struct TileCtl {
     unsigned long long recheck;
@@ -552,12 +562,14 @@ __device__ __forceinline__ void tile_block(const XiKernelArgs &a, const TileArgs
                 fill += __popcll(mb);
             }
             if (fill == 0) break;
+            wave_lds_fence();
             int n = kRun;
             if (fill < kRun) {
                 // padding entries read the zero block and repeat the last K
                 n = (fill + 3) & ~3;
                 const uint4 last = queue[fill - 1];
                 if (lane < n - fill) queue[fill + lane] = make_uint4(0u, 0u, last.z, last.w);
+                wave_lds_fence();
             }
             // four entries at a time; each operand register is loaded for the
             // entry four ahead as soon as its visit is done
@@ -594,8 +606,10 @@ __device__ __forceinline__ void tile_block(const XiKernelArgs &a, const TileArgs
                 }
             }
             const int rest = fill > kRun ? fill - kRun : 0;   // at most kChunk
+            wave_lds_fence();          // the visits' reads
             if (rest > 0) {
                 const uint4 x = queue[kRun + lane], y = queue[kRun + (kWave + lane < kChunk ? kWave + lane : lane)];
+                wave_lds_fence();
                 queue[lane] = x;
                 queue[kWave + lane] = y;
             }
