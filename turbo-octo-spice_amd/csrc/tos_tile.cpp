@@ -273,6 +273,8 @@ constexpr int64_t kTileMinPairs = 400;
 static bool tile_able(const tos_pairs *p, const tos_grid &g)
 {
     const tos_catalog *cat = p->cat;
+    // the plan's kernels step past a group's last pair in 32 bits
+    if (p->n_pairs > INT32_MAX - kMaxGroup) return false;
     if (p->n_pairs < kTileMinPairs || cat->ladder.state == 2 || p->tiles.state == 2 || !(cat->l_step > 0)) return false;
     // the edge bound needs squared separations well above their rounding
     if (!(cat->dmin > 1e-3) || cat->dmax > 1e5) return false;
