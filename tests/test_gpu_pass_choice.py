@@ -58,7 +58,8 @@ def test_batches_and_sky_bins(dev, lists):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("change", ["off_ladder", "two_wavelengths", "descending", "overflow", "few_pairs", "shape"])
+@pytest.mark.parametrize("change", ["off_ladder", "two_wavelengths", "descending", "overflow", "few_pairs", "shape",
+                                    "both_signs"])
 def test_passes_without_a_ladder(dev, lists, change):
     cat = lists[0]
     kw = {k: getattr(cat, k).copy() for k in ("value", "loglam", "weight", "distance")}
@@ -70,6 +71,8 @@ def test_passes_without_a_ladder(dev, lists, change):
     elif change == "descending":
         for k in ("distance", "loglam"):
             kw[k][a:b] = kw[k][a:b][::-1]
+    elif change == "both_signs":    # half of the ladder behind the origin
+        kw["distance"] -= np.float32(np.median(kw["distance"])) + np.float32(0.37)
     elif change == "overflow":
         kw["weight"][n // 3] = kw["value"][n // 3] = 1e30
     c = synth.Catalog(cat.ra, cat.dec, cat.offsets, kw["value"], kw["loglam"], kw["weight"], kw["distance"], cat.zq,

@@ -92,7 +92,8 @@ static int survey_ladder(tos_ctx *ctx, tos_catalog *cat)
         steps.push_back(s);
     }
     std::sort(steps.begin(), steps.end(), [](const Step &x, const Step &y) { return x.d < y.d; });
-    bool ok = !steps.empty() && steps.size() <= (size_t)kMaxLadder;
+    // (K of an edge is formed with 1 / (d1 d2), which must not change sign)
+    bool ok = !steps.empty() && steps.size() <= (size_t)kMaxLadder && steps[0].d > 0.0f;
     for (size_t k = 1; ok && k < steps.size(); ++k) ok = steps[k].d > steps[k - 1].d && steps[k].l > steps[k - 1].l;
     if (!ok) return TOS_OK;
     L.n_steps = (int)steps.size();
