@@ -112,6 +112,8 @@ typedef struct {
 
 int tos_catalog_upload(tos_ctx *ctx, const tos_sightlines *s, tos_catalog **out);
 int tos_catalog_free(tos_ctx *ctx, tos_catalog *cat);
+/* device_bytes: held now; a first pass may add the pixels on their wavelength
+ * ladder. */
 int tos_catalog_info(const tos_catalog *cat, int64_t *n_los, int64_t *n_pix,
                      int64_t *device_bytes);
 

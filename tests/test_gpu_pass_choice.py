@@ -202,3 +202,24 @@ def test_batches_choose_as_a_whole(dev):
     for dcat, p in made:
         p.free()
         dcat.free()
+
+
+@pytest.mark.gpu
+def test_catalogue_bytes_count_the_ladder(dev):
+    cat = synth.lya_catalog(500, area_deg2=40.0, seed=3)
+    grid = GridSpec.cartesian()
+    dcat = dev.upload(cat)
+    pairs = dcat.pairs(grid.max_angular_scale(cat.scale), order=3, nthreads=8)
+
+    def held():
+        n = ctypes.c_int64(0)
+        assert _lib.lib().tos_catalog_info(dcat.h, None, None, ctypes.byref(n)) == 0
+        return n.value
+
+    before = held()
+    pairs.run(grid, precision=tos_amd.FP32C)
+    assert pairs.last_pass() == tos_amd.PASS_LADDER
+    # three floats a step of a block, and a place for each sightline
+    assert held() >= before + 12 * cat.n_pix + 8 * cat.n_los
+    pairs.free()
+    dcat.free()

@@ -456,7 +456,13 @@ extern "C" int tos_catalog_info(const tos_catalog *cat, int64_t *n_los, int64_t 
     if (!cat) return TOS_ERR_INVALID;
     if (n_los) *n_los = cat->n_los;
     if (n_pix) *n_pix = cat->n_pix;
-    if (device_bytes) *device_bytes = (int64_t)(cat->pix.bytes + cat->los.bytes + cat->trig.bytes);
+    if (device_bytes) {
+        size_t n = 0;
+        for (const DevBuf *b : {&cat->pix, &cat->los, &cat->trig, &cat->ladder.pix, &cat->ladder.d, &cat->ladder.l,
+                                &cat->ladder.place})
+            n += b->bytes;
+        *device_bytes = (int64_t)n;
+    }
     return TOS_OK;
 }
 
