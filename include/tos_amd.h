@@ -203,6 +203,9 @@ typedef struct {
     int32_t precision;        /* enum tos_precision */
     int32_t accum;            /* enum tos_accum */
     int32_t per_skybin;       /* 1: also return per-sky-bin subsamples */
+    /* A launch shape of one's own is one of the general pair kernel: a value
+     * other than 0 here keeps a catalogue off the pass on its wavelength
+     * ladder, which is the faster one where it applies (see tos_pass). */
     int32_t block_size;       /* 0 = tuned default; else 64..1024, multiple of 64 */
     int32_t blocks_per_cu;    /* 0 = tuned default */
     int32_t flags;            /* TOS_XI_* bits below (0 = all optimisations on) */
@@ -211,7 +214,8 @@ typedef struct {
 } tos_xi_opts;
 
 /* tos_xi_opts.flags: switch off individual work-saving schemes (results are
- * identical either way; used for A/B timing). */
+ * identical either way; used for A/B timing).  They are the general pair
+ * kernel's: with any of them a pass takes that kernel. */
 enum {
     TOS_XI_NO_WINDOW = 1,     /* evaluate partner pixels outside the r_par window */
     TOS_XI_NO_TRANSPOSE = 2,  /* keep short primary remainders on the lanes */
@@ -234,7 +238,7 @@ typedef struct {
     double *sub_didj, *sub_wgt;
     /* written by the call */
     uint64_t num_pixel_pairs_used;   /* XiEstimator.cc:151 */
-    uint64_t num_guard_rechecks;     /* FP32C pairs re-binned in FP64 */
+    uint64_t num_guard_rechecks;     /* FP32C pairs binned in FP64 one by one */
     uint64_t num_pairs_evaluated;    /* pixel pairs the kernel evaluated (pairs
                                         outside the r_par window are rejected
                                         without evaluation) */
@@ -280,15 +284,16 @@ typedef struct {
 int tos_batch_run(tos_ctx *ctx, int32_t n, const tos_batch_job *jobs, int use_graph,
                   tos_xi_result *out, double *batch_ms);
 
-/* Times the pair kernel of one job over a small set of launch shapes and
- * keeps the fastest for this context and kernel variant: workgroup size
+/* Times the general pair kernel of one job over a small set of launch shapes
+ * and keeps the fastest for this context and kernel variant: workgroup size
  * 256/512/1024 x workgroups per CU 1/2/4/8 (as the LDS allows), then
  * workgroups per resident slot 4/8/16/64, then the work-item size
  * (partner pixels per item, 1024-16384; the pair list's items are rebuilt
  * for each).  Later tos_xi_run (block_size = 0), tos_xi_run_per_skybin and
- * tos_batch_run calls use it (the server keeps the default shape).  No
- * counterpart in the reference, whose CUDA launch shape is fixed
- * (gpu/brute.cu:121-149). */
+ * tos_batch_run calls use it where they take that kernel (the server keeps
+ * the default shape); passes on a wavelength ladder have a shape of their own,
+ * and *best_ms is not their time.  No counterpart in the reference, whose
+ * CUDA launch shape is fixed (gpu/brute.cu:121-149). */
 int tos_xi_autotune(tos_ctx *ctx, const tos_catalog *cat, const tos_pairs *pairs,
                     const tos_grid *grid, int32_t precision, int32_t *best_block,
                     int32_t *best_blocks_per_cu, double *best_ms);

@@ -138,7 +138,9 @@ class Device:
 
     def autotune(self, pairs, grid, precision=_lib.FP32C):
         """Pick the fastest launch shape for this kernel variant
-        (tos_xi_autotune); returns (block, blocks_per_cu, kernel_ms)."""
+        (tos_xi_autotune); returns (block, blocks_per_cu, kernel_ms).  The
+        shape is the general pair kernel's; passes on a wavelength ladder
+        do not take it."""
         b, bpc, ms = C.c_int32(0), C.c_int32(0), C.c_double(0)
         g = grid.to_c()
         check(lib().tos_xi_autotune(self.h, pairs.dcat.h, pairs.h, C.byref(g), int(precision), C.byref(b),
