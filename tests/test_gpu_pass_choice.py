@@ -223,3 +223,30 @@ def test_catalogue_bytes_count_the_ladder(dev):
     assert held() >= before + 12 * cat.n_pix + 8 * cat.n_los
     pairs.free()
     dcat.free()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("scale", [3e-21, 1e-22, 1e-30])
+def test_products_below_the_normal_floats(dev, ora, lists, scale):
+    """w1 w2 and (w d)1 (w d)2 round to subnormal floats like the reference's
+    (types.h:77-87), and to zero below them."""
+    cat = lists[0]
+    c = synth.Catalog(cat.ra, cat.dec, cat.offsets, cat.value, cat.loglam, cat.weight * np.float32(scale),
+                      cat.distance, cat.zq, cat.scale)
+    if scale > 1e-30:
+        p = np.float64(np.median(c.weight)) ** 2
+        assert 2.0 ** -149 < p < 2.0 ** -126
+    grid = GridSpec.cartesian()
+    ref = ora.xi_run(c, grid, c.scale, order=3, nthreads=8)["raw"]
+    dcat = dev.upload(c)
+    pairs = dcat.pairs(grid.max_angular_scale(c.scale), order=3, nthreads=8)
+    print(f"case: weights times {scale}", flush=True)
+    h = pairs.run(grid, precision=tos_amd.FP64)
+    assert pairs.last_pass() == tos_amd.PASS_LADDER
+    close(h, ref["num_pairs"], ref)
+    assert (scale == 1e-30) == (h.wgt.max() == 0.0)
+    a = pairs.run(grid, precision=tos_amd.FP64, accum=tos_amd.ACC_ALL)
+    assert pairs.last_pass() == tos_amd.PASS_LADDER
+    close(a, ref["num_pairs"], ref)
+    pairs.free()
+    dcat.free()
