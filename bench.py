@@ -43,6 +43,17 @@ PEAK_FP32 = 157.3
 PEAK_FP64 = 78.6
 # algorithmic flops per evaluated pixel pair (reference formula, once per pair)
 F_ALG = {"cartesian": 20, "polar": 18, "observing": 11}
+# the pass on a wavelength ladder forms no separation per pixel pair: it adds
+# both products of one in FP64 (an FMA of the peak is two operations)
+F_LADDER = 2
+PEAK_FP64_ADD = PEAK_FP64 / 2
+COMPUTE_UNIT = {
+    False: "VALU (no MFMA: pair counting is not a dense contraction); peak = MI355X FP32 157.3 TFLOP/s; "
+           "F_alg = 20 flop per evaluated pixel pair",
+    True: "VALU FP64 additions, two per evaluated pixel pair (their f32 products come from MFMA, one "
+          "v_mfma_f32_16x16x1_4b for 256 pixel pairs); peak = half of MI355X FP64 78.6 TFLOP/s, which counts an FMA "
+          "as two",
+}
 
 CONFIGS = {
     "c2": dict(n_qso=160000, area=10000.0, seed=3000,
@@ -148,12 +159,12 @@ def copy_calibration(mib: int):
     print(json.dumps({"copy_bytes_read": n * 4, "copy_bytes_written": n * 4, "launches": 5}))
 
 
-def traffic_from_profile(workload_key: str):
-    """HBM bytes per launch of the FP32C pair kernel on this workload, from the
+def traffic_from_profile(workload_key: str, ladder: bool):
+    """HBM bytes per launch of the pair kernel on this workload, from its
     committed rocprofv3 FETCH_SIZE / WRITE_SIZE summary (counters scaled by a
     plain copy of known size): its lines `traffic <config> fp32c <bytes>`.
     None when no summary covers the workload."""
-    path = os.path.join(ROOT, "profiles", "xi_pairs_hbm_traffic.txt")
+    path = os.path.join(ROOT, "profiles", "tile_pass_c2_counters.txt" if ladder else "xi_pairs_hbm_traffic.txt")
     if not os.path.exists(path):
         return None
     with open(path) as f:
@@ -164,12 +175,13 @@ def traffic_from_profile(workload_key: str):
     return None
 
 
-def counters_from_profile(workload_key: str):
-    """VALU issue rate and LDS busy fraction of the FP32C pair kernel on
-    this workload, from the committed rocprofv3 SQ counter summary: its
+def counters_from_profile(workload_key: str, ladder: bool):
+    """VALU issue rate and LDS busy fraction of the pair kernel on this
+    workload, from its committed rocprofv3 SQ counter summary: its
     lines `counters <config> fp32c <valu per CU-cycle> <lds busy>`.  None
     when no summary covers the workload."""
-    path = os.path.join(ROOT, "profiles", "xi_pairs_c2_sq_counters.txt")
+    name = "tile_pass_c2_counters.txt" if ladder else "xi_pairs_c2_sq_counters.txt"
+    path = os.path.join(ROOT, "profiles", name)
     if not os.path.exists(path):
         return None
     with open(path) as f:
@@ -177,8 +189,7 @@ def counters_from_profile(workload_key: str):
             tok = line.split()
             if len(tok) == 5 and tok[0] == "counters" and tok[1] == workload_key and tok[2] == "fp32c":
                 return {"valu_instructions_per_cu_cycle": float(tok[3]), "lds_busy_of_cu_cycles": float(tok[4]),
-                        "source": "profiles/xi_pairs_c2_sq_counters.txt (rocprofv3 SQ counters, peak 1 VALU "
-                                  "instruction per CU-cycle)"}
+                        "source": f"profiles/{name} (rocprofv3 SQ counters, peak 1 VALU instruction per CU-cycle)"}
     return None
 
 
@@ -189,8 +200,9 @@ def nthreads_host():
 def bench_c3(args):
     """Batched mocks: 128 realisations of the Lyman-alpha generator (seeds
     4000+i, sightline counts uniform in [2000, 40000], 2000 deg^2), Cartesian
-    50x50, FP32C, all in one hipGraph-captured batched launch with the
-    autotuned launch shape; against 128 sequential runs."""
+    50x50, FP32C, all in one hipGraph-captured batched launch (jobs off a
+    wavelength ladder with the autotuned launch shape); against 128
+    sequential runs."""
     import numpy as np
     import tos_amd
     from tos_amd import GridSpec, synth
@@ -661,18 +673,20 @@ def main():
         dt = time.perf_counter() - t0
         log(f"grid {g.type} precision {prec}: {steps} steps {dt:.3f} s, kernel avg {np.mean(kms):.3f} ms, "
             f"rechecks {h.num_guard_rechecks}, evaluated {h.num_pairs_evaluated:.4e}")
-        return dt, float(np.mean(kms)), h
+        return dt, float(np.mean(kms)), h, pairs.last_pass() == tos_amd.PASS_LADDER
 
     n64 = args.fp64_steps if args.fp64_steps is not None else max(1, args.steps // 2)
 
     def both(g, fname, steps):
-        dt32, k32, h32 = timed(g, tos_amd.FP32C, steps, args.warmup)
-        dt64, k64, h64 = timed(g, tos_amd.FP64, n64, min(args.warmup, 1))
-        f = F_ALG[fname]
+        dt32, k32, h32, ladder = timed(g, tos_amd.FP32C, steps, args.warmup)
+        dt64, k64, h64, ladder64 = timed(g, tos_amd.FP64, n64, min(args.warmup, 1))
+        f, peak = (F_LADDER, PEAK_FP64_ADD) if ladder else (F_ALG[fname], PEAK_FP32)
+        f64, peak64 = (F_LADDER, PEAK_FP64_ADD) if ladder64 else (F_ALG[fname], PEAK_FP64)
         return {"dt32": dt32, "k32": k32, "h32": h32, "dt64": dt64, "k64": k64, "h64": h64,
                 "v32": npp * steps / dt32, "v64": npp * n64 / dt64,
+                "ladder": ladder, "f": f, "peak": peak, "peak64": peak64,
                 "achieved": h32.num_pairs_evaluated * f / (k32 * 1e-3) / 1e12,
-                "achieved64": h64.num_pairs_evaluated * f / (k64 * 1e-3) / 1e12}
+                "achieved64": h64.num_pairs_evaluated * f64 / (k64 * 1e-3) / 1e12}
 
     C = both(grid, "cartesian", args.steps)
     P = both(polar, "polar", max(1, args.steps // 2))
@@ -700,29 +714,27 @@ def main():
         "pixel_pairs_per_step": npp,
         "pixel_pairs_evaluated_per_step": C["h32"].num_pairs_evaluated,
         "fp64": {"value": C["v64"], "ms_per_step": C["dt64"] / n64 * 1e3, "steps": n64, "kernel_ms": C["k64"],
-                 "roofline_frac_fp64": C["achieved64"] / PEAK_FP64},
+                 "roofline_frac_fp64": C["achieved64"] / C["peak64"]},
         "fp32c_over_fp64": C["v32"] / C["v64"],
         "kernel_fp32c_over_fp64": C["k64"] / C["k32"],
         "counts_fp32c_equal_fp64": bool(np.array_equal(C["h32"].num_pairs, C["h64"].num_pairs)),
         "fp32c_per_bin_error_vs_fp64": per_bin_error(C["h32"], C["h64"]),
         "guard_rechecks_per_pair": C["h32"].num_guard_rechecks / max(1, C["h32"].num_pixel_pairs_used),
-        "roofline": {"bound": "valu", "achieved": C["achieved"], "peak": PEAK_FP32, "unit": "TFLOP/s",
-                     "frac": C["achieved"] / PEAK_FP32, "traffic": traffic_from_profile(args.config),
-                     "compute_unit": "VALU (no MFMA: pair counting is not a dense contraction); "
-                                     "peak = MI355X FP32 157.3 TFLOP/s; F_alg = 20 flop per evaluated "
-                                     "pixel pair",
-                     "frac_of_unpacked_fp32": C["achieved"] / (PEAK_FP32 / 2),
-                     "achieved_over_all_candidate_pairs": npp * F_ALG["cartesian"] / (C["k32"] * 1e-3) / 1e12,
-                     "kernel_ms": C["k32"], "issue": counters_from_profile(args.config)},
+        "kernel": "tile_pass_kernel (wavelength ladder)" if C["ladder"] else "xi_pairs_kernel",
+        "roofline": {"bound": "valu", "achieved": C["achieved"], "peak": C["peak"], "unit": "TFLOP/s",
+                     "frac": C["achieved"] / C["peak"], "traffic": traffic_from_profile(args.config, C["ladder"]),
+                     "compute_unit": COMPUTE_UNIT[C["ladder"]],
+                     "kernel_ms": C["k32"], "issue": counters_from_profile(args.config, C["ladder"])},
         "polar": {"grid": "polar [0:200]*50 x [0:1]*20 x [3.556:3.735]*1",
                   "value_fp32c": P["v32"], "value_fp64": P["v64"], "fp32c_over_fp64": P["v32"] / P["v64"],
                   "kernel_ms_fp32c": P["k32"], "kernel_ms_fp64": P["k64"],
                   "pixel_pairs_evaluated_per_step": P["h32"].num_pairs_evaluated,
                   "counts_fp32c_equal_fp64": bool(np.array_equal(P["h32"].num_pairs, P["h64"].num_pairs)),
                   "fp32c_per_bin_error_vs_fp64": per_bin_error(P["h32"], P["h64"]),
-                  "roofline": {"bound": "valu", "achieved": P["achieved"], "peak": PEAK_FP32, "unit": "TFLOP/s",
-                               "frac": P["achieved"] / PEAK_FP32, "f_alg": F_ALG["polar"],
-                               "frac_fp64": P["achieved64"] / PEAK_FP64}},
+                  "kernel": "tile_pass_kernel (wavelength ladder)" if P["ladder"] else "xi_pairs_kernel",
+                  "roofline": {"bound": "valu", "achieved": P["achieved"], "peak": P["peak"], "unit": "TFLOP/s",
+                               "frac": P["achieved"] / P["peak"], "f_alg": P["f"],
+                               "frac_fp64": P["achieved64"] / P["peak64"]}},
     }
     if not args.no_cpu:
         out["cpu_baseline"], sample = cpu_baseline(cat, grid)

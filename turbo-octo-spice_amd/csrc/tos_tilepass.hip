@@ -18,13 +18,13 @@
 //             bound, is binned with the reference arithmetic (slow_bin).
 // So 64 pixel pairs cost some 9 VALU instructions (two conversions, two FP64
 // additions and one count each, and a share of the scan and the edges) in
-// place of 26 and three LDS atomics (xi_pairs_kernel).  VALU issue and, for
-// large catalogues, L2 misses on the sightlines' blocks bound the pass: 23
+// place of 26 and three LDS atomics (xi_pairs_kernel).  VALU issue (0.82 of its
+// peak for 37 million sightline pairs) and, for large catalogues, L2 misses on
+// the sightlines' blocks (7.4e11 bytes at 6.5 TB/s there) bound the pass: 23
 // instructions a visit of 256 pairs of steps and some 115 where an edge is
 // passed.  Sorting larger groups (kMaxGroup) makes edges rarer: 46
-// instructions a visit at 16384 pairs, 39 at 65536 (37 million pairs; Polar
-// 136 and 85).  0.77 of a visit's 256 are pixel pairs, the rest covers ends of
-// sightlines.
+// instructions a visit at 16384 pairs, 39 at 65536, 33 at 1048576 (Polar 41).
+// 0.89 of a visit's 256 are pixel pairs, the rest covers ends of sightlines.
 //
 // Polar grids have both their axes move with K, at a K of its own for each
 // pair of steps; the edges come from a table in LDS, so one formula serves
