@@ -458,9 +458,7 @@ extern "C" int tos_catalog_info(const tos_catalog *cat, int64_t *n_los, int64_t 
     if (n_pix) *n_pix = cat->n_pix;
     if (device_bytes) {
         size_t n = 0;
-        for (const DevBuf *b : {&cat->pix, &cat->los, &cat->trig, &cat->ladder.pix, &cat->ladder.d, &cat->ladder.l,
-                                &cat->ladder.place})
-            n += b->bytes;
+        for (const DevBuf *b : {&cat->pix, &cat->los, &cat->trig, &cat->ladder.pix, &cat->ladder.mem}) n += b->bytes;
         *device_bytes = (int64_t)n;
     }
     return TOS_OK;
@@ -648,7 +646,7 @@ void catalog_detach(tos_catalog *cat, std::vector<void *> &dev)
     detach(cat->pix, dev);
     detach(cat->los, dev);
     detach(cat->trig, dev);
-    for (DevBuf *b : {&cat->ladder.pix, &cat->ladder.d, &cat->ladder.l, &cat->ladder.place}) detach(*b, dev);
+    for (DevBuf *b : {&cat->ladder.pix, &cat->ladder.mem}) detach(*b, dev);
     delete cat;
 }
 
@@ -659,8 +657,7 @@ void pairs_detach(tos_pairs *p, std::vector<void *> &dev)
     detach(p->items, dev);
     detach(p->cost_prefix, dev);
     detach(p->theta, dev);
-    TilePlan &t = p->tiles;
-    for (DevBuf *b : {&t.masks, &t.rec, &t.batch_ptr, &t.visits}) detach(*b, dev);
+    detach(p->tiles.mem, dev);
     delete p;
 }
 

@@ -47,10 +47,12 @@ struct Ladder {
     int nblk = 0;
     int n_steps = 0;
     double mean_nb = 0;           // blocks a sightline covers
-    DevBuf pix, d, l, place;
+    DevBuf pix;
+    DevBuf mem;                   // of the following
+    float *d = nullptr, *l = nullptr;   // [16 nblk]
+    LadderLos *place = nullptr;
     std::vector<float> h_d, h_l;  // [16 nblk]
-    std::vector<uint64_t> table;  // state 3: the survey's hash table and the step of each slot
-    std::vector<uint16_t> step_of;
+    std::vector<uint64_t> table;  // state 3: the survey's hash table, a clear state, the step of each slot
     void release();
 };
 
@@ -60,7 +62,11 @@ struct TilePlan {
     int n_batches = 0;
     int words = 0;                // mask words of a batch
     uint64_t total = 0;           // visits of all tiles
-    DevBuf masks, rec, batch_ptr, visits;
+    DevBuf mem;                   // of the following (TileArgs)
+    uint64_t *masks = nullptr;
+    uint4 *rec = nullptr;
+    int32_t *batch_ptr = nullptr;
+    uint32_t *visits = nullptr;
     void release();
 };
 

@@ -14,13 +14,20 @@ namespace tos {
 
 namespace {
 
-struct Scratch {   // released on every return
-    DevBuf b[7];
-    ~Scratch()
+// Places in one allocation (an allocation takes some 10 to 100 us, a plan and
+// a ladder were 17 of them).
+struct Carve {
+    size_t bytes = 0;
+    size_t add(size_t n)
     {
-        for (DevBuf &x : b) x.release();
+        const size_t at = (bytes + 255) & ~(size_t)255;
+        bytes = at + n;
+        return at;
     }
 };
+// A plan's temporaries up to this size lie in the context's scratch, which
+// stays; larger ones are allocated for it.
+constexpr size_t kKeepScratch = (size_t)32 << 20;
 
 int copy_back(tos_ctx *ctx, void *dst, const void *src, size_t n, const char *what)
 {
@@ -33,16 +40,18 @@ int copy_back(tos_ctx *ctx, void *dst, const void *src, size_t n, const char *wh
 
 void Ladder::release()
 {
-    for (DevBuf *x : {&pix, &d, &l, &place}) x->release();
+    pix.release();
+    mem.release();
 }
 
 void TilePlan::release()
 {
-    for (DevBuf *x : {&masks, &rec, &batch_ptr, &visits}) x->release();
+    mem.release();
     state = 0;
 }
 
 constexpr size_t kTableBytes = (size_t)kLadderTable * 8;
+constexpr size_t kStateWords = 2, kStepWords = kLadderTable / 4;   // behind the table
 
 static LadderArgs ladder_args(const tos_catalog *cat)
 {
@@ -65,7 +74,7 @@ static int survey_ladder(tos_ctx *ctx, tos_catalog *cat)
     // the table and the state in the context's scratch: a catalogue without a
     // ladder costs no allocation
     uint32_t st[3] = {0, 0, 0};
-    if (ctx->scratch_a.reserve(kTableBytes + 16) != TOS_OK) return TOS_OK;
+    if (ctx->scratch_a.reserve(kTableBytes + 8 * (kStateWords + kStepWords)) != TOS_OK) return TOS_OK;
     int rc;
     LadderArgs a = ladder_args(cat);
     a.table = (uint64_t *)ctx->scratch_a.ptr;
@@ -98,11 +107,12 @@ static int survey_ladder(tos_ctx *ctx, tos_catalog *cat)
     if (!ok) return TOS_OK;
     L.n_steps = (int)steps.size();
     L.nblk = (int)((steps.size() + kBlockSteps - 1) / kBlockSteps);
-    L.step_of.assign(kLadderTable, 0);
+    tab.resize(kLadderTable + kStateWords + kStepWords, 0);
+    uint16_t *step_of = (uint16_t *)(tab.data() + kLadderTable + kStateWords);
     L.h_d.assign((size_t)L.nblk * kBlockSteps, steps.back().d);
     L.h_l.assign((size_t)L.nblk * kBlockSteps, steps.back().l);
     for (size_t k = 0; k < steps.size(); ++k) {
-        L.step_of[(size_t)steps[k].slot] = (uint16_t)k;
+        step_of[steps[k].slot] = (uint16_t)k;
         L.h_d[k] = steps[k].d;
         L.h_l[k] = steps[k].l;
     }
@@ -138,24 +148,26 @@ static int build_ladder(tos_ctx *ctx, tos_catalog *cat)
 {
     Ladder &L = cat->ladder;
     if (L.state != 3) return TOS_OK;
-    constexpr size_t kStepBytes = (size_t)kLadderTable * 2;
     uint32_t st[3] = {0, 0, 0};
     int rc;
-    if (ctx->scratch_b.reserve(kStepBytes + (size_t)cat->n_los * 4) != TOS_OK ||
-        L.place.reserve((size_t)cat->n_los * sizeof(LadderLos)) != TOS_OK)
+    Carve c;
+    const size_t key_bytes = L.h_d.size() * 4, at_keys = c.add(2 * key_bytes), at_place = c.add((size_t)cat->n_los * sizeof(LadderLos));
+    if (ctx->scratch_b.reserve((size_t)cat->n_los * 4) != TOS_OK || L.mem.reserve(c.bytes) != TOS_OK)
         return give_up(L, TOS_ERR_NOMEM);
-    L.table.resize(kLadderTable + 2, 0);   // and the state, cleared
+    L.d = (float *)((char *)L.mem.ptr + at_keys);
+    L.l = L.d + L.h_d.size();
+    L.place = (LadderLos *)((char *)L.mem.ptr + at_place);
+    std::vector<float> keys(L.h_d);
+    keys.insert(keys.end(), L.h_l.begin(), L.h_l.end());
     if ((rc = upload(ctx, ctx->scratch_a, L.table.data(), L.table.size() * 8, "ladder table")) != TOS_OK ||
-        (rc = upload(ctx, ctx->scratch_b, L.step_of.data(), kStepBytes, "ladder steps")) != TOS_OK ||
-        (rc = upload(ctx, L.d, L.h_d.data(), L.h_d.size() * 4, "ladder distances")) != TOS_OK ||
-        (rc = upload(ctx, L.l, L.h_l.data(), L.h_l.size() * 4, "ladder wavelengths")) != TOS_OK)
+        (rc = upload(ctx, L.mem, keys.data(), keys.size() * 4, "ladder steps")) != TOS_OK)
         return give_up(L, rc);
     LadderArgs a = ladder_args(cat);
     a.table = (uint64_t *)ctx->scratch_a.ptr;
     a.state = (uint32_t *)((char *)ctx->scratch_a.ptr + kTableBytes);
-    a.step = (const uint16_t *)ctx->scratch_b.ptr;
-    a.place = (LadderLos *)L.place.ptr;
-    a.nblk_of = (uint32_t *)((char *)ctx->scratch_b.ptr + kStepBytes);
+    a.step = (const uint16_t *)((char *)ctx->scratch_a.ptr + kTableBytes + 8 * kStateWords);
+    a.place = L.place;
+    a.nblk_of = (uint32_t *)ctx->scratch_b.ptr;
     int e = launch_ladder_place(a, ctx->stream);
     if (e != hipSuccess) return give_up(L, hip_fail(ctx, (hipError_t)e, "ladder placement"));
     if ((rc = copy_back(ctx, st, a.state, sizeof(st), "ladder block count")) != TOS_OK) return give_up(L, rc);
@@ -169,7 +181,6 @@ static int build_ladder(tos_ctx *ctx, tos_catalog *cat)
     if (st[0]) return give_up(L, TOS_OK);
     L.state = 1;
     L.table = std::vector<uint64_t>();
-    L.step_of = std::vector<uint16_t>();
     return TOS_OK;
 }
 
@@ -218,46 +229,60 @@ static int ensure_tile_plan(tos_ctx *ctx, tos_pairs *p)
     for (size_t k = 0; k + 1 < bp.size(); ++k) q = std::max(q, bp[k + 1] - bp[k]);
     T.n_batches = (int)bp.size() - 1;
     if ((int64_t)T.n_batches * L.nblk * (2 * L.nblk + 1) >= (1ll << 31)) return TOS_OK;
-    Scratch sc;
-    DevBuf &rlos = sc.b[0], &rptr = sc.b[1], &state = sc.b[2], &cover = sc.b[3], &keys = sc.b[4], &groups = sc.b[5], &keys2 = sc.b[6];
     T.words = (int)((q + 63) / 64);
     const size_t np = (size_t)p->n_pairs, rows = (size_t)T.n_batches * L.nblk;
-    if (cover.reserve(np * 4) != TOS_OK || T.masks.reserve(rows * 2 * T.words * 8) != TOS_OK ||
-        T.rec.reserve(np * 16) != TOS_OK || T.visits.reserve(rows * L.nblk * 4) != TOS_OK ||
-        (max_group > kSortRun && (keys.reserve(np * 8) != TOS_OK || keys2.reserve(np * 8) != TOS_OK)))
-        return give_up(T, TOS_ERR_NOMEM);
+    Carve c, tmp;
+    const size_t at_masks = c.add(rows * 2 * T.words * 8), at_rec = c.add(np * 16), at_visits = c.add(rows * L.nblk * 4),
+                 at_batches = c.add(bp.size() * 4);
+    const HostPairs &h = p->h;
+    const size_t at_state = tmp.add(16), at_groups = tmp.add(gp.size() * 4), at_rlos = tmp.add(h.row_los.size() * 4),
+                 at_rptr = tmp.add(h.row_ptr.size() * 8), head = tmp.bytes, at_cover = tmp.add(np * 4),
+                 sorted = max_group > kSortRun ? np * 8 : 0, at_keys = tmp.add(sorted), at_keys2 = tmp.add(sorted);
+    struct Local {
+        DevBuf b;
+        ~Local() { b.release(); }
+    } local;
+    DevBuf &work = tmp.bytes <= kKeepScratch ? ctx->scratch_c : local.b;
+    if (T.mem.reserve(c.bytes) != TOS_OK || work.reserve(tmp.bytes) != TOS_OK) return give_up(T, TOS_ERR_NOMEM);
+    char *const mem = (char *)T.mem.ptr, *const w = (char *)work.ptr;
+    T.masks = (uint64_t *)(mem + at_masks);
+    T.rec = (uint4 *)(mem + at_rec);
+    T.visits = (uint32_t *)(mem + at_visits);
+    T.batch_ptr = (int32_t *)(mem + at_batches);
+    std::vector<char> up(head, 0);
+    std::memcpy(up.data() + at_groups, gp.data(), gp.size() * 4);
+    std::memcpy(up.data() + at_rlos, h.row_los.data(), h.row_los.size() * 4);
+    std::memcpy(up.data() + at_rptr, h.row_ptr.data(), h.row_ptr.size() * 8);
+    hipError_t he = hipMemcpyAsync(w, up.data(), head, hipMemcpyHostToDevice, ctx->stream);
+    if (he == hipSuccess)
+        he = hipMemcpyAsync(T.batch_ptr, bp.data(), bp.size() * 4, hipMemcpyHostToDevice, ctx->stream);
+    if (he != hipSuccess) return give_up(T, hip_fail(ctx, he, "tile plan tables"));
     uint64_t st[2] = {0, 0};
-    if ((rc = upload(ctx, T.batch_ptr, bp.data(), bp.size() * 4, "tile batches")) != TOS_OK ||
-        (rc = upload(ctx, groups, gp.data(), gp.size() * 4, "tile groups")) != TOS_OK ||
-        (rc = upload(ctx, rlos, p->h.row_los.data(), p->h.row_los.size() * 4, "tile rows")) != TOS_OK ||
-        (rc = upload(ctx, rptr, p->h.row_ptr.data(), p->h.row_ptr.size() * 8, "tile row offsets")) != TOS_OK ||
-        (rc = upload(ctx, state, st, sizeof(st), "tile state")) != TOS_OK)
-        return give_up(T, rc);
     TilePlanArgs a{};
-    a.row_los = (const int32_t *)rlos.ptr;
-    a.row_ptr = (const int64_t *)rptr.ptr;
+    a.row_los = (const int32_t *)(w + at_rlos);
+    a.row_ptr = (const int64_t *)(w + at_rptr);
     a.other = (const int32_t *)p->other.ptr;
     a.csep = (const double *)p->csep.ptr;
-    a.place = (const LadderLos *)L.place.ptr;
+    a.place = L.place;
     a.n_rows = p->n_rows;
     a.n_batches = T.n_batches;
     a.max_batch = q;
     a.n_groups = (int32_t)gp.size() - 1;
     a.max_group = max_group;
-    a.group_ptr = (const int32_t *)groups.ptr;
+    a.group_ptr = (const int32_t *)(w + at_groups);
     a.nblk = L.nblk;
-    a.batch_ptr = (const int32_t *)T.batch_ptr.ptr;
+    a.batch_ptr = T.batch_ptr;
     a.words = T.words;
-    a.keys = (uint64_t *)keys.ptr;
-    a.keys2 = (uint64_t *)keys2.ptr;
-    a.cover = (uint32_t *)cover.ptr;
-    a.masks = (uint64_t *)T.masks.ptr;
-    a.rec = (uint4 *)T.rec.ptr;
-    a.visits = (uint32_t *)T.visits.ptr;
-    a.state = (unsigned long long *)state.ptr;
+    a.keys = (uint64_t *)(w + at_keys);
+    a.keys2 = (uint64_t *)(w + at_keys2);
+    a.cover = (uint32_t *)(w + at_cover);
+    a.masks = T.masks;
+    a.rec = T.rec;
+    a.visits = T.visits;
+    a.state = (unsigned long long *)(w + at_state);
     const int e = launch_tile_plan(a, ctx->stream);
     if (e != hipSuccess) return give_up(T, hip_fail(ctx, (hipError_t)e, "tile plan"));
-    if ((rc = copy_back(ctx, st, state.ptr, sizeof(st), "tile state copy")) != TOS_OK) return give_up(T, rc);
+    if ((rc = copy_back(ctx, st, a.state, sizeof(st), "tile state copy")) != TOS_OK) return give_up(T, rc);
     if (st[0]) return give_up(T, TOS_OK);
     T.total = st[1];
     T.state = 1;
@@ -316,17 +341,29 @@ static double tile_s_min(const tos_catalog *cat)
 
 // What the passes of a launch's jobs are expected to take, in us.
 struct PassCost {
-    // general path: the longest chain of one work item, and the pairs' work
-    double gen_lat = 0, gen = 0;
+    int jobs = 0;
+    // general path: the longest chain of one work item, the sightline pairs'
+    // work, and that of N pixel pairs (w_pix: weighted)
+    double gen_lat = 0, gen_pairs = 0, w_pix = 0, N = 0;
     // tile path: start, the visits' work, the longest chain of edges, of close
     // pairs; the plan
     double base = 140, tile = 0, edges = 0, near = 0, plan = 0;
-    double general() const { return 150 + std::hypot(gen_lat, gen); }
-    double tiles() const { return base + std::max(tile, edges) + near; }
+    double general() const
+    {
+        const double pix = N > 0 ? std::min(2e-6 * w_pix, 3000.0 * w_pix / N + 3e-7 * w_pix) : 0.0;
+        return 150 + (jobs > 1 ? 15.0 * jobs : 0.0) + std::hypot(gen_lat, gen_pairs + pix);
+    }
+    // (many jobs fill the device better than one that starts and ends alone)
+    double tiles() const { return base + std::max(jobs > 1 ? 300 + 0.6 * tile : tile, edges) + near; }
+    // (and their plans' memory is not that of a list just freed)
+    double plans() const { return jobs > 1 ? 1.35 * plan : plan; }
     void add(const PassCost &o)
     {
+        jobs += o.jobs;
         gen_lat = std::max(gen_lat, o.gen_lat);
-        gen += o.gen;
+        gen_pairs += o.gen_pairs;
+        w_pix += o.w_pix;
+        N += o.N;
         base = std::max(base, o.base);
         tile += o.tile;
         edges = std::max(edges, o.edges);
@@ -376,10 +413,14 @@ static PassCost pass_cost(const tos_ctx *ctx, const tos_pairs *p, const tos_grid
     const double partners = P / (double)std::max<int64_t>(1, p->n_rows), pix = std::sqrt(N / P);
     const double item = std::max(pix * std::sqrt(partners), partners * std::min(4.8, 0.25 * pix));
     c.gen_lat = (all ? 2.0 : f) * (fixed ? 1.0 : 1.6 * bands) * std::min(380.0, item) * (0.2 + 0.75 * w);
-    c.gen = f * bands * (fixed ? 1.0 : prec == TOS_FP64 ? 1.9 : 3.5) * (2e-3 * P + std::min(2e-6 * Nw, 3000.0 + 3e-7 * Nw));
+    const double g_all = f * bands * (fixed ? 1.0 : prec == TOS_FP64 ? 1.9 : 3.5);
+    c.jobs = 1;
+    c.gen_pairs = g_all * 2e-3 * P;
+    c.w_pix = g_all * Nw;
+    c.N = Nw;
     // tile path
     if (polar) c.base = 245;
-    if (p->tiles.state == 0) c.plan = 240 + 11e-3 * std::min(P, 16384.0) + 0.6e-3 * P;
+    if (p->tiles.state == 0) c.plan = 190 + 11e-3 * std::min(P, 16384.0) + 0.8e-3 * P;
     const double all_visits = p->tiles.state == 1 ? (double)p->tiles.total : P * nb * nb;
     const double visits = std::max(1.0, all_visits * std::min(1.0, (2.0 * band + 1.0) / std::max(1.0, nb)));
     const double tiles = nblk * (2.0 * band + 1.0), bins = polar ? (double)tile_edges(g) : (double)ge.n[1];
@@ -402,7 +443,7 @@ static PassCost pass_cost(const tos_ctx *ctx, const tos_pairs *p, const tos_grid
 // went without it: a list that is used again and again gets one at last.
 static bool tiles_pay(const PassCost &c, int32_t passes_before)
 {
-    return (c.general() - c.tiles()) * (passes_before + 1.0) >= c.plan;
+    return (c.general() - c.tiles()) * (passes_before + 1.0) >= c.plans();
 }
 
 int choose_tiles(tos_ctx *ctx, int n, const TileJob *jobs, char *take)
@@ -468,13 +509,13 @@ bool tile_args(const tos_pairs *p, const tos_grid &g, TileArgs &t)
     const TilePlan &T = p->tiles;
     t = TileArgs{};
     t.pix = (const float *)L.pix.ptr;
-    t.d = (const float *)L.d.ptr;
-    t.l = (const float *)L.l.ptr;
-    t.masks = (const uint64_t *)T.masks.ptr;
+    t.d = L.d;
+    t.l = L.l;
+    t.masks = T.masks;
     t.words = T.words;
-    t.rec = (const uint4 *)T.rec.ptr;
-    t.batch_ptr = (const int32_t *)T.batch_ptr.ptr;
-    t.visits = (const uint32_t *)T.visits.ptr;
+    t.rec = T.rec;
+    t.batch_ptr = T.batch_ptr;
+    t.visits = T.visits;
     t.nblk = L.nblk;
     t.n_batches = T.n_batches;
     t.width0 = g.width[0];
