@@ -277,7 +277,6 @@ extern "C" int tos_catalog_upload(tos_ctx *ctx, const tos_sightlines *s, tos_cat
     struct LosScan {
         float lmin, lmax;
         double dmin, dmax, labs;
-        float step;   // smallest loglam step
         bool d_sorted, l_sorted, finite;
     };
     std::vector<LosScan> scan((size_t)bad_off);
@@ -285,13 +284,11 @@ extern "C" int tos_catalog_upload(tos_ctx *ctx, const tos_sightlines *s, tos_cat
     // its scan
     auto pack = [&](int64_t k, float4 *dst) {
         const int64_t a = s->offsets[k], b = s->offsets[k + 1];
-        LosScan r{INFINITY, -INFINITY, INFINITY, 0.0, 0.0, INFINITY, true, true, true};
+        LosScan r{INFINITY, -INFINITY, INFINITY, 0.0, 0.0, true, true, true};
         for (int64_t p = a; p < b; ++p) {
             if (p > a) {
                 if (!(s->distance[p] >= s->distance[p - 1])) r.d_sorted = false;
                 if (!(s->loglam[p] >= s->loglam[p - 1])) r.l_sorted = false;
-                const float up = s->loglam[p] - s->loglam[p - 1];
-                if (up > 0.0f) r.step = std::min(r.step, up);
             }
             const float d = s->distance[p], l = s->loglam[p], w = s->weight[p], v = s->value[p];
             // {distance, loglam, weight, f32(weight * value)} (types.h:78)
@@ -406,7 +403,7 @@ extern "C" int tos_catalog_upload(tos_ctx *ctx, const tos_sightlines *s, tos_cat
     // sampled wavelength geometry: the step is the one that a tenth of the
     // sightlines undercut (the smallest might be an odd pixel's)
     double l_lo = INFINITY, l_hi = -INFINITY, span = 0;
-    std::vector<float> steps;
+    int64_t spans = 0;
     const int64_t every = std::max<int64_t>(1, nl / 1024);
     for (int64_t k = 0; k < nl; k += every) {
         if (c->h_los[(size_t)k].n < 2) continue;
@@ -414,14 +411,25 @@ extern "C" int tos_catalog_upload(tos_ctx *ctx, const tos_sightlines *s, tos_cat
         l_lo = std::min(l_lo, (double)r.lmin);
         l_hi = std::max(l_hi, (double)r.lmax);
         span += (double)r.lmax - (double)r.lmin;
-        steps.push_back(r.step);
+        ++spans;
     }
-    if (!steps.empty()) {
+    std::vector<float> steps;
+    const int64_t seldom = std::max<int64_t>(1, nl / 64);
+    for (int64_t k = 0; k < nl; k += seldom) {
+        const int64_t a = s->offsets[k], b = std::min(s->offsets[k + 1], a + 64);
+        float step = INFINITY;
+        for (int64_t p = a + 1; p < b; ++p) {
+            const float up = s->loglam[p] - s->loglam[p - 1];
+            if (up > 0.0f) step = std::min(step, up);
+        }
+        if (b - a >= 2) steps.push_back(step);
+    }
+    if (!steps.empty() && spans > 0) {
         std::nth_element(steps.begin(), steps.begin() + (std::ptrdiff_t)(steps.size() / 10), steps.end());
         const float step = steps[steps.size() / 10];
         c->l_step = std::isfinite(step) ? (double)step : 0.0;
         c->l_range = l_hi - l_lo;
-        c->l_span = span / (double)steps.size();
+        c->l_span = span / (double)spans;
     }
     rc = upload(ctx, c->los, c->h_los.data(), c->h_los.size() * sizeof(LosInfo), "catalog sightlines");
     if (rc == TOS_OK) {
