@@ -182,7 +182,7 @@ def test_a_small_list_gets_its_plan_once_it_has_paid(dev):
 
 @pytest.mark.gpu
 def test_batches_choose_as_a_whole(dev):
-    """Jobs too small for a plan each share the launch's verdict, and a sparse
+    """Jobs too small for a plan each share the launch's choice, and a sparse
     job stays on the general kernel among full ones."""
     grid = GridSpec.cartesian()
     full = synth.lya_catalog(700, area_deg2=100.0, seed=4)
